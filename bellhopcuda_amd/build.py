@@ -20,6 +20,11 @@ CXX_SOURCES = ["host2d.cpp", "host3d.cpp", "writers2d.cpp"]
 COMMON = ["-O3", "-std=c++17", "-fPIC", "-ffp-contract=off", "-fno-fast-math"]
 DEVICE = ["--offload-arch=" + ARCH, "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
           "-Wno-unused-value"]
+# The trace kernels' ray loops hold hundreds of FP64 constants (division, atan2,
+# hypot, reflection). Hoisted out of the loop by the machine-level LICM they
+# take a register pair each and push the ray state into AGPRs and scratch;
+# loaded where they are used they cost one move.
+LOOPS = ["-mllvm", "-disable-machine-licm", "-mllvm", "-sink-insts-to-avoid-spills"]
 
 
 def _run(cmd):
@@ -37,7 +42,7 @@ def build(verbose=False):
     objs = []
     for src in HIP_SOURCES:
         obj = os.path.join(objdir, src + ".o")
-        _run([HIPCC] + COMMON + DEVICE + ["-x", "hip", "-c", os.path.join(CSRC, src), "-o", obj])
+        _run([HIPCC] + COMMON + DEVICE + (LOOPS if src == "trace2d.hip" else []) + ["-x", "hip", "-c", os.path.join(CSRC, src), "-o", obj])
         objs.append(obj)
     for src in CXX_SOURCES:
         obj = os.path.join(objdir, src + ".o")

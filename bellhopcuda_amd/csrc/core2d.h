@@ -54,6 +54,14 @@ template<typename real> __host__ __device__ inline real spacing(real v)
     return std::fabs(std::nextafter(v, (real)0) - v);
 }
 
+// d < 1000 spacing(x). The spacing is at most 2 EPS |x| + the smallest normal,
+// so a longer d needs no look at x's neighbour.
+template<typename real> __host__ __device__ inline bool tiny_length(real d, real x)
+{
+    if(d > RL(3.0e3) * RC<real>::EPS * std::fabs(x) + RL(1.0e4) * RC<real>::MINPOS) return false;
+    return d < RL(1.0e3) * spacing(x);
+}
+
 // ---------------------------------------------------------------------------
 // Complex arithmetic as gcc lowers std::complex / C99 complex (no contraction)
 // ---------------------------------------------------------------------------
@@ -76,22 +84,18 @@ template<typename real> __host__ __device__ inline cpx<real> cmul(cpx<real> a, c
 }
 template<typename real> __host__ __device__ inline cpx<real> rmul(real r, cpx<real> b) { return C(r * b.re, r * b.im); }
 template<typename real> __host__ __device__ inline cpx<real> rdivc(cpx<real> a, real r) { return C(a.re / r, a.im / r); }
-// libgcc __divdc3 (Smith's method), finite inputs.
+// libgcc __divdc3 (Smith's method), finite inputs. The method's two cases are
+// the same three divisions on exchanged operands.
 template<typename real> __host__ __device__ inline cpx<real> cdiv(cpx<real> n, cpx<real> dd)
 {
-    real a = n.re, b = n.im, c = dd.re, d = dd.im, ratio, denom, x, y;
-    if(std::fabs(c) < std::fabs(d)) {
-        ratio = c / d;
-        denom = (c * ratio) + d;
-        x = ((a * ratio) + b) / denom;
-        y = ((b * ratio) - a) / denom;
-    } else {
-        ratio = d / c;
-        denom = (d * ratio) + c;
-        x = ((b * ratio) + a) / denom;
-        y = (b - (a * ratio)) / denom;
-    }
-    return C(x, y);
+    const bool sw = std::fabs(dd.re) < std::fabs(dd.im);
+    const real p = sw ? dd.re : dd.im, q = sw ? dd.im : dd.re;
+    const real ratio = p / q;
+    const real denom = (p * ratio) + q;
+    const real u = (sw ? n.re : n.im) * ratio, v = (sw ? n.im : n.re) * ratio;
+    const real x = u + (sw ? n.im : n.re);
+    const real y = sw ? v - n.re : n.im - v;
+    return C(x / denom, y / denom);
 }
 template<typename real> __host__ __device__ inline cpx<real> realdiv(real r, cpx<real> dd)
 {
@@ -229,6 +233,26 @@ template<typename real> struct SSPOut {
     real rho, czz, crr, crz;
 };
 
+// Sound speed at a ray's current point, carried from the end of one step (or
+// from the ray's start, or past a reflection) to the start of the next: the
+// next step would evaluate the same point with the same tangent and segment
+// state. `ok` is 0 when that evaluation raised an error or warning; the next
+// step then evaluates again, so that it is counted again.
+template<typename real> struct SSPAt {
+    v2<real> gradc;
+    cpx<real> c;
+    real czz, crr, crz;
+    int32_t ok;
+};
+template<typename real> __host__ __device__ inline void carry(SSPAt<real> &a, const SSPOut<real> &o)
+{
+    a.gradc = o.gradc;
+    a.c = o.c;
+    a.czz = o.czz;
+    a.crr = o.crr;
+    a.crz = o.crz;
+}
+
 struct Err {
     uint32_t err, warn, nerr, nwarn;
     __host__ __device__ void error(int code)
@@ -246,9 +270,8 @@ struct Err {
 template<typename real> struct Trace {
     int32_t iz, ir;             // SSP segment state
     BdryState<real> top, bot;
-    HSd<real> htop, hbot;       // per-segment geoacoustics (type[1]=='L')
-    real xs_y;
     real DistBegTop, DistBegBot, DistEndTop, DistEndBot;
+    SSPAt<real> at;
 };
 
 template<typename real> struct Infl {
@@ -281,6 +304,14 @@ __host__ __device__ inline void UpdateSSPSegment(real x, real t, const real *arr
 }
 
 template<typename real> __host__ __device__ inline cpx<real> ldc(const real *p, int i) { return C(p[2 * i], p[2 * i + 1]); }
+
+// |a| > 1e10. Parts within 7e9 keep the magnitude below 9.9e9, so the hypot
+// (some 40 instructions) is left to values near the limit and NaN.
+template<typename real> __host__ __device__ inline bool cabs_over_1e10(cpx<real> a)
+{
+    if(std::fabs(a.re) <= RL(7.0e9) && std::fabs(a.im) <= RL(7.0e9)) return false;
+    return cabs_(a) > RL(1.0e10);
+}
 
 // ST: SSP type fixed at compile time ('C','S','P','N','Q','A'), or 0 to read it
 // from the problem at run time.
@@ -318,8 +349,7 @@ __host__ __device__ inline void EvaluateSSP(v2<real> x, v2<real> t, SSPOut<real>
             cpx<real> c0 = ldc(cf, iz), c1 = ldc(cf + n2, iz), c2 = ldc(cf + 2 * n2, iz), c3 = ldc(cf + 3 * n2, iz);
             real xt = x.y - z[iz];
             if(std::fabs(xt) > RL(1.0e10)) e.warning(16);
-            if(cabs_(c0) > RL(1.0e10) || cabs_(c1) > RL(1.0e10) || cabs_(c2) > RL(1.0e10) || cabs_(c3) > RL(1.0e10))
-                e.warning(17);
+            if(cabs_over_1e10(c0) || cabs_over_1e10(c1) || cabs_over_1e10(c2) || cabs_over_1e10(c3)) e.warning(17);
             o.c = c0 + rmul(xt, c1 + rmul(xt, c2 + rmul(xt, c3)));
             o.gradc = V(RL(0.0), (c1 + rmul(xt, rmul(RL(2.0), c2) + rmul(xt, rmul(RL(3.0), c3)))).re);
             o.czz = (rmul(RL(2.0), c2) + rmul(xt, rmul(RL(6.0), c3))).re;
@@ -376,12 +406,22 @@ __host__ __device__ inline void EvaluateSSP(v2<real> x, v2<real> t, SSPOut<real>
     }
 }
 
+// Density as EvaluateSSP interpolates it in segment iz (LinInterpDensity, ssp.hpp:53-59).
+template<typename real, char ST = 0>
+__host__ __device__ inline real DensityAt(real xz, const Prob2D<real> &P, const real *B, int iz)
+{
+    if((ST ? ST : P.ssp_type) == 'A') return FL(1.0);
+    const real *z = B + P.o_z, *rho = B + P.o_rho;
+    const real w = (xz - z[iz]) / (z[iz + 1] - z[iz]);
+    return (RL(1.0) - w) * rho[iz] + w * rho[iz + 1];
+}
+
 // ---------------------------------------------------------------------------
 // Boundary segment lookup (reference src/boundary.hpp:66-227, 2D)
 // ---------------------------------------------------------------------------
 template<typename real>
 __host__ __device__ inline void GetBdrySeg(v2<real> x, v2<real> t, BdryState<real> &bds, const real *bd, int n,
-                                           int NODE, bool longfmt, HSd<real> &hs, bool isTop, bool isInit, Err &e)
+                                           int NODE, bool isTop, bool isInit, Err &e)
 {
     if(!isInit
        && !(x.x < bds.lmin || (x.x == bds.lmin && t.x < FL(0.0)) || x.x > bds.lmax
@@ -405,11 +445,6 @@ __host__ __device__ inline void GetBdrySeg(v2<real> x, v2<real> t, BdryState<rea
     bds.lmax = b0[NODE + BN_XX];
     bds.x = V(b0[BN_XX], b0[BN_XY]);
     bds.n = V(b0[BN_NX], b0[BN_NY]);
-    if(longfmt) {
-        hs.cP = C(b0[BN_CPR], b0[BN_CPI]);
-        hs.cS = C(b0[BN_CSR], b0[BN_CSI]);
-        hs.rho = b0[BN_RHO];
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -420,24 +455,20 @@ template<typename real> __host__ __device__ inline bool outside_box(v2<real> x, 
     return dim == 0 ? std::fabs(x.x - RL(0.0)) >= P.box_r : std::fabs(x.y - RL(0.0)) >= P.box_z;
 }
 
+// The layer of iz0 is [zl, zh]. One division serves both sides (a step leaves
+// through one of them).
 template<typename real>
 __host__ __device__ inline void DepthInterfaceCrossing(bool stepTo, real &hInt, v2<real> &x, v2<real> x0,
-                                                       v2<real> u, int iz0, const real *z)
+                                                       v2<real> u, real zl, real zh)
 { // step.hpp:41-79
     if(!stepTo) hInt = RC<real>::MAXV;
-    if(std::fabs(u.y) > RC<real>::EPS) {
-        if(z[iz0] > x.y) {
-            hInt = (z[iz0] - x0.y) / u.y;
-            if(stepTo) {
-                x = x0 + sc(hInt, u);
-                x.y = z[iz0];
-            }
-        } else if(z[iz0 + 1] < x.y) {
-            hInt = (z[iz0 + 1] - x0.y) / u.y;
-            if(stepTo) {
-                x = x0 + sc(hInt, u);
-                x.y = z[iz0 + 1];
-            }
+    const bool above = zl > x.y;
+    if((above || zh < x.y) && std::fabs(u.y) > RC<real>::EPS) {
+        const real zi = above ? zl : zh;
+        hInt = (zi - x0.y) / u.y;
+        if(stepTo) {
+            x = x0 + sc(hInt, u);
+            x.y = zi;
         }
     }
 }
@@ -495,52 +526,44 @@ __host__ __device__ inline void TopBotSegCrossing(bool stepTo, real &hSeg, const
         smax = rmin(smax, segr[ir0 + 1]);
     }
     if(!stepTo) hSeg = RC<real>::MAXV;
-    if(std::fabs(u.x) > RC<real>::EPS) {
-        if(x.x < smin) {
-            hSeg = -(x0.x - smin) / u.x;
-            if(stepTo) {
-                x = x0 + sc(hSeg, u);
-                x.x = smin;
-                topRefl = botRefl = false;
-            }
-        } else if(x.x > smax) {
-            hSeg = -(x0.x - smax) / u.x;
-            if(stepTo) {
-                x = x0 + sc(hSeg, u);
-                x.x = smax;
-                topRefl = botRefl = false;
-            }
+    const bool left = x.x < smin;
+    if((left || x.x > smax) && std::fabs(u.x) > RC<real>::EPS) {
+        const real si = left ? smin : smax;
+        hSeg = -(x0.x - si) / u.x;
+        if(stepTo) {
+            x = x0 + sc(hSeg, u);
+            x.x = si;
+            topRefl = botRefl = false;
         }
     }
 }
 
 template<typename real>
-__host__ __device__ inline void ReduceStep(v2<real> x0, v2<real> u, int iz0, int ir0, const Trace<real> &S,
+__host__ __device__ inline void ReduceStep(v2<real> x0, v2<real> u, real zl, real zh, int ir0, const Trace<real> &S,
                                            const Prob2D<real> &P, const real *B, Err &e, real &h)
 { // step.hpp:271-342
     real hInt, hBoxxr, hBoxyz, hTop, hBot, hxSeg;
     bool dummy;
     v2<real> x = x0 + sc(h, u);
-    DepthInterfaceCrossing(false, hInt, x, x0, u, iz0, B + P.o_z);
+    DepthInterfaceCrossing(false, hInt, x, x0, u, zl, zh);
     BeamBoxCrossing(false, 0, hBoxxr, x, x0, u, P);
     BeamBoxCrossing(false, 1, hBoxyz, x, x0, u, P);
     TopBotCrossing(false, hTop, S.top, x, x0, u, dummy);
     TopBotCrossing(false, hBot, S.bot, x, x0, u, dummy);
     TopBotSegCrossing(false, hxSeg, S.top, S.bot, ir0, x, x0, u, P, B, dummy, dummy);
-    const real BIG = RC<real>::MAXV;
-    h = rmin(rmin(rmin(h, hInt), rmin(rmin(rmin(hBoxxr, hBoxyz), BIG), rmin(hTop, hBot))),
-             rmin(rmin(hxSeg, BIG), rmin(BIG, BIG)));
+    // (the reference's unused crossings stay at the largest value and never win)
+    h = rmin(rmin(rmin(h, hInt), rmin(rmin(hBoxxr, hBoxyz), rmin(hTop, hBot))), hxSeg);
     if(h < RL(-1e-4)) e.warning(8);
     if(h < RC<real>::INF_STEP * P.deltas) h = RC<real>::INF_STEP * P.deltas;
 }
 
 template<typename real>
 __host__ __device__ inline void StepToBdry(v2<real> x0, v2<real> &x2, v2<real> u, real &h, bool &topRefl, bool &botRefl,
-                                           int iz0, int ir0, const Trace<real> &S, const Prob2D<real> &P,
+                                           real zl, real zh, int ir0, const Trace<real> &S, const Prob2D<real> &P,
                                            const real *B)
 { // step.hpp:347-424
     x2 = x0 + sc(h, u);
-    DepthInterfaceCrossing(true, h, x2, x0, u, iz0, B + P.o_z);
+    DepthInterfaceCrossing(true, h, x2, x0, u, zl, zh);
     BeamBoxCrossing(true, 0, h, x2, x0, u, P);
     BeamBoxCrossing(true, 1, h, x2, x0, u, P);
     TopBotCrossing(true, h, S.top, x2, x0, u, topRefl);
@@ -562,61 +585,123 @@ __host__ __device__ inline void StepToBdry(v2<real> x0, v2<real> &x2, v2<real> u
     }
 }
 
+// r / c for a real r. A lossless medium (zero imaginary part) needs the real
+// quotient only; its imaginary part is then zero, as the full division gives.
+template<typename real> __host__ __device__ inline cpx<real> slowness_term(real r, cpx<real> c)
+{
+    if(c.im == (real)0) return C(r / c.re, (real)0);
+    return realdiv(r, c);
+}
+
+// After a reflection from p1 to p2: the evaluation at p2 as the next step
+// would make it, kept in S.at. It depends on the point and the profile
+// segment only, so it is made again only where one of them changed (beam
+// shift; a point on a knot). Its errors and warnings are left to that step.
+template<typename real, char ST>
+__host__ __device__ inline void CarrySSP(v2<real> x1, v2<real> x, v2<real> t, Trace<real> &S, const Prob2D<real> &P,
+                                         const real *B)
+{
+    if(!S.at.ok) return;
+    const char sst = ST ? ST : P.ssp_type;
+    int iz = S.iz, ir = S.ir;
+    if(sst != 'A') UpdateSSPSegment(x.y, t.y, B + P.o_z, P.npts, iz);
+    if(sst == 'Q') UpdateSSPSegment(x.x, t.x, B + P.o_segr, P.Nr, ir);
+    if(iz == S.iz && ir == S.ir && x.x == x1.x && x.y == x1.y) return;
+    SSPOut<real> o;
+    Err ec = {0, 0, 0, 0};
+    iz = S.iz;
+    ir = S.ir;
+    EvaluateSSP<real, ST>(x, t, o, P, B, iz, ir, ec);
+    S.at.ok = (ec.nerr | ec.nwarn) == 0u;
+    if(!S.at.ok) return;
+    S.iz = iz;
+    S.ir = ir;
+    carry(S.at, o);
+}
+
+// One polygon step. Profiles of depth alone (every type but 'Q') have no
+// range derivatives: the terms they would multiply are zero and are left out
+// (adding or subtracting zero changes no value). The step's own evaluations
+// are two: the start's is carried (S.at).
 template<typename real, char ST = 0>
 __host__ __device__ inline void Step(const RayPt<real> &ray0, RayPt<real> &ray2, Trace<real> &S, const Prob2D<real> &P,
                                      const real *B, Err &e, bool &topRefl, bool &botRefl)
 { // step.hpp:654-811 (2D)
-    SSPOut<real> o0, o1, o2;
-    EvaluateSSP<real, ST>(ray0.x, ray0.t, o0, P, B, S.iz, S.ir, e);
-    real c0 = o0.c.re;
-    real cnn0 = o0.crr * (ray0.t.y * ray0.t.y) - FL(2.0) * o0.crz * ray0.t.x * ray0.t.y + o0.czz * (ray0.t.x * ray0.t.x);
-    v2<real> pq0p = sc(-cnn0, ray0.q), pq0q = sc(c0, ray0.p);
-    int iz0 = S.iz, ir0 = S.ir;
-    real csq0 = c0 * c0;
-    v2<real> u0 = sc(c0, ray0.t);
+    const char sst = ST ? ST : P.ssp_type;
+    const bool inr = sst == 'Q';           // sound speed varies with range
+    const bool nocurv = sst == 'C';        // and has no second derivatives
+    SSPOut<real> o1, o2;
+    if(!S.at.ok) {
+        EvaluateSSP<real, ST>(ray0.x, ray0.t, o1, P, B, S.iz, S.ir, e);
+        carry(S.at, o1);
+    }
+    const SSPAt<real> o0 = S.at;
+    auto bend = [&](real crr, real crz, real czz, v2<real> t) { // -c^2 times the normal second derivative
+        if(inr) return crr * (t.y * t.y) - FL(2.0) * crz * t.x * t.y + czz * (t.x * t.x);
+        return czz * (t.x * t.x);
+    };
+    auto turned = [&](v2<real> t, real h, v2<real> gradc, real csq) {
+        if(inr) return t - dv(sc(h, gradc), csq);
+        return V(t.x, t.y - (h * gradc.y) / csq);
+    };
+    const real c0 = o0.c.re;
+    v2<real> pq0p = V((real)0, (real)0);
+    if(!nocurv) pq0p = sc(-bend(o0.crr, o0.crz, o0.czz, ray0.t), ray0.q);
+    const v2<real> pq0q = sc(c0, ray0.p);
+    const int iz0 = S.iz, ir0 = S.ir;
+    const real zl = B[P.o_z + iz0], zh = B[P.o_z + iz0 + 1];
+    const real csq0 = c0 * c0;
+    const v2<real> u0 = sc(c0, ray0.t);
     real h = P.deltas;
-    ReduceStep(ray0.x, u0, iz0, ir0, S, P, B, e, h);
-    real halfh = FL(0.5) * h;
+    ReduceStep(ray0.x, u0, zl, zh, ir0, S, P, B, e, h);
+    const real halfh = FL(0.5) * h;
     RayPt<real> ray1;
     ray1.x = ray0.x + sc(halfh, u0);
-    ray1.t = ray0.t - dv(sc(halfh, o0.gradc), csq0);
-    ray1.p = ray0.p + sc(halfh, pq0p);
-    ray1.q = ray0.q + sc(halfh, pq0q);
+    ray1.t = turned(ray0.t, halfh, o0.gradc, csq0);
+    ray1.p = nocurv ? ray0.p : ray0.p + sc(halfh, pq0p);
 
     EvaluateSSP<real, ST>(ray1.x, ray1.t, o1, P, B, S.iz, S.ir, e);
-    real c1 = o1.c.re;
-    real cnn1 = o1.crr * (ray1.t.y * ray1.t.y) - FL(2.0) * o1.crz * ray1.t.x * ray1.t.y + o1.czz * (ray1.t.x * ray1.t.x);
-    v2<real> pq1p = sc(-cnn1, ray1.q), pq1q = sc(c1, ray1.p);
-    real csq1 = c1 * c1;
-    v2<real> u1 = sc(c1, ray1.t);
-    ReduceStep(ray0.x, u1, iz0, ir0, S, P, B, e, h);
+    const real c1 = o1.c.re;
+    v2<real> pq1p = V((real)0, (real)0);
+    if(!nocurv) {
+        ray1.q = ray0.q + sc(halfh, pq0q);
+        pq1p = sc(-bend(o1.crr, o1.crz, o1.czz, ray1.t), ray1.q);
+    }
+    const v2<real> pq1q = sc(c1, ray1.p);
+    const real csq1 = c1 * c1;
+    const v2<real> u1 = sc(c1, ray1.t);
+    ReduceStep(ray0.x, u1, zl, zh, ir0, S, P, B, e, h);
 
-    real w1 = h / (RL(2.0) * halfh);
-    real w0 = RL(1.0) - w1;
-    v2<real> u2 = sc(w0, u0) + sc(w1, u1);
+    const real w1 = h / (RL(2.0) * halfh);
+    const real w0 = RL(1.0) - w1;
+    const v2<real> u2 = sc(w0, u0) + sc(w1, u1);
     v2<real> x2;
-    StepToBdry(ray0.x, x2, u2, h, topRefl, botRefl, iz0, ir0, S, P, B);
+    StepToBdry(ray0.x, x2, u2, h, topRefl, botRefl, zl, zh, ir0, S, P, B);
     ray2.x = x2;
-    real hw0 = h * w0, hw1 = h * w1;
-    ray2.t = (ray0.t - dv(sc(hw0, o0.gradc), csq0)) - dv(sc(hw1, o1.gradc), csq1);
-    ray2.tau = (ray0.tau + realdiv(hw0, o0.c)) + realdiv(hw1, o1.c);
-    ray2.p = ray0.p + sc(hw0, pq0p);
+    const real hw0 = h * w0, hw1 = h * w1;
+    ray2.t = turned(turned(ray0.t, hw0, o0.gradc, csq0), hw1, o1.gradc, csq1);
+    ray2.tau = (ray0.tau + slowness_term(hw0, o0.c)) + slowness_term(hw1, o1.c);
+    ray2.p = ray0.p;
+    if(!nocurv) ray2.p = (ray0.p + sc(hw0, pq0p)) + sc(hw1, pq1p);
     ray2.q = ray0.q + sc(hw0, pq0q);
-    ray2.p = ray2.p + sc(hw1, pq1p);
     ray2.q = ray2.q + sc(hw1, pq1q);
     ray2.Amp = ray0.Amp;
     ray2.Phase = ray0.Phase;
     ray2.NumTopBnc = ray0.NumTopBnc;
     ray2.NumBotBnc = ray0.NumBotBnc;
 
+    const uint32_t seen = e.nerr + e.nwarn;
     EvaluateSSP<real, ST>(ray2.x, ray2.t, o2, P, B, S.iz, S.ir, e);
+    S.at.ok = e.nerr + e.nwarn == seen;
+    carry(S.at, o2);
     ray2.c = o2.c.re;
     if(S.iz != iz0 || S.ir != ir0) { // CurvatureCorrection 2D, step.hpp:626-648
-        v2<real> gj = o2.gradc - o0.gradc;
-        v2<real> ray2n = V(-ray2.t.y, ray2.t.x);
-        real cnjump = dot(gj, ray2n);
-        real csjump = dot(gj, ray2.t);
-        real rm = (S.iz != iz0) ? ray2.t.x / ray2.t.y : -ray2.t.y / ray2.t.x;
+        const v2<real> gj = o2.gradc - o0.gradc;
+        const v2<real> ray2n = V(-ray2.t.y, ray2.t.x);
+        const real cnjump = inr ? dot(gj, ray2n) : gj.y * ray2n.y;
+        const real csjump = inr ? dot(gj, ray2.t) : gj.y * ray2.t.y;
+        const bool dz = !inr || S.iz != iz0;
+        real rm = (dz ? ray2.t.x : -ray2.t.y) / (dz ? ray2.t.y : ray2.t.x);
         real rn = rm * (FL(2.0) * cnjump - rm * csjump) / ray2.c;
         ray2.p = ray2.p - sc(rn, ray2.q);
     }
@@ -666,7 +751,7 @@ __host__ __device__ inline void BeamShift(const RayPt<real> &oldp, RayPt<real> &
 template<typename real, char ST = 0>
 __host__ __device__ inline void Reflect(const RayPt<real> &oldp, RayPt<real> &newp, const HSd<real> &hs, bool isTop,
                                         v2<real> tB, v2<real> nB, real kappa, const Prob2D<real> &P, const real *B,
-                                        const real *G, int &iz, int &ir, Err &e)
+                                        const real *G, Trace<real> &S, Err &e)
 {
     real Th = dot(oldp.t, nB);
     real Tg = dot(oldp.t, tB);
@@ -674,8 +759,14 @@ __host__ __device__ inline void Reflect(const RayPt<real> &oldp, RayPt<real> &ne
     newp.NumBotBnc = oldp.NumBotBnc + (isTop ? 0 : 1);
     newp.x = oldp.x;
     newp.t = oldp.t - sc(FL(2.0) * Th, nB);
+    // the profile at the reflection point: the step that ended there evaluated it
     SSPOut<real> o;
-    EvaluateSSP<real, ST>(oldp.x, oldp.t, o, P, B, iz, ir, e);
+    if(S.at.ok) {
+        o.c = S.at.c;
+        o.gradc = S.at.gradc;
+    } else {
+        EvaluateSSP<real, ST>(oldp.x, oldp.t, o, P, B, S.iz, S.ir, e);
+    }
     real c = o.c.re;
     newp.c = c;
     newp.tau = oldp.tau;
@@ -751,6 +842,7 @@ __host__ __device__ inline void Reflect(const RayPt<real> &oldp, RayPt<real> &ne
             g = C(hs.rho, (real)0);
         }
         cpx<real> J = C((real)0, (real)1);
+        if(S.at.ok) o.rho = DensityAt<real, ST>(oldp.x.y, P, B, S.iz);
         cpx<real> a = rmul(o.rho, f), b = cmul(cmul(J, kz), g);
         cpx<real> Refl = cdiv(-(a - b), a + b);
         real aR = cabs_(Refl);
@@ -816,11 +908,13 @@ __host__ __device__ inline bool RayInit(int isz, int ialpha, RayPt<real> &p0, Tr
     I.SrcDeclAngle = RadDeg * alpha;
     S.iz = S.ir = 0;
     v2<real> xs = V((real)FL(0.0), (real)P.Sz[isz]);
-    S.xs_y = xs.y;
     v2<real> tinit = V(G[P.o_acos + ialpha], G[P.o_asin + ialpha]);
     SSPOut<real> o;
     EvaluateSSP<real, ST>(xs, tinit, o, P, B, S.iz, S.ir, e);
     real c = o.c.re;
+    // (p0.t = tinit / c has tinit's signs: the first step's evaluation is this one)
+    S.at.ok = (e.nerr | e.nwarn) == 0u;
+    carry(S.at, o);
     {
         real DalphaOpt = std::sqrt(c / (FL(6.0) * P.freq0 * G[P.o_Rr + P.NRr - 1]));
         int NalphaOpt = 2 + (int)((G[P.o_alpha + P.Nalpha - 1] - G[P.o_alpha]) / DalphaOpt);
@@ -845,11 +939,9 @@ __host__ __device__ inline bool RayInit(int isz, int ialpha, RayPt<real> &p0, Tr
     p0.p = V((real)FL(1.0), (real)FL(0.0));
     p0.q = V((real)FL(0.0), (real)FL(1.0));
     if(P.run1 == 'G') p0.q = V((real)FL(0.0), (real)FL(0.0));
-    S.htop = P.top;
-    S.hbot = P.bot;
     S.top.Iseg = S.bot.Iseg = 0;
-    GetBdrySeg(xs, p0.t, S.top, B + P.o_ati, P.ati_n, P.node, P.ati_long == 'L', S.htop, true, true, e);
-    GetBdrySeg(xs, p0.t, S.bot, B + P.o_bty, P.bty_n, P.node, P.bty_long == 'L', S.hbot, false, true, e);
+    GetBdrySeg(xs, p0.t, S.top, B + P.o_ati, P.ati_n, P.node, true, true, e);
+    GetBdrySeg(xs, p0.t, S.bot, B + P.o_bty, P.bty_n, P.node, false, true, e);
     Distances(xs, S, S.DistBegTop, S.DistBegBot);
     if(S.DistBegTop <= FL(0.0) || S.DistBegBot <= FL(0.0)) {
         e.warning(4);
@@ -879,34 +971,55 @@ __host__ __device__ inline bool RayInit(int isz, int ialpha, RayPt<real> &p0, Tr
     return true;
 }
 
+// RayUpdate (trace.hpp:274-381, 2D) in its two parts: the step to p1, which
+// reports the boundary it ends on (0 none, 1 top, 2 bottom), and the
+// reflection there.
+template<typename real, char ST = 0>
+__host__ __device__ inline int RayStep(const RayPt<real> &p0, RayPt<real> &p1, Trace<real> &S, const Prob2D<real> &P,
+                                       const real *B, Err &e)
+{
+    bool topRefl = false, botRefl = false;
+    Step<real, ST>(p0, p1, S, P, B, e, topRefl, botRefl);
+    GetBdrySeg(p1.x, p1.t, S.top, B + P.o_ati, P.ati_n, P.node, true, false, e);
+    GetBdrySeg(p1.x, p1.t, S.bot, B + P.o_bty, P.bty_n, P.node, false, false, e);
+    Distances(p1.x, S, S.DistEndTop, S.DistEndBot);
+    return topRefl ? 1 : (botRefl ? 2 : 0);
+}
+
+template<typename real, char ST = 0>
+__host__ __device__ inline void RayReflect(const RayPt<real> &p1, RayPt<real> &p2, bool topRefl, Trace<real> &S,
+                                           const Prob2D<real> &P, const real *B, const real *G, Err &e)
+{
+    const real *b0 = B + (topRefl ? P.o_ati + S.top.Iseg * P.node : P.o_bty + S.bot.Iseg * P.node);
+    const real *b1 = b0 + P.node;
+    v2<real> nI, tI;
+    if((topRefl ? P.ati_curv : P.bty_curv) == 'C') {
+        const v2<real> bx = V(topRefl ? S.top.x.x : S.bot.x.x, topRefl ? S.top.x.y : S.bot.x.y);
+        real sss = dot(p1.x - bx, V(b0[BN_TX], b0[BN_TY])) / b0[BN_LEN];
+        nI = sc(FL(1.0) - sss, V(b0[BN_NDNX], b0[BN_NDNY])) + sc(sss, V(b1[BN_NDNX], b1[BN_NDNY]));
+        tI = sc(FL(1.0) - sss, V(b0[BN_NDTX], b0[BN_NDTY])) + sc(sss, V(b1[BN_NDTX], b1[BN_NDTY]));
+    } else {
+        nI = V(b0[BN_NX], b0[BN_NY]);
+        tI = V(b0[BN_TX], b0[BN_TY]);
+    }
+    HSd<real> hs = topRefl ? P.top : P.bot;
+    if((topRefl ? P.ati_long : P.bty_long) == 'L') { // the segment's own geoacoustics
+        hs.cP = C(b0[BN_CPR], b0[BN_CPI]);
+        hs.cS = C(b0[BN_CSR], b0[BN_CSI]);
+        hs.rho = b0[BN_RHO];
+    }
+    Reflect<real, ST>(p1, p2, hs, topRefl, tI, nI, b0[BN_KAPPA], P, B, G, S, e);
+    CarrySSP<real, ST>(p1.x, p2.x, p2.t, S, P, B);
+    Distances(p2.x, S, S.DistEndTop, S.DistEndBot);
+}
+
 template<typename real, char ST = 0>
 __host__ __device__ inline bool RayUpdate(const RayPt<real> &p0, RayPt<real> &p1, RayPt<real> &p2, Trace<real> &S,
                                           const Prob2D<real> &P, const real *B, const real *G, Err &e)
-{ // trace.hpp:274-381 (2D)
-    bool topRefl = false, botRefl = false;
-    Step<real, ST>(p0, p1, S, P, B, e, topRefl, botRefl);
-    GetBdrySeg(p1.x, p1.t, S.top, B + P.o_ati, P.ati_n, P.node, P.ati_long == 'L', S.htop, true, false, e);
-    GetBdrySeg(p1.x, p1.t, S.bot, B + P.o_bty, P.bty_n, P.node, P.bty_long == 'L', S.hbot, false, false, e);
-    Distances(p1.x, S, S.DistEndTop, S.DistEndBot);
-    if(topRefl || botRefl) {
-        const real *bd = B + (topRefl ? P.o_ati : P.o_bty);
-        const BdryState<real> &bs = topRefl ? S.top : S.bot;
-        const real *b0 = bd + bs.Iseg * P.node;
-        const real *b1 = b0 + P.node;
-        v2<real> nI, tI;
-        if((topRefl ? P.ati_curv : P.bty_curv) == 'C') {
-            real sss = dot(p1.x - bs.x, V(b0[BN_TX], b0[BN_TY])) / b0[BN_LEN];
-            nI = sc(FL(1.0) - sss, V(b0[BN_NDNX], b0[BN_NDNY])) + sc(sss, V(b1[BN_NDNX], b1[BN_NDNY]));
-            tI = sc(FL(1.0) - sss, V(b0[BN_NDTX], b0[BN_NDTY])) + sc(sss, V(b1[BN_NDTX], b1[BN_NDTY]));
-        } else {
-            nI = V(b0[BN_NX], b0[BN_NY]);
-            tI = V(b0[BN_TX], b0[BN_TY]);
-        }
-        Reflect<real, ST>(p1, p2, topRefl ? S.htop : S.hbot, topRefl, tI, nI, b0[BN_KAPPA], P, B, G, S.iz, S.ir, e);
-        Distances(p2.x, S, S.DistEndTop, S.DistEndBot);
-        return true;
-    }
-    return false;
+{
+    const int refl = RayStep<real, ST>(p0, p1, S, P, B, e);
+    if(refl) RayReflect<real, ST>(p1, p2, refl == 1, S, P, B, G, e);
+    return refl != 0;
 }
 
 // Returns 0 to continue, 1 for a normal stop (Nsteps = is + 1), 2 when the
@@ -1049,31 +1162,38 @@ __host__ __device__ inline void desc_common(SegDesc<real> &d, const RayPt<real> 
     d.is = is;
 }
 
-// Cartesian prelude: influence.hpp:1201-1297 and the receiver walk :1388-1402.
-// WINDOW = false leaves the segment's depth window to the scatter (every
-// depth in the descriptor; the scatter's per-column band and the zmin / zmax
-// test of each receiver select the same contributions): a batched trace,
-// latency-bound at one wavefront per SIMD, hands that search to the scatter.
-template<typename real, bool WINDOW = true>
-__host__ __device__ inline void prelude_cart(SegDesc<real> &d, const RayPt<real> &p0, const RayPt<real> &p1,
-                                             Infl<real> &I, int is, const Prob2D<real> &P, const real *G,
-                                             const real *RzT, int isz, int ialpha)
+// A step's influence update in two parts. seg_begin applies the update of the
+// ray's influence state and tells whether the step's segment is handed to the
+// scatter; seg_fill then forms its descriptor, and seg_end ends the update.
+// In between a kernel reserves the descriptor's slot, so that the descriptor's
+// fields can go from the ray's registers straight to memory.
+template<typename real> struct SegGeo {
+    v2<real> t;                 // Cartesian: step vector; ray-centred: the ray normal at the end
+    real rlen;
+    int32_t first, ir;          // Cartesian: first and last visited receiver range
+    int32_t moved;              // ray-centred: the normal becomes the next step's start
+};
+
+// Cartesian: influence.hpp:1201-1297 and the receiver walk :1388-1402.
+template<typename real>
+__host__ __device__ inline bool cart_begin(SegGeo<real> &g, const RayPt<real> &p0, const RayPt<real> &p1,
+                                           Infl<real> &I, const Prob2D<real> &P, const real *G, real &lo, real &hi)
 {
     const real *Rr = G + P.o_Rr;
-    d.nitems = 0;
     real rA = I.x.x, rB = p1.x.x;
-    v2<real> rayt = p1.x - p0.x;
-    real rlen = std::sqrt(dot(rayt, rayt));
-    if(rlen < RL(1.0e3) * spacing(p1.x.x)) return;
+    g.t = p1.x - p0.x;
+    g.rlen = std::sqrt(dot(g.t, g.t));
+    if(tiny_length(g.rlen, p1.x.x)) return false;
     real phaseq = p0.q.x;
     if(IsAtCaustic(I.qOld, phaseq)) I.phase += RC<real>::PI / FL(2.0);
     I.qOld = phaseq;
-    d.lo = rmin(rA, rB);
-    d.hi = rmax(rA, rB);
+    lo = rmin(rA, rB);
+    hi = rmax(rA, rB);
     // walk: the set of visited receiver ranges is contiguous. The bracket
     // (Rr[ir], Rr[ir + 1]) travels with the ray, so a step that crosses no
     // receiver range reads no range from memory; the comparisons are the walk's.
-    int ir = I.ir, first = I.ir;
+    int ir = I.ir;
+    g.first = ir;
     real rlo = I.rbr.x, rhi = I.rbr.y;
     const real rfirst = rlo;    // Rr[first]
     for(;;) {
@@ -1097,18 +1217,30 @@ __host__ __device__ inline void prelude_cart(SegDesc<real> &d, const RayPt<real>
     I.ir = ir;
     I.rbr = V(rlo, rhi);
     I.x = p1.x;
+    g.ir = ir;
     // A step that crosses no receiver range has the one column Rr[first]:
     // outside [lo, hi) the scatter's column test accepts none of its
     // receivers, so the segment is not handed to the scatter at all.
-    if(ir == first && !(rfirst >= d.lo && rfirst < d.hi)) return;
+    return !(ir == g.first && !(rfirst >= lo && rfirst < hi));
+}
+
+// WINDOW = false leaves the segment's depth window to the scatter (every
+// depth in the descriptor; the scatter's per-column band and the zmin / zmax
+// test of each receiver select the same contributions): a batched trace,
+// latency-bound at one wavefront per SIMD, hands that search to the scatter.
+template<typename real, bool WINDOW>
+__host__ __device__ inline void cart_fill(SegDesc<real> &d, const SegGeo<real> &g, const RayPt<real> &p0,
+                                          const RayPt<real> &p1, const Infl<real> &I, int is, const Prob2D<real> &P,
+                                          const real *RzT, int isz, int ialpha)
+{
     // the beam's reach: only for steps handed to the scatter
-    rayt = dv(rayt, rlen);
+    const v2<real> rayt = dv(g.t, g.rlen);
     real sigma = rmax(std::fabs(p0.q.x), std::fabs(p1.q.x)) * I.rcp_q0 / std::fabs(rayt.x);
     if(P.isGaussian) {
         real lambda = p0.c / P.freq0;
         sigma = rmax(sigma, rmin(FL(0.2) * P.freq0 * p1.tau.re, RC<real>::PI * lambda));
     }
-    real RadiusMax = I.BeamWindow * sigma;
+    real RadiusMax = (P.isGaussian ? RL(4.0) : RL(1.0)) * sigma;
     if(std::fabs(rayt.x) > FL(0.50001)) {
         d.zmin = rmin(p0.x.y, p1.x.y) - RadiusMax;
         d.zmax = rmax(p0.x.y, p1.x.y) + RadiusMax;
@@ -1116,10 +1248,10 @@ __host__ __device__ inline void prelude_cart(SegDesc<real> &d, const RayPt<real>
         d.zmin = -RC<real>::MAXV;
         d.zmax = RC<real>::MAXV;
     }
-    d.ir0 = first;
-    d.ir1 = ir;
-    d.dir = (ir >= first) ? 1 : -1;
-    int nr = (ir >= first ? ir - first : first - ir) + 1;
+    d.ir0 = g.first;
+    d.ir1 = g.ir;
+    d.dir = (g.ir >= g.first) ? 1 : -1;
+    int nr = (g.ir >= g.first ? g.ir - g.first : g.first - g.ir) + 1;
     d.iz0 = 0;
     d.nz = P.NRz_per_range;
     if(WINDOW && P.rz_sorted && P.run4 != 'I' && d.zmin > -RC<real>::MAXV) {
@@ -1131,38 +1263,39 @@ __host__ __device__ inline void prelude_cart(SegDesc<real> &d, const RayPt<real>
     d.nitems = nr * d.nz;
     d.xa = p0.x;
     d.ta = rayt;
-    d.rlen = rlen;
+    d.rlen = g.rlen;
     // the receiver angle enters arrivals only (TL runs skip the atan2)
     d.RcvrDecl = tl_run(P.run0) ? RL(0.0) : (RL(180.0) / RC<real>::PI) * std::atan2(rayt.y, rayt.x);
     desc_common(d, p0, p1, I, P, is, isz, ialpha);
 }
 
-// Ray-centred prelude: influence.hpp:1030-1071.
+// Ray-centred: influence.hpp:1030-1071.
 template<typename real>
-__host__ __device__ inline void prelude_raycen(SegDesc<real> &d, const RayPt<real> &p0, const RayPt<real> &p1,
-                                               Infl<real> &I, int is, const Prob2D<real> &P, const real *RzT, int isz,
-                                               int ialpha)
+__host__ __device__ inline bool raycen_begin(SegGeo<real> &g, const RayPt<real> &p0, const RayPt<real> &p1,
+                                             Infl<real> &I)
 {
-    d.nitems = 0;
+    g.moved = 0;
     real phaseq = p0.q.x;
     if(IsAtCaustic(I.qOld, phaseq)) I.phase += RC<real>::PI / FL(2.0);
     I.qOld = phaseq;
-    v2<real> rayn1 = sc(p1.c, V(p1.t.y, -p1.t.x));
-    if(std::fabs(rayn1.y) < RL(1e-10)) return;
-    if(std::fabs(p1.x.x - p0.x.x) < RL(1.0e3) * spacing(p1.x.x)) {
-        I.lastValid = 1;
-        I.x = p1.x;
-        I.rayn1 = rayn1;
-        return;
-    }
+    g.t = sc(p1.c, V(p1.t.y, -p1.t.x));
+    if(std::fabs(g.t.y) < RL(1e-10)) return false;
+    g.moved = 1;
+    return !tiny_length(std::fabs(p1.x.x - p0.x.x), p1.x.x);
+}
+
+template<typename real>
+__host__ __device__ inline void raycen_fill(SegDesc<real> &d, const SegGeo<real> &g, const RayPt<real> &p0,
+                                            const RayPt<real> &p1, const Infl<real> &I, int is, const Prob2D<real> &P,
+                                            const real *RzT, int isz, int ialpha)
+{
     d.lastValid = I.lastValid;
     d.xa = I.x;
     d.ta = I.rayn1;
     d.xb = p1.x;
-    d.tb = rayn1;
+    d.tb = g.t;
     d.RcvrDecl = tl_run(P.run0) ? RL(0.0) : (RL(180.0) / RC<real>::PI) * std::atan2(p1.t.y, p1.t.x);
     desc_common(d, p0, p1, I, P, is, isz, ialpha);
-    d.nitems = P.NRz_per_range;
     {
         // sigma(s) <= max(|q0|, |q1|) * rcp_q0 (q is linear in s), raised to the
         // AdjustSigma floor; 1e-4 relative slack covers the rounding of s and n1.
@@ -1190,9 +1323,36 @@ __host__ __device__ inline void prelude_raycen(SegDesc<real> &d, const RayPt<rea
         d.nz = imax(0, i1 - i0 + 1);
     }
     d.nitems = d.nz;
-    I.lastValid = 1;
-    I.x = p1.x;
-    I.rayn1 = rayn1;
+}
+
+template<typename real>
+__host__ __device__ inline bool seg_begin(SegGeo<real> &g, const RayPt<real> &p0, const RayPt<real> &p1, Infl<real> &I,
+                                          const Prob2D<real> &P, const real *G, real &lo, real &hi)
+{
+    if(P.isRayCen) return raycen_begin(g, p0, p1, I);
+    return cart_begin(g, p0, p1, I, P, G, lo, hi);
+}
+
+// RzT: the receiver depths as reals (the staged copy when the problem's
+// tables sit in LDS).
+template<typename real, bool WINDOW>
+__host__ __device__ inline void seg_fill(SegDesc<real> &d, const SegGeo<real> &g, const RayPt<real> &p0,
+                                         const RayPt<real> &p1, const Infl<real> &I, int is, const Prob2D<real> &P,
+                                         const real *RzT, int isz, int ialpha)
+{
+    if(P.isRayCen) raycen_fill(d, g, p0, p1, I, is, P, RzT, isz, ialpha);
+    else cart_fill<real, WINDOW>(d, g, p0, p1, I, is, P, RzT, isz, ialpha);
+}
+
+template<typename real>
+__host__ __device__ inline void seg_end(const SegGeo<real> &g, const RayPt<real> &p1, Infl<real> &I,
+                                        const Prob2D<real> &P)
+{
+    if(P.isRayCen && g.moved) {
+        I.lastValid = 1;
+        I.x = p1.x;
+        I.rayn1 = g.t;
+    }
 }
 
 // cos and sin of an FP64 phase at FP32 accuracy: Cody-Waite reduction by 2*pi
@@ -1444,15 +1604,17 @@ __host__ __device__ inline void item_raycen(const SegDesc<real> &d, int iz, cons
     for(int ir = blo; ir <= bhi; ++ir) raycen_one<real, RT, Sink, FAST>(d, ir, iz, nA, rA, nB, rB, P, Rr, sink);
 }
 
-// RzT: the receiver depths as reals (the staged copy when the problem's
-// tables sit in LDS).
+// The whole update of one step, with its descriptor (nitems = 0: not handed to
+// the scatter).
 template<typename real, bool WINDOW = true>
 __host__ __device__ inline void prelude(SegDesc<real> &d, const RayPt<real> &p0, const RayPt<real> &p1, Infl<real> &I,
                                         int is, const Prob2D<real> &P, const real *G, const real *RzT, int isz,
                                         int ialpha)
 {
-    if(P.isRayCen) prelude_raycen(d, p0, p1, I, is, P, RzT, isz, ialpha);
-    else prelude_cart<real, WINDOW>(d, p0, p1, I, is, P, G, RzT, isz, ialpha);
+    SegGeo<real> g;
+    d.nitems = 0;
+    if(seg_begin(g, p0, p1, I, P, G, d.lo, d.hi)) seg_fill<real, WINDOW>(d, g, p0, p1, I, is, P, RzT, isz, ialpha);
+    seg_end(g, p1, I, P);
 }
 
 template<typename real, int RT, typename Sink, bool FAST = false>

@@ -90,6 +90,8 @@ template<typename real> struct alignas(16) Seg {
 // buffer in all.
 template<typename real> constexpr int SEG_NC = (int)((seg_core_bytes<real>() + 15) / 16);
 template<typename real> constexpr int SEG_NW = (int)((sizeof(SegDesc<real>) + 15) / 16);
+// Slots whose 16-byte words all lie within a 32-bit offset of the word's row.
+constexpr size_t SEG_CAP_MAX = ((size_t)1 << 28) - 1;
 static_assert(SEG_NW<double> * 16 <= sizeof(Seg<double>) && SEG_NW<float> * 16 <= sizeof(Seg<float>), "slot size");
 template<typename real> union SegWords {
     SegDesc<real> d;
@@ -140,6 +142,7 @@ struct DevOut {
     uint32_t *errw;             // err, warn, nerr, nwarn
     int32_t *work;              // ray work counter (relative to job_begin)
     int32_t job_begin, job_end; // ray range of this trace pass
+    int32_t lanes;              // 2D / Nx2D trace: lanes of a wavefront that take rays (fan_lanes)
     void *segs;                 // segment buffer: seg_cap descriptor cores, then seg_cap rests (seg_core / seg_rest)
     uint32_t *seg_count;
     uint32_t seg_cap;
@@ -293,17 +296,15 @@ template<typename real> __device__ inline void seal_block(const SegBlock &B, int
     }
 }
 
-// Append this lane's descriptor (if it has work items) to the segment buffer:
-// all of it, or its core when `full` is false (seg_full). Called by all lanes
-// of the wavefront. A slot beyond the buffer sets the overflow flag: the host
+// A slot of the segment buffer for this lane (if has), called by all lanes of
+// the wavefront. A slot beyond the buffer sets the overflow flag: the host
 // then discards the pass and splits the ray range.
 template<typename real>
-__device__ inline void append_seg(const SegDesc<real> &d, int lane, const DevOut &O, SegBlock &B, bool full)
+__device__ inline uint32_t reserve_seg(bool has, int lane, const DevOut &O, SegBlock &B)
 {
-    bool has = d.nitems > 0;
-    unsigned long long m = __ballot(has);
-    if(!m) return;
-    uint32_t cnt = (uint32_t)__popcll(m);
+    const unsigned long long m = __ballot(has);
+    if(!m) return 0xFFFFFFFFu;
+    const uint32_t cnt = (uint32_t)__popcll(m);
     if(B.used + cnt > B.cap) {
         seal_block<real>(B, lane, O);
         uint32_t base = 0;
@@ -312,29 +313,54 @@ __device__ inline void append_seg(const SegDesc<real> &d, int lane, const DevOut
         B.used = 0;
         B.cap = SEG_BLOCK;
     }
-    if(has) {
-        uint32_t slot = B.base + B.used + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
-        if(slot < O.seg_cap) {
-            // 16-byte stores through a global-memory pointer (global_store,
-            // counted apart from LDS reads; a generic store would make every
-            // later LDS wait wait for it too)
-            typedef __attribute__((address_space(1))) unsigned long long gu64;
-            SegWords<real> u;
-            u.d = d;
-            gu64 *dst = (gu64 *)O.segs + 2 * (size_t)slot;
-            const size_t cap2 = 2 * (size_t)O.seg_cap;
-            const int nw = full ? SEG_NW<real> : SEG_NC<real>;
-#pragma unroll
-            for(int k = 0; k < SEG_NW<real>; ++k)
-                if(k < nw) {
-                    dst[k * cap2] = u.w[2 * k];
-                    dst[k * cap2 + 1] = u.w[2 * k + 1];
-                }
-        } else {
-            atomicOr(O.overflow, 1u);
-        }
-    }
+    const uint32_t slot = B.base + B.used + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
     B.used += cnt;
+    return slot;
+}
+
+// Store a descriptor in its slot: all of it, or its core when `full` is false
+// (seg_full).
+template<typename real>
+__device__ inline void store_seg(const SegDesc<real> &d, uint32_t slot, const DevOut &O, bool full)
+{
+    if(slot >= O.seg_cap) {
+        atomicOr(O.overflow, 1u);
+        return;
+    }
+    // 16-byte stores through a global-memory pointer (global_store, counted
+    // apart from LDS reads; a generic store would make every later LDS wait
+    // wait for it too). Word k's address is a scalar base, advanced from word
+    // to word, plus the slot's 32-bit offset: the empty asm keeps the compiler
+    // from holding all the words' addresses from one step to the next.
+    typedef unsigned long long u64x2 __attribute__((ext_vector_type(2)));
+    typedef __attribute__((address_space(1))) char gchar;
+    typedef __attribute__((address_space(1))) u64x2 gu64x2;
+    SegWords<real> u;
+    u.d = d;
+    const uint32_t off = slot * 16u;
+    const unsigned long long stride = 16ull * (uint32_t)__builtin_amdgcn_readfirstlane((int)O.seg_cap);
+    const unsigned long long at = (unsigned long long)O.segs;
+    unsigned long long base = (unsigned long long)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)at)
+        | ((unsigned long long)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(at >> 32)) << 32);
+    auto store = [&](int k) {
+        *(gu64x2 *)((gchar *)base + off) = u64x2{u.w[2 * k], u.w[2 * k + 1]};
+        base += stride;
+        asm volatile("" : "+s"(base));
+    };
+#pragma unroll
+    for(int k = 0; k < SEG_NC<real>; ++k) store(k);
+    if(full) {
+#pragma unroll
+        for(int k = SEG_NC<real>; k < SEG_NW<real>; ++k) store(k);
+    }
+}
+
+template<typename real>
+__device__ inline void append_seg(const SegDesc<real> &d, int lane, const DevOut &O, SegBlock &B, bool full)
+{
+    const bool has = d.nitems > 0;
+    const uint32_t slot = reserve_seg<real>(has, lane, O, B);
+    if(has) store_seg(d, slot, O, full);
 }
 
 // Exclusive prefix sum of cnt over the wavefront; returns the total.
@@ -406,54 +432,117 @@ __device__ inline void scatter_seg(const SegDesc<real> &d, const Prob2D<real> &P
     }
 }
 
+// One step of the wavefront's rays (RayUpdate and both influence updates of
+// the ray loop, src/trace.hpp:525-589): p0 moves to the step's end, or past the
+// reflection there. reserve(has) is called by all lanes and gives the lanes
+// with a segment its slot; out(d, slot) takes the descriptor. The reflected
+// point's segment has no length on Cartesian beams unless the beam is shifted:
+// its influence update then changes nothing and is left out. Both segments run
+// through one copy of the code, the descriptor is formed where it is stored,
+// and the reflection is made after that, so that descriptor, reflection and
+// the points between are not held in registers side by side.
+template<typename real, char ST, bool WINDOW, typename Reserve, typename Out>
+__device__ inline void step_ray(bool active, RayPt<real> &p0, Trace<real> &S, Infl<real> &I, int &is,
+                                const Prob2D<real> &P, const real *B, const real *G, int isz, int ia, Err &e,
+                                Reserve reserve, Out out)
+{
+    RayPt<real> p1;
+    int refl = 0;
+    bool go = active;
+    if(active) refl = RayStep<real, ST>(p0, p1, S, P, B, e);
+#pragma unroll 1
+    for(;;) {
+        SegGeo<real> g;
+        real lo, hi;
+        const bool has = go && seg_begin(g, p0, p1, I, P, G, lo, hi);
+        const uint32_t slot = reserve(has);
+        if(has) {
+            SegDesc<real> d;
+            d.lo = lo;
+            d.hi = hi;
+            seg_fill<real, WINDOW>(d, g, p0, p1, I, is, P, B + P.o_rzs, isz, ia);
+            out(d, slot);
+        }
+        if(go) {
+            seg_end(g, p1, I, P);
+            ++is;
+            p0 = p1;
+        }
+        go = false;
+        if(refl) {
+            RayReflect<real, ST>(p0, p1, refl == 1, S, P, B, G, e);
+            refl = 0;
+            go = P.isRayCen || p1.x.x != p0.x.x || p1.x.y != p0.x.y;
+            if(!go) {
+                ++is;
+                p0 = p1;
+            }
+        }
+        if(!__any(go)) break;
+    }
+}
+
 // Trace kernel of the field modes (TL / arrivals / eigen): the ray loop of
 // MainFieldModes (src/trace.hpp:525-589). Each step's influence state update
 // is done here (prelude); the receiver work goes to the segment buffer.
-template<typename real, char ST>
-__global__ void __launch_bounds__(256) k_trace2d(Prob2D<real> P, DevOut O)
+// STAGED: the problem's tables are read from their LDS copy, through a pointer
+// the compiler knows to be LDS; else from global memory, known to be global (a
+// generic pointer's loads wait for LDS and for the descriptor stores alike).
+template<typename real, char ST, bool STAGED>
+__global__ void __launch_bounds__(WAVE) k_trace2d(Prob2D<real> P, DevOut O)
 {
     extern __shared__ __align__(16) unsigned char lds_raw[];
-    const real *B = stage(P, lds_raw);
-    const real *G = P.base;
-    const int lane = threadIdx.x & (WAVE - 1);
+    const real *G = as_global(P.base);
+    const real *B;
+    if constexpr(STAGED) {
+        real *L = reinterpret_cast<real *>(lds_raw);
+        for(int i = threadIdx.x; i < P.staged_reals; i += WAVE) L[i] = G[i];
+        __syncthreads();
+        B = L;
+    } else {
+        B = G;
+    }
+    const int lane = threadIdx.x;
     const int njobs = O.job_end - O.job_begin;
+    const bool full = seg_full(P);
+    int32_t *const stats = as_global(O.stats);
+    double *const xend = as_global(O.xend);
     Err e = {0, 0, 0, 0};
     RayPt<real> p0;
     Trace<real> S;
     Infl<real> I;
     int job = 0, isz = 0, ia = 0, is = 0;
-    bool active = false, exhausted = false, init_fail = false;
+    bool active = false, exhausted = false;
     unsigned long long steps = 0;
     SegBlock blk{0u, 0u, 0u};
     for(int iter = 0;; ++iter) {
         if(!exhausted) {
-            unsigned long long need = __ballot(!active);
+            const bool want = !active && lane < O.lanes;
+            const unsigned long long need = __ballot(want);
             if(need) {
-                int cnt = __popcll(need);
-                int leader = __ffsll((unsigned long long)need) - 1;
+                const int cnt = __popcll(need);
+                const int leader = __ffsll(need) - 1;
                 int base = 0;
                 if(lane == leader) base = atomicAdd(O.work, cnt);
                 base = __shfl(base, leader);
                 if(base + cnt >= njobs) exhausted = true;
-                if(!active) {
-                    int my = base + __popcll(need & ((1ull << lane) - 1ull));
-                    if(my < njobs) {
-                        job = O.job_begin + my;
-                        JobIndices(job, P, isz, ia);
-                        is = 0;
-                        active = RayInit<real, ST>(isz, ia, p0, S, I, P, B, G, e);
-                        init_fail = !active;
-                        if(!active && O.stats) {
-                            O.stats[3 * job] = 0;
-                            O.stats[3 * job + 1] = 0;
-                            O.stats[3 * job + 2] = 0;
-                            O.xend[2 * job] = 0.0;
-                            O.xend[2 * job + 1] = 0.0;
-                        }
+                bool init_fail = false;
+                const int my = base + __popcll(need & ((1ull << lane) - 1ull));
+                if(want && my < njobs) {
+                    job = O.job_begin + my;
+                    JobIndices(job, P, isz, ia);
+                    is = 0;
+                    active = RayInit<real, ST>(isz, ia, p0, S, I, P, B, G, e);
+                    init_fail = !active;
+                    if(!active && O.stats) {
+                        stats[3 * job] = 0;
+                        stats[3 * job + 1] = 0;
+                        stats[3 * job + 2] = 0;
+                        xend[2 * job] = 0.0;
+                        xend[2 * job + 1] = 0.0;
                     }
                 }
                 note_done(O.prog, init_fail);
-                init_fail = false;
             }
         }
         if(!__any(active)) {
@@ -473,38 +562,22 @@ __global__ void __launch_bounds__(256) k_trace2d(Prob2D<real> P, DevOut O)
                 continue;
             }
         }
-        RayPt<real> p1, p2;
-        SegDesc<real> d;
-        d.nitems = 0;
-        bool two = false;
-        if(active) {
-            two = RayUpdate<real, ST>(p0, p1, p2, S, P, B, G, e);
-            prelude(d, p0, p1, I, is, P, G, B + P.o_rzs, isz, ia);
-            ++is;
-        }
-        append_seg(d, lane, O, blk, seg_full(P));
-        if(__any(two)) {
-            d.nitems = 0;
-            if(active && two) {
-                prelude(d, p1, p2, I, is, P, G, B + P.o_rzs, isz, ia);
-                ++is;
-            }
-            append_seg(d, lane, O, blk, seg_full(P));
-        }
+        step_ray<real, ST, true>(active, p0, S, I, is, P, B, G, isz, ia, e,
+                                 [&](bool has) { return reserve_seg<real>(has, lane, O, blk); },
+                                 [&](const SegDesc<real> &d, uint32_t slot) { store_seg(d, slot, O, full); });
         bool fin = false;
         if(active) {
-            p0 = two ? p2 : p1;
             int t = RayTerminate(p0, is, S, MAXN, P, e);
             if(t) {
                 active = false;
                 fin = true;
                 steps += (unsigned long long)is;
                 if(O.stats) {
-                    O.stats[3 * job] = is;
-                    O.stats[3 * job + 1] = p0.NumTopBnc;
-                    O.stats[3 * job + 2] = p0.NumBotBnc;
-                    O.xend[2 * job] = (double)p0.x.x;
-                    O.xend[2 * job + 1] = (double)p0.x.y;
+                    stats[3 * job] = is;
+                    stats[3 * job + 1] = p0.NumTopBnc;
+                    stats[3 * job + 2] = p0.NumBotBnc;
+                    xend[2 * job] = (double)p0.x.x;
+                    xend[2 * job + 1] = (double)p0.x.y;
                 }
             }
         }
@@ -874,7 +947,8 @@ __global__ void __launch_bounds__(64) k_tracenx2d(Prob2D<real> P, bhc3d::Prob3D<
     SegBlock blk{0u, 0u, 0u};
     for(int iter = 0;; ++iter) {
         if(!exhausted) {
-            unsigned long long need = __ballot(!active);
+            const bool want = !active && lane < O.lanes;
+            unsigned long long need = __ballot(want);
             if(need) {
                 int cnt = __popcll(need);
                 int leader = __ffsll((unsigned long long)need) - 1;
@@ -882,7 +956,7 @@ __global__ void __launch_bounds__(64) k_tracenx2d(Prob2D<real> P, bhc3d::Prob3D<
                 if(lane == leader) base = atomicAdd(O.work, cnt);
                 base = __shfl(base, leader);
                 if(base + cnt >= njobs) exhausted = true;
-                if(!active) {
+                if(want) {
                     int my = base + __popcll(need & ((1ull << lane) - 1ull));
                     if(my < njobs) {
                         job = O.job_begin + my;
@@ -1648,6 +1722,17 @@ int ensure_segs(bhc_ctx *c)
     return 0;
 }
 
+// Lanes of a wavefront that take rays: a fan smaller than the GPU's lanes is
+// spread over one wavefront per SIMD (four SIMDs per CU) instead of filling few
+// wavefronts. A wavefront walks the code of every case that one of its lanes
+// meets in a step (reflection, profile knot, receiver range, refill), so
+// fewer rays per wavefront make each step shorter.
+int fan_lanes(int nrays, int num_cus)
+{
+    const int simds = std::max(1, 4 * num_cus);
+    return std::min(WAVE, std::max(1, (nrays + simds - 1) / simds));
+}
+
 template<typename real> const bhc3d::Prob3D<real> &nx_of(const bhc_dev_problem *dp);
 template<> const bhc3d::Prob3D<double> &nx_of<double>(const bhc_dev_problem *dp) { return dp->N64; }
 template<> const bhc3d::Prob3D<float> &nx_of<float>(const bhc_dev_problem *dp) { return dp->N32; }
@@ -1670,7 +1755,7 @@ int run_passes(bhc_dev_problem *dp, const Prob2D<real> &P, DevOut O, void *segbu
     O.segs = segbuf;
     O.seg_count = c->d_seg_count;
     O.overflow = c->d_overflow;
-    O.seg_cap = (uint32_t)std::min<size_t>(segbytes / sizeof(Seg<real>), 0xFFFFFFF0u);
+    O.seg_cap = (uint32_t)std::min<size_t>(segbytes / sizeof(Seg<real>), SEG_CAP_MAX);
     std::vector<std::pair<int, int>> todo{{0, dp->njobs}};
     c->passes = 0;
     c->ph_trace_ms = c->ph_scatter_ms = 0.0;
@@ -1685,10 +1770,10 @@ int run_passes(bhc_dev_problem *dp, const Prob2D<real> &P, DevOut O, void *segbu
         HIPCHECK(hipMemsetAsync(c->d_overflow, 0, sizeof(uint32_t), s));
         HIPCHECK(hipMemsetAsync(dp->d_work, 0, sizeof(int32_t), s));
         int nj = r.second - r.first;
-        int waves = (nj + WAVE - 1) / WAVE;
+        O.lanes = fan_lanes(nj, c->num_cus);
         // one wavefront per workgroup spreads the rays over all CUs (the trace
         // kernel is register-bound at one wavefront per SIMD)
-        int tblocks = std::max(1, std::min(waves, c->num_cus * 4 * c->bpc));
+        int tblocks = std::max(1, std::min((nj + O.lanes - 1) / O.lanes, c->num_cus * 4 * c->bpc));
         // error / warning words as the completed passes left them (stream
         // order: after the previous pass's scatter), restored if this trace
         // pass overflows and its rays are traced again
@@ -1700,13 +1785,22 @@ int run_passes(bhc_dev_problem *dp, const Prob2D<real> &P, DevOut O, void *segbu
         HIPCHECK(hipEventRecord(c->pa, s));
         if(dp->nx2d) {
             hipLaunchKernelGGL((k_tracenx2d<real>), dim3(tblocks), dim3(WAVE), 0, s, P, nx_of<real>(dp), O);
-        } else switch(P.ssp_type) {
-        case 'C': hipLaunchKernelGGL((k_trace2d<real, 'C'>), dim3(tblocks), dim3(WAVE), dp->lds_bytes, s, P, O); break;
-        case 'S': hipLaunchKernelGGL((k_trace2d<real, 'S'>), dim3(tblocks), dim3(WAVE), dp->lds_bytes, s, P, O); break;
-        case 'P': hipLaunchKernelGGL((k_trace2d<real, 'P'>), dim3(tblocks), dim3(WAVE), dp->lds_bytes, s, P, O); break;
-        case 'N': hipLaunchKernelGGL((k_trace2d<real, 'N'>), dim3(tblocks), dim3(WAVE), dp->lds_bytes, s, P, O); break;
-        case 'Q': hipLaunchKernelGGL((k_trace2d<real, 'Q'>), dim3(tblocks), dim3(WAVE), dp->lds_bytes, s, P, O); break;
-        default: hipLaunchKernelGGL((k_trace2d<real, 'A'>), dim3(tblocks), dim3(WAVE), dp->lds_bytes, s, P, O); break;
+        } else {
+#define BHC_TRACE(ST)                                                                                                  \
+    if(dp->lds_bytes)                                                                                                  \
+        hipLaunchKernelGGL((k_trace2d<real, ST, true>), dim3(tblocks), dim3(WAVE), dp->lds_bytes, s, P, O);            \
+    else                                                                                                               \
+        hipLaunchKernelGGL((k_trace2d<real, ST, false>), dim3(tblocks), dim3(WAVE), 0, s, P, O);                       \
+    break;
+            switch(P.ssp_type) {
+            case 'C': BHC_TRACE('C')
+            case 'S': BHC_TRACE('S')
+            case 'P': BHC_TRACE('P')
+            case 'N': BHC_TRACE('N')
+            case 'Q': BHC_TRACE('Q')
+            default: BHC_TRACE('A')
+            }
+#undef BHC_TRACE
         }
         HIPCHECK(hipGetLastError());
         HIPCHECK(hipEventRecord(c->pb, s));
@@ -2242,6 +2336,8 @@ extern "C" int bhc_ray_runnx2d(bhc_ctx *ctx, const bhc_problem3d *prob, bhc_ray_
 // ===========================================================================
 namespace {
 
+// (p.y and q.y, the second components of p and q, reach no output of a sweep
+// and are not kept)
 template<typename real> struct RaySave {
     RayPt<real> p0;
     Trace<real> S;
@@ -2338,6 +2434,7 @@ __device__ __attribute__((noinline)) int run_problem(const BatchDev<real> &Bdref
         P.ray_xend = as_global(P.ray_xend);
     }
     const int nr = P.njobs;
+    const bool full = seg_full(P);
     bool pexh = false, active = false, init_fail = false;
     int result = 0;
     Err e = {0, 0, 0, 0};
@@ -2349,6 +2446,7 @@ __device__ __attribute__((noinline)) int run_problem(const BatchDev<real> &Bdref
     if(resume) {
         const RaySave<real> &sv = resume[lane];
         p0 = sv.p0;
+        p0.p.y = p0.q.y = (real)0;
         S = sv.S;
         I = sv.I;
         job = sv.job;
@@ -2405,7 +2503,9 @@ __device__ __attribute__((noinline)) int run_problem(const BatchDev<real> &Bdref
                 u = __shfl(u, 0);
                 if(lane == 0) Bd.save_out_pid[u] = pid;
                 RaySave<real> &sv = Bd.save_out[(size_t)u * WAVE + lane];
-                sv.p0 = p0;
+                RayPt<real> keep = p0;
+                keep.p.y = keep.q.y = (real)0;
+                sv.p0 = keep;
                 sv.S = S;
                 sv.I = I;
                 sv.job = job;
@@ -2417,41 +2517,24 @@ __device__ __attribute__((noinline)) int run_problem(const BatchDev<real> &Bdref
                 break;
             }
         }
-        RayPt<real> p1, p2;
-        SegDesc<real> d;
-        d.nitems = 0;
-        bool two = false;
-        if(active) {
-            two = RayUpdate<real, ST>(p0, p1, p2, S, P, B, G, e);
-            prelude<real, MODE != TRACE_DESC>(d, p0, p1, I, is, P, G, B + P.o_rzs, isz, ia);
-            d.prob = pid;
-            ++is;
-        }
-        if constexpr(MODE == TRACE_DESC) {
-            append_seg(d, lane, O, blk, seg_full(P));
-        } else {
-            DevSink<real> sink{&O, &P, 0};
-            seg_items<real, RT_TL, DevSink<real>, MODE == TRACE_FUSED_FAST>(d, P, G, P.Rz, sink);
-            contrib += sink.nc;
-        }
-        if(__any(two)) {
-            d.nitems = 0;
-            if(active && two) {
-                prelude<real, MODE != TRACE_DESC>(d, p1, p2, I, is, P, G, B + P.o_rzs, isz, ia);
+        step_ray<real, ST, MODE != TRACE_DESC>(
+            active, p0, S, I, is, P, B, G, isz, ia, e,
+            [&](bool has) {
+                if constexpr(MODE == TRACE_DESC) return reserve_seg<real>(has, lane, O, blk);
+                else return 0u;
+            },
+            [&](SegDesc<real> &d, uint32_t slot) {
                 d.prob = pid;
-                ++is;
-            }
-            if constexpr(MODE == TRACE_DESC) {
-                append_seg(d, lane, O, blk, seg_full(P));
-            } else {
-                DevSink<real> sink{&O, &P, 0};
-                seg_items<real, RT_TL, DevSink<real>, MODE == TRACE_FUSED_FAST>(d, P, G, P.Rz, sink);
-                contrib += sink.nc;
-            }
-        }
+                if constexpr(MODE == TRACE_DESC) {
+                    store_seg(d, slot, O, full);
+                } else {
+                    DevSink<real> sink{&O, &P, 0};
+                    seg_items<real, RT_TL, DevSink<real>, MODE == TRACE_FUSED_FAST>(d, P, G, P.Rz, sink);
+                    contrib += sink.nc;
+                }
+            });
         bool fin = false;
         if(active) {
-            p0 = two ? p2 : p1;
             if(RayTerminate(p0, is, S, MAXN, P, e)) {
                 active = false;
                 fin = true;
@@ -2881,7 +2964,7 @@ template<typename real> DevOut batch_out(bhc_sweep *sw)
     O.segs = c->segs;
     O.seg_count = c->d_seg_count;
     O.overflow = c->d_overflow;
-    O.seg_cap = (uint32_t)std::min<size_t>(c->seg_bytes / sizeof(Seg<real>), 0xFFFFFFF0u);
+    O.seg_cap = (uint32_t)std::min<size_t>(c->seg_bytes / sizeof(Seg<real>), SEG_CAP_MAX);
     O.prog = prog_of(c);
     return O;
 }
