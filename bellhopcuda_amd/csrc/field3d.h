@@ -745,11 +745,11 @@ int ray3d(bhc_ctx *c, const bhc_problem3d *p, bhc_ray_out3d *out, const bhc_eige
         (void)hipStreamSynchronize(s);
         void *ptrs[] = {d_blob, d_Rz, d_Sz, d_pts, d_ns, d_errw, d_hits};
         for(void *q : ptrs)
-            if(q) (void)hipFree(q);
+            c->pool.put(q);
     };
-    if(dalloc(&d_blob, blob.size()) || dalloc(&d_Rz, (size_t)p->NRz) || dalloc(&d_Sz, (size_t)p->NSz)
-       || dalloc(&d_pts, (size_t)njobs * M) || dalloc(&d_ns, (size_t)njobs) || dalloc(&d_errw, 4)
-       || (hits && dalloc(&d_hits, (size_t)njobs))) {
+    if(palloc(c, &d_blob, blob.size()) || palloc(c, &d_Rz, (size_t)p->NRz) || palloc(c, &d_Sz, (size_t)p->NSz)
+       || palloc(c, &d_pts, (size_t)njobs * M) || palloc(c, &d_ns, (size_t)njobs) || palloc(c, &d_errw, 4)
+       || (hits && palloc(c, &d_hits, (size_t)njobs))) {
         cleanup();
         return -1;
     }
@@ -822,7 +822,7 @@ template<typename real> int run3d(bhc_ctx *c, const bhc_problem3d *p, bhc_field_
         void *ptrs[] = {d_blob, d_Rz, d_Sz, d_field, d_stats, d_work, d_xend, d_cnt, d_errw,
                         d_cand, d_ncand, d_narr, d_neigen, d_arr, d_hits};
         for(void *q : ptrs)
-            if(q) (void)hipFree(q);
+            c->pool.put(q);
     };
     int rc = 0;
 #define TRY(x) \
@@ -841,16 +841,16 @@ template<typename real> int run3d(bhc_ctx *c, const bhc_problem3d *p, bhc_field_
             return -1; \
         } \
     } while(0)
-    TRY(dalloc(&d_blob, blob.size()));
-    TRY(dalloc(&d_Rz, (size_t)p->NRz));
-    TRY(dalloc(&d_Sz, (size_t)p->NSz));
-    TRY(dalloc(&d_field, 2 * nrcv));
-    TRY(dalloc(&d_work, 1));
-    TRY(dalloc(&d_cnt, 2));
-    TRY(dalloc(&d_errw, 4));
+    TRY(palloc(c, &d_blob, blob.size()));
+    TRY(palloc(c, &d_Rz, (size_t)p->NRz));
+    TRY(palloc(c, &d_Sz, (size_t)p->NSz));
+    TRY(palloc(c, &d_field, 2 * nrcv));
+    TRY(palloc(c, &d_work, 1));
+    TRY(palloc(c, &d_cnt, 2));
+    TRY(palloc(c, &d_errw, 4));
     if(out->ray_nsteps) {
-        TRY(dalloc(&d_stats, 3 * (size_t)njobs));
-        TRY(dalloc(&d_xend, 3 * (size_t)njobs));
+        TRY(palloc(c, &d_stats, 3 * (size_t)njobs));
+        TRY(palloc(c, &d_xend, 3 * (size_t)njobs));
     }
     HTRY(hipMemcpyAsync(d_blob, blob.data(), blob.size() * sizeof(real), hipMemcpyHostToDevice, s));
     HTRY(hipMemcpyAsync(d_Rz, p->Rz, p->NRz * sizeof(float), hipMemcpyHostToDevice, s));
@@ -868,15 +868,15 @@ template<typename real> int run3d(bhc_ctx *c, const bhc_problem3d *p, bhc_field_
         size_t want = 8 * (size_t)out->max_narr;
         if(cap < want && want * per <= ((size_t)64 << 30)) cap = want;
         cand_cap = (int)cap;
-        TRY(dalloc(&d_cand, nrcv * cap));
-        TRY(dalloc(&d_ncand, nrcv));
-        TRY(dalloc(&d_arr, nrcv * (size_t)out->max_narr));
-        TRY(dalloc(&d_narr, nrcv));
+        TRY(palloc(c, &d_cand, nrcv * cap));
+        TRY(palloc(c, &d_ncand, nrcv));
+        TRY(palloc(c, &d_arr, nrcv * (size_t)out->max_narr));
+        TRY(palloc(c, &d_narr, nrcv));
         HTRY(hipMemsetAsync(d_ncand, 0, nrcv * sizeof(int32_t), s));
     }
     if(hits_too) {
-        TRY(dalloc(&d_hits, (size_t)out->eigen_memsize));
-        TRY(dalloc(&d_neigen, 1));
+        TRY(palloc(c, &d_hits, (size_t)out->eigen_memsize));
+        TRY(palloc(c, &d_neigen, 1));
         HTRY(hipMemsetAsync(d_neigen, 0, sizeof(int32_t), s));
     }
     P.base = d_blob;

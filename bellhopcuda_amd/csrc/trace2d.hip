@@ -32,8 +32,10 @@
 #include <algorithm>
 #include <cmath>
 #include <atomic>
+#include <map>
 #include <mutex>
 #include <thread>
+#include <unordered_map>
 
 #include "../../include/bhc_hip.h"
 #include "core2d.h"
@@ -1192,6 +1194,102 @@ __global__ void __launch_bounds__(256) k_arr_merge(const ArrCand *cand, const in
 // ===========================================================================
 // Host side of the C ABI
 // ===========================================================================
+
+// Device blocks of a context that its problems and runs gave back, for the
+// next ones: a run allocates a dozen arrays, among them the arrivals'
+// candidate slots (up to 16 GiB, for which hipMalloc waits until the driver
+// has cleared as much memory: 249 ms for a 2121-receiver run whose kernels
+// take 7 ms, 4 ms when cleared memory was at hand). At most POOL_BYTES are
+// kept; destroying the context gives them back to the device, and any
+// allocation of the library that finds no memory first gives back those of
+// every context (bhc_give_back_pools). A block is put here only after the
+// context's stream has been waited for, so an idle block is in no one's use.
+constexpr size_t POOL_BYTES = size_t(20) << 30;
+struct DevPool;
+std::mutex g_pools_mu;
+std::vector<DevPool *> g_pools;                     // of every context
+struct DevPool {
+    std::mutex mu;
+    std::multimap<size_t, void *> idle;             // by size
+    std::unordered_map<void *, size_t> size;        // of every block handed out or idle
+    size_t held = 0;                                // bytes idle
+    DevPool()
+    {
+        std::lock_guard<std::mutex> lk(g_pools_mu);
+        g_pools.push_back(this);
+    }
+    ~DevPool()
+    {
+        {
+            std::lock_guard<std::mutex> lk(g_pools_mu);
+            g_pools.erase(std::find(g_pools.begin(), g_pools.end(), this));
+        }
+        trim();
+    }
+    void trim()
+    {
+        std::lock_guard<std::mutex> lk(mu);
+        for(auto &b : idle) {
+            (void)hipFree(b.second);
+            size.erase(b.second);
+        }
+        idle.clear();
+        held = 0;
+    }
+    // a block of at least n bytes, and at most twice that (or 1 MiB) from the idle ones
+    hipError_t get(void **p, size_t n);
+    void put(void *p)
+    {
+        if(!p) return;
+        std::lock_guard<std::mutex> lk(mu);
+        const size_t n = size[p];
+        if(held + n > POOL_BYTES) {
+            size.erase(p);
+            (void)hipFree(p);
+            return;
+        }
+        idle.emplace(n, p);
+        held += n;
+    }
+};
+
+void bhc_give_back_pools()
+{
+    std::lock_guard<std::mutex> lk(g_pools_mu);
+    for(DevPool *p : g_pools) p->trim();
+}
+
+// hipMalloc that gives the pools back before it gives up
+hipError_t bhc_device_malloc(void **p, size_t n)
+{
+    hipError_t e = hipMalloc(p, n);
+    if(e == hipSuccess) return e;
+    (void)hipGetLastError();
+    bhc_give_back_pools();
+    return hipMalloc(p, n);
+}
+
+hipError_t DevPool::get(void **p, size_t n)
+{
+    n = (n + 255) / 256 * 256;
+    {
+        std::lock_guard<std::mutex> lk(mu);
+        auto it = idle.lower_bound(n);
+        if(it != idle.end() && it->first <= std::max(2 * n, size_t(1) << 20)) {
+            *p = it->second;
+            held -= it->first;
+            idle.erase(it);
+            return hipSuccess;
+        }
+    }
+    const hipError_t e = bhc_device_malloc(p, n);
+    if(e == hipSuccess) {
+        std::lock_guard<std::mutex> lk(mu);
+        size[*p] = n;
+    }
+    return e;
+}
+
 struct bhc_ctx {
     int device;
     hipStream_t stream;
@@ -1226,6 +1324,7 @@ struct bhc_ctx {
     std::string async_msg;
     // device address of the static scratch array on this context's device
     void *scratch = nullptr;
+    DevPool pool;
 };
 
 namespace {
@@ -1505,7 +1604,16 @@ template<typename T> int dalloc(T **p, size_t n)
 {
     *p = nullptr;
     if(n == 0) return 0;
-    HIPCHECK(hipMalloc((void **)p, n * sizeof(T)));
+    HIPCHECK(bhc_device_malloc((void **)p, n * sizeof(T)));
+    return 0;
+}
+
+// dalloc from the context's pool (given back with ctx->pool.put)
+template<typename T> int palloc(bhc_ctx *c, T **p, size_t n)
+{
+    *p = nullptr;
+    if(n == 0) return 0;
+    HIPCHECK(c->pool.get((void **)p, n * sizeof(T)));
     return 0;
 }
 
@@ -1533,8 +1641,7 @@ extern "C" void bhc_problem_release(bhc_dev_problem *dp)
     void *ptrs[] = {dp->d_bins, dp->d_blob, dp->d_Rz,   dp->d_Sz,     dp->d_field,    dp->d_cand, dp->d_ncand,
                     dp->d_arr,  dp->d_narr, dp->d_hits,   dp->d_neigen,   dp->d_stats, dp->d_xend,
                     dp->d_counters, dp->d_errw, dp->d_work};
-    for(void *p : ptrs)
-        if(p) (void)hipFree(p);
+    for(void *p : ptrs) dp->ctx->pool.put(p);
     delete dp;
 }
 
@@ -1570,7 +1677,7 @@ extern "C" int bhc_problem_upload2d(bhc_ctx *ctx, const bhc_problem2d *prob, con
         if(!rc) {
             blob_bytes = blob.size() * sizeof(double);
             staged = (size_t)dp->P64.staged_reals * sizeof(double);
-            rc = dalloc((unsigned char **)&dp->d_blob, blob_bytes);
+            rc = palloc(ctx, (unsigned char **)&dp->d_blob, blob_bytes);
             if(!rc && hipMemcpy(dp->d_blob, blob.data(), blob_bytes, hipMemcpyHostToDevice) != hipSuccess)
                 rc = fail("blob upload failed");
         }
@@ -1582,7 +1689,7 @@ extern "C" int bhc_problem_upload2d(bhc_ctx *ctx, const bhc_problem2d *prob, con
         if(!rc) {
             blob_bytes = blob.size() * sizeof(float);
             staged = (size_t)dp->P32.staged_reals * sizeof(float);
-            rc = dalloc((unsigned char **)&dp->d_blob, blob_bytes);
+            rc = palloc(ctx, (unsigned char **)&dp->d_blob, blob_bytes);
             if(!rc && hipMemcpy(dp->d_blob, blob.data(), blob_bytes, hipMemcpyHostToDevice) != hipSuccess)
                 rc = fail("blob upload failed");
         }
@@ -1599,8 +1706,8 @@ extern "C" int bhc_problem_upload2d(bhc_ctx *ctx, const bhc_problem2d *prob, con
     }
     dp->P64.base = (const double *)dp->d_blob;
     dp->P32.base = (const float *)dp->d_blob;
-    if(dalloc(&dp->d_Rz, prob->NRz) || dalloc(&dp->d_Sz, prob->NSz) || dalloc(&dp->d_counters, 2)
-       || dalloc(&dp->d_errw, 4) || dalloc(&dp->d_work, 1)) {
+    if(palloc(ctx, &dp->d_Rz, prob->NRz) || palloc(ctx, &dp->d_Sz, prob->NSz) || palloc(ctx, &dp->d_counters, 2)
+       || palloc(ctx, &dp->d_errw, 4) || palloc(ctx, &dp->d_work, 1)) {
         bhc_problem_release(dp);
         return -1;
     }
@@ -1616,7 +1723,7 @@ extern "C" int bhc_problem_upload2d(bhc_ctx *ctx, const bhc_problem2d *prob, con
         bhc_problem_release(dp);
         return fail("unknown run type '%c'", r0);
     }
-    if(tl && dalloc(&dp->d_field, 2 * dp->nrcv)) {
+    if(tl && palloc(ctx, &dp->d_field, 2 * dp->nrcv)) {
         bhc_problem_release(dp);
         return -1;
     }
@@ -1641,7 +1748,7 @@ extern "C" int bhc_problem_upload2d(bhc_ctx *ctx, const bhc_problem2d *prob, con
             }
             size_t cap = ctx->seg_bytes / sizeof(Seg<float>);
             dp->max_chunks = (int)std::min<size_t>(cap / dp->chunk + dp->nbins + 1, 0x7FFFFFFF);
-            if(dalloc(&dp->d_bins, 3 * (size_t)dp->nbins + 1 + dp->max_chunks)) {
+            if(palloc(ctx, &dp->d_bins, 3 * (size_t)dp->nbins + 1 + dp->max_chunks)) {
                 bhc_problem_release(dp);
                 return -1;
             }
@@ -1660,8 +1767,8 @@ extern "C" int bhc_problem_upload2d(bhc_ctx *ctx, const bhc_problem2d *prob, con
         cap = std::min<size_t>(cap, 65536);
         cap = std::max<size_t>(cap, 8 * (size_t)dp->max_narr);
         dp->cand_cap = (int)cap;
-        if(dalloc(&dp->d_cand, dp->nrcv * cap) || dalloc(&dp->d_ncand, dp->nrcv)
-           || dalloc(&dp->d_arr, dp->nrcv * dp->max_narr) || dalloc(&dp->d_narr, dp->nrcv)) {
+        if(palloc(ctx, &dp->d_cand, dp->nrcv * cap) || palloc(ctx, &dp->d_ncand, dp->nrcv)
+           || palloc(ctx, &dp->d_arr, dp->nrcv * dp->max_narr) || palloc(ctx, &dp->d_narr, dp->nrcv)) {
             bhc_problem_release(dp);
             return -1;
         }
@@ -1672,13 +1779,13 @@ extern "C" int bhc_problem_upload2d(bhc_ctx *ctx, const bhc_problem2d *prob, con
             bhc_problem_release(dp);
             return fail("eigenray run needs eigen_memsize >= 1");
         }
-        if(dalloc(&dp->d_hits, dp->eigen_memsize) || dalloc(&dp->d_neigen, 1)) {
+        if(palloc(ctx, &dp->d_hits, dp->eigen_memsize) || palloc(ctx, &dp->d_neigen, 1)) {
             bhc_problem_release(dp);
             return -1;
         }
     }
     if(spec && spec->ray_nsteps) {
-        if(dalloc(&dp->d_stats, 3 * (size_t)dp->njobs) || dalloc(&dp->d_xend, 2 * (size_t)dp->njobs)) {
+        if(palloc(ctx, &dp->d_stats, 3 * (size_t)dp->njobs) || palloc(ctx, &dp->d_xend, 2 * (size_t)dp->njobs)) {
             bhc_problem_release(dp);
             return -1;
         }
@@ -1716,9 +1823,9 @@ int ensure_segs(bhc_ctx *c)
 {
     if(c->segs) return 0;
     c->seg_bytes = c->seg_mb << 20;
-    HIPCHECK(hipMalloc(&c->segs, c->seg_bytes));
+    HIPCHECK(bhc_device_malloc(&c->segs, c->seg_bytes));
     size_t maxseg = c->seg_bytes / sizeof(Seg<float>);
-    HIPCHECK(hipMalloc((void **)&c->d_bin_idx, maxseg * sizeof(uint32_t)));
+    HIPCHECK(bhc_device_malloc((void **)&c->d_bin_idx, maxseg * sizeof(uint32_t)));
     return 0;
 }
 
@@ -2069,16 +2176,16 @@ extern "C" int bhc_ray_run2d_list(bhc_ctx *ctx, const bhc_problem2d *prob, bhc_r
     bhc_ray_pt2d *d_pts = nullptr;
     int rc = 0;
     size_t npts = (size_t)njobs * out->max_points_per_ray;
-    if(dalloc(&d_pts, npts) || dalloc(&d_nout, njobs)) rc = -1;
+    if(palloc(ctx, &d_pts, npts) || palloc(ctx, &d_nout, njobs)) rc = -1;
     if(!rc && ialpha) {
-        if(dalloc(&d_ia, njobs) || dalloc(&d_isz, njobs)) rc = -1;
+        if(palloc(ctx, &d_ia, njobs) || palloc(ctx, &d_isz, njobs)) rc = -1;
         else {
             hipMemcpy(d_ia, ialpha, njobs * sizeof(int32_t), hipMemcpyHostToDevice);
             hipMemcpy(d_isz, isz, njobs * sizeof(int32_t), hipMemcpyHostToDevice);
         }
     }
     if(!rc && nsteps_in) {
-        if(dalloc(&d_nin, njobs)) rc = -1;
+        if(palloc(ctx, &d_nin, njobs)) rc = -1;
         else hipMemcpy(d_nin, nsteps_in, njobs * sizeof(int32_t), hipMemcpyHostToDevice);
     }
     if(!rc && njobs > 0) {
@@ -2109,7 +2216,7 @@ extern "C" int bhc_ray_run2d_list(bhc_ctx *ctx, const bhc_problem2d *prob, bhc_r
     }
     void *fr[] = {d_ia, d_isz, d_nin, d_nout, d_pts};
     for(void *p : fr)
-        if(p) (void)hipFree(p);
+        ctx->pool.put(p);
     bhc_problem_release(dp);
     if(!rc) ctx->prog_final = 1;
     return rc;
@@ -2205,26 +2312,26 @@ int upload_nx2d(bhc_ctx *ctx, const bhc_problem3d *p, const bhc_field_out *spec,
     dp->xend_dim = 3;
     int rc = 0;
     if(dp->d_xend) {
-        (void)hipFree(dp->d_xend);
+        ctx->pool.put(dp->d_xend);
         dp->d_xend = nullptr;
-        rc = dalloc(&dp->d_xend, 3 * (size_t)nj);
+        rc = palloc(ctx, &dp->d_xend, 3 * (size_t)nj);
     }
     // the Nx2D blob replaces the stand-in's
-    (void)hipFree(dp->d_blob);
+    ctx->pool.put(dp->d_blob);
     dp->d_blob = nullptr;
     std::string err;
     if(!rc && p->precision == 64) {
         std::vector<double> blob;
         rc = bhc3d::pack_nx<double>(p, blob, dp->N64, dp->P64, err);
         if(rc) fail("%s", err.c_str());
-        if(!rc) rc = dalloc((double **)&dp->d_blob, blob.size());
+        if(!rc) rc = palloc(ctx, (double **)&dp->d_blob, blob.size());
         if(!rc && hipMemcpy(dp->d_blob, blob.data(), blob.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess)
             rc = fail("blob upload failed");
     } else if(!rc) {
         std::vector<float> blob;
         rc = bhc3d::pack_nx<float>(p, blob, dp->N32, dp->P32, err);
         if(rc) fail("%s", err.c_str());
-        if(!rc) rc = dalloc((float **)&dp->d_blob, blob.size());
+        if(!rc) rc = palloc(ctx, (float **)&dp->d_blob, blob.size());
         if(!rc && hipMemcpy(dp->d_blob, blob.data(), blob.size() * sizeof(float), hipMemcpyHostToDevice) != hipSuccess)
             rc = fail("blob upload failed");
     }
@@ -2287,7 +2394,7 @@ extern "C" int bhc_ray_runnx2d(bhc_ctx *ctx, const bhc_problem3d *prob, bhc_ray_
     bhc_ray_pt2d *d_pts = nullptr;
     int rc = 0;
     const size_t npts = (size_t)njobs * out->max_points_per_ray;
-    if(dalloc(&d_pts, npts) || dalloc(&d_nout, njobs) || dalloc(&d_org, 4 * (size_t)njobs)) rc = -1;
+    if(palloc(ctx, &d_pts, npts) || palloc(ctx, &d_nout, njobs) || palloc(ctx, &d_org, 4 * (size_t)njobs)) rc = -1;
     if(!rc) {
         O.points = d_pts;
         O.nsteps_out = d_nout;
@@ -2314,7 +2421,7 @@ extern "C" int bhc_ray_runnx2d(bhc_ctx *ctx, const bhc_problem3d *prob, bhc_ray_
     }
     void *fr[] = {d_nout, d_pts, d_org};
     for(void *q : fr)
-        if(q) (void)hipFree(q);
+        ctx->pool.put(q);
     bhc_problem_release(dp);
     if(!rc) ctx->prog_final = 1;
     return rc;
