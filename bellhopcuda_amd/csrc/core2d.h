@@ -1355,17 +1355,71 @@ __host__ __device__ inline void seg_end(const SegGeo<real> &g, const RayPt<real>
     }
 }
 
-// cos and sin of an FP64 phase at FP32 accuracy: Cody-Waite reduction by 2*pi
-// in FP64 (two-part constant, exact to ~1e-11 rad for |a| < 1e6), then the FP32
-// sincos of the remainder in [-pi, pi].
+// cos and sin of an FP64 phase at FP32 accuracy. The quarter turns are counted
+// and taken off in FP64 (to 1e-10 rad for |a| < 1e6); the rest, within pi / 4,
+// goes through the Taylor polynomials of degree 9 and 8, whose remainders
+// (2e-9 and 3e-8) lie below the FP32 rounding. About 30 instructions; sincosf
+// with its own range reduction takes twice as many.
 __host__ __device__ inline void sincos_phase(double a, float &s, float &c)
 {
-    const double INV_2PI = 0.15915494309189535;
-    const double TWO_PI_HI = 6.283185307179586;       // 2*pi rounded to double
-    const double TWO_PI_LO = 2.4492935982947064e-16;  // 2*pi - TWO_PI_HI
-    double k = std::rint(a * INV_2PI);
-    double r = (a - k * TWO_PI_HI) - k * TWO_PI_LO;
-    sincosf((float)r, &s, &c);
+    const double y = a * 0.63661977236758134;            // 2 / pi
+    const double k = std::rint(y);
+    const float x = (float)((y - k) * 1.5707963267948966); // pi / 2
+    const int q = (int)(k - 4.0 * std::floor(0.25 * k));   // quarter turns modulo 4
+    const float x2 = x * x;
+    float ps = __builtin_fmaf(x2, 2.7557319e-6f, -1.9841270e-4f);
+    ps = __builtin_fmaf(x2, ps, 8.3333333e-3f);
+    ps = __builtin_fmaf(x2, ps, -0.16666667f);
+    ps = __builtin_fmaf(x * x2, ps, x);
+    float pc = __builtin_fmaf(x2, 2.4801587e-5f, -1.3888889e-3f);
+    pc = __builtin_fmaf(x2, pc, 4.1666667e-2f);
+    pc = __builtin_fmaf(x2, pc, -0.5f);
+    pc = __builtin_fmaf(x2, pc, 1.0f);
+    const float u = (q & 1) ? pc : ps, v = (q & 1) ? ps : pc;
+    s = (q & 2) ? -u : u;
+    c = ((q + 1) & 2) ? -v : v;
+}
+
+// 1 / x and 1 / sqrt(x) for the fast scatter: in FP64 on the GPU, the
+// hardware's estimate (24 bits) and two Newton steps, within an ulp or two of
+// the division, in half its instructions and without its scaling of
+// subnormals. FP32 keeps the division.
+template<typename real> __host__ __device__ inline real recip(real x)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    if constexpr(sizeof(real) == 8) {
+        double y = __builtin_amdgcn_rcp((double)x);
+        y = __builtin_fma(__builtin_fma(-(double)x, y, 1.0), y, y);
+        return (real)__builtin_fma(__builtin_fma(-(double)x, y, 1.0), y, y);
+    }
+#endif
+    return RL(1.0) / x;
+}
+template<typename real> __host__ __device__ inline real recip_sqrt(real x)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    if constexpr(sizeof(real) == 8) {
+        double y = __builtin_amdgcn_rsq((double)x);
+        const double h = 0.5 * (double)x;
+        y = __builtin_fma(__builtin_fma(-(h * y), y, 0.5), y, y);
+        return (real)__builtin_fma(__builtin_fma(-(h * y), y, 0.5), y, y);
+    }
+#endif
+    return RL(1.0) / std::sqrt(x);
+}
+
+// A field contribution at receiver (ir, iz) of source isz: to the sink's cell
+// if it takes cells, else to the field's index.
+template<typename real, typename Sink>
+__host__ __device__ inline auto put_field(Sink &sink, const Prob2D<real> &P, int isz, int iz, int ir, float fr, float fi, int)
+    -> decltype(sink.add_cell(P, isz, iz, ir, fr, fi))
+{
+    sink.add_cell(P, isz, iz, ir, fr, fi);
+}
+template<typename real, typename Sink>
+__host__ __device__ inline void put_field(Sink &sink, const Prob2D<real> &P, int isz, int iz, int ir, float fr, float fi, long)
+{
+    sink.add_field(P, ((size_t)isz * P.NRz_per_range + iz) * P.NRr + ir, fr, fi);
 }
 
 // InfluenceGeoCore (influence.hpp:897-1024, 2D) + ApplyContribution (:432-473).
@@ -1385,18 +1439,24 @@ __host__ __device__ inline void contrib(const SegDesc<real> &d, real s, real n1,
     real BW = P.isGaussian ? RL(4.0) : RL(1.0);
     if(n1 > BW * sigma || n1 == BW * sigma) return;
     cpx<real> delay = d.tau0 + rmul(s, d.dtau);
-    real cnst = d.A0 / std::sqrt(std::fabs(qFinal));
-    real w;
+    real cnst, w;
+    if constexpr(FAST) cnst = d.A0 * recip_sqrt(std::fabs(qFinal));
+    else cnst = d.A0 / std::sqrt(std::fabs(qFinal));
     if(P.isGaussian) {
-        real t = n1 / sigma;
-        if constexpr(FAST) w = (real)expf((float)(FL(-0.5) * (t * t))) * (sigma_orig / sigma);
-        else w = std::exp(FL(-0.5) * (t * t)) * (sigma_orig / sigma);
+        if constexpr(FAST) {
+            const real rs = recip(sigma);
+            const real t = n1 * rs;
+            w = (real)expf((float)(FL(-0.5) * (t * t))) * (sigma_orig * rs);
+        } else {
+            real t = n1 / sigma;
+            w = std::exp(FL(-0.5) * (t * t)) * (sigma_orig / sigma);
+        }
     } else {
-        w = (sigma - n1) / sigma;
+        if constexpr(FAST) w = (sigma - n1) * recip(sigma);
+        else w = (sigma - n1) / sigma;
     }
     real phaseInt = d.phasePt + d.phase;
     if(IsAtCaustic(d.qOld, qFinal)) phaseInt = d.phase + RC<real>::PI / FL(2.0);
-    size_t idx = ((size_t)d.isz * P.NRz_per_range + iz) * P.NRr + ir;
     real omega = FL(2.0) * RC<real>::PI * P.freq0;
     if constexpr(RT == RT_TL) {
         float fr, fi;
@@ -1407,7 +1467,8 @@ __host__ __device__ inline void contrib(const SegDesc<real> &d, real s, real n1,
                 // e^{-i arg} = e^{arg.im} (cos arg.re - i sin arg.re)
                 float sn, cs;
                 sincos_phase((double)arg.re, sn, cs);
-                float m = (float)(cnst * w) * expf((float)arg.im);
+                float m = (float)(cnst * w);
+                if(arg.im != (real)0) m *= expf((float)arg.im);
                 fr = m * cs;
                 fi = -(m * sn);
             } else {
@@ -1425,8 +1486,9 @@ __host__ __device__ inline void contrib(const SegDesc<real> &d, real s, real n1,
             fr = (float)v;
             fi = 0.0f;
         }
-        sink.add_field(P, idx, fr, fi);
+        put_field(sink, P, d.isz, iz, ir, fr, fi, 0);
     } else if constexpr(RT == RT_ARR) {
+        const size_t idx = ((size_t)d.isz * P.NRz_per_range + iz) * P.NRr + ir;
         sink.add_arrival(idx, cnst * w, phaseInt, delay, d.SrcDecl, d.RcvrDecl, d.ntop, d.nbot, d.ialpha, d.isz,
                          d.is);
         if(P.run0 == 'V' || P.run0 == 'v') sink.add_eigen(d.is, ir, iz, d.isz, d.ialpha);

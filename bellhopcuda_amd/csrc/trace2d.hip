@@ -767,16 +767,17 @@ template<typename real> struct TileSink {
     float *tile;          // LDS [tile_w][nz] complex
     int col0, tile_w, nz, nrr;
     unsigned long long nc;
-    __device__ void add_field(const Prob2D<real> &Pp, size_t idx, float re, float im)
+    // (the cell, not its index: an index would have to be divided back into
+    // range and depth, several hundred instructions of 64-bit division)
+    __device__ void add_cell(const Prob2D<real> &Pp, int isz, int iz, int ir, float re, float im)
     {
-        int ir = (int)(idx % (size_t)nrr);
-        int iz = (int)((idx / (size_t)nrr) % (size_t)nz);
-        int c = ir - col0;
-        if(c >= 0 && c < tile_w && (idx / ((size_t)nrr * nz)) == 0) {
+        const int c = ir - col0;
+        if(c >= 0 && c < tile_w && isz == 0) {
             int k = c * nz + iz; // real parts first, then imaginary parts (bank-conflict free)
             atomicAdd(tile + k, re);
             atomicAdd(tile + tile_w * nz + k, im);
         } else {
+            const size_t idx = ((size_t)isz * nz + iz) * nrr + ir;
             unsafeAtomicAdd(Pp.field + 2 * idx, re);
             unsafeAtomicAdd(Pp.field + 2 * idx + 1, im);
         }
