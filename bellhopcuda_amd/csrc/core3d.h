@@ -131,6 +131,7 @@ template<typename real> struct BState3 {
     int32_t ix, iy;
     real xmin, xmax, ymin, ymax;
     v3<real> x, xmid, n;
+    v2<real> tri;           // unit normal of the cell's diagonal (its depth component is 0)
     bool onEdge, side, justSteppedTo, outgoingSide;
     int32_t prov;           // 'L' grids: the current cell's province (CopyHSInfo, boundary.hpp:134-140)
 };
@@ -141,7 +142,21 @@ template<typename real> struct SSPOut3 {
     real rho, cxx, cyy, czz, cxy, cxz, cyz;
 };
 
+// Sound speed at a ray's current point, carried from the end of one step (or
+// from a reflection, which evaluates with the reflected tangent) to the start
+// of the next, which would evaluate the same point. `ok` is 0 at the ray's
+// start and where the evaluation raised an error or warning: the next step
+// then evaluates (again). The other second derivatives are zero in every
+// profile type.
+template<typename real> struct SSPAt3 {
+    v3<real> gradc;
+    cpx<real> c;
+    real czz;
+    int32_t ok;
+};
+
 template<typename real> struct Trace3 {
+    SSPAt3<real> at;
     int32_t sx, sy, sz, sr;     // SSP segment state
     BState3<real> top, bot;
     v3<real> xs;
@@ -151,6 +166,24 @@ template<typename real> struct Trace3 {
 // ---------------------------------------------------------------------------
 // SSP: Hexahedral (src/ssp.hpp:220-307) and the 3D EvaluateSSP (:377-465)
 // ---------------------------------------------------------------------------
+template<typename real> __host__ __device__ inline void carry3(SSPAt3<real> &a, const SSPOut3<real> &o, bool ok)
+{
+    a.gradc = o.gradc;
+    a.c = o.c;
+    a.czz = o.czz;
+    a.ok = ok;
+}
+template<typename real> __host__ __device__ inline SSPOut3<real> carried3(const SSPAt3<real> &a)
+{
+    SSPOut3<real> o;
+    o.gradc = a.gradc;
+    o.c = a.c;
+    o.rho = (real)0;        // not carried
+    o.czz = a.czz;
+    o.cxx = o.cyy = o.cxy = o.cxz = o.cyz = (real)0;
+    return o;
+}
+
 template<typename real>
 __host__ __device__ inline void EvaluateSSP3(v3<real> x, v3<real> t, SSPOut3<real> &o, const Prob3D<real> &P,
                                              Trace3<real> &S, Err &e)
@@ -218,53 +251,62 @@ __host__ __device__ inline void GetBdrySeg3(v3<real> x, v3<real> t, BState3<real
 { // prov: the grid's per-node extras when it has provinces, else null
 #define BX(i) bd[(size_t)(i) * NODE3 + 0]
 #define BY(i) bd[(size_t)(i) * NODE3 + 1]
-    b.ix = imin(imax(b.ix, 0), nx - 2);
-    b.iy = imin(imax(b.iy, 0), ny - 2);
-    if(t.x >= FL(0.0)) {
-        while(b.ix >= 0 && BX(b.ix * ny) > x.x) --b.ix;
-        while(b.ix >= 0 && b.ix < nx - 1 && BX((b.ix + 1) * ny) <= x.x) ++b.ix;
-    } else {
-        while(b.ix < nx - 1 && BX((b.ix + 1) * ny) < x.x) ++b.ix;
-        while(b.ix >= 0 && b.ix < nx - 1 && BX(b.ix * ny) >= x.x) --b.ix;
-    }
-    if(t.y >= FL(0.0)) {
-        while(b.iy >= 0 && BY(b.iy) > x.y) --b.iy;
-        while(b.iy >= 0 && b.iy < ny - 1 && BY(b.iy + 1) <= x.y) ++b.iy;
-    } else {
-        while(b.iy < ny - 1 && BY(b.iy + 1) < x.y) ++b.iy;
-        while(b.iy >= 0 && b.iy < ny - 1 && BY(b.iy) >= x.y) --b.iy;
-    }
-    if(b.ix == -1 && BX(0) == x.x) b.ix = 0;
-    if(b.ix == nx - 1 && BX((nx - 1) * ny) == x.x) b.ix = nx - 2;
-    if(b.iy == -1 && BY(0) == x.y) b.iy = 0;
-    if(b.iy == ny - 1 && BY(ny - 1) == x.y) b.iy = ny - 2;
-    if(b.ix < 0 || b.ix >= nx - 1 || b.iy < 0 || b.iy >= ny - 1) {
-        e.warning(isTop ? 6 : 7);
+    // Still in the cell: its data is kept, and only the side of the diagonal
+    // is looked at (no load from the grid, no square root or division). The
+    // tests are those under which the searches below stay where they are.
+    const bool same = !isInit
+        && (t.x >= FL(0.0) ? b.xmin <= x.x && x.x < b.xmax : b.xmin < x.x && x.x <= b.xmax)
+        && (t.y >= FL(0.0) ? b.ymin <= x.y && x.y < b.ymax : b.ymin < x.y && x.y <= b.ymax);
+    if(!same) {
         b.ix = imin(imax(b.ix, 0), nx - 2);
         b.iy = imin(imax(b.iy, 0), ny - 2);
-    }
-    b.xmin = BX(b.ix * ny);
-    b.xmax = BX((b.ix + 1) * ny);
-    b.ymin = BY(b.iy);
-    b.ymax = BY(b.iy + 1);
+        if(t.x >= FL(0.0)) {
+            while(b.ix >= 0 && BX(b.ix * ny) > x.x) --b.ix;
+            while(b.ix >= 0 && b.ix < nx - 1 && BX((b.ix + 1) * ny) <= x.x) ++b.ix;
+        } else {
+            while(b.ix < nx - 1 && BX((b.ix + 1) * ny) < x.x) ++b.ix;
+            while(b.ix >= 0 && b.ix < nx - 1 && BX(b.ix * ny) >= x.x) --b.ix;
+        }
+        if(t.y >= FL(0.0)) {
+            while(b.iy >= 0 && BY(b.iy) > x.y) --b.iy;
+            while(b.iy >= 0 && b.iy < ny - 1 && BY(b.iy + 1) <= x.y) ++b.iy;
+        } else {
+            while(b.iy < ny - 1 && BY(b.iy + 1) < x.y) ++b.iy;
+            while(b.iy >= 0 && b.iy < ny - 1 && BY(b.iy) >= x.y) --b.iy;
+        }
+        if(b.ix == -1 && BX(0) == x.x) b.ix = 0;
+        if(b.ix == nx - 1 && BX((nx - 1) * ny) == x.x) b.ix = nx - 2;
+        if(b.iy == -1 && BY(0) == x.y) b.iy = 0;
+        if(b.iy == ny - 1 && BY(ny - 1) == x.y) b.iy = ny - 2;
+        if(b.ix < 0 || b.ix >= nx - 1 || b.iy < 0 || b.iy >= ny - 1) {
+            e.warning(isTop ? 6 : 7);
+            b.ix = imin(imax(b.ix, 0), nx - 2);
+            b.iy = imin(imax(b.iy, 0), ny - 2);
+        }
+        b.xmin = BX(b.ix * ny);
+        b.xmax = BX((b.ix + 1) * ny);
+        b.ymin = BY(b.iy);
+        b.ymax = BY(b.iy + 1);
 #undef BX
 #undef BY
-    const real *n0 = bd + ((size_t)b.ix * ny + b.iy) * NODE3;
-    const real *n11 = bd + ((size_t)(b.ix + 1) * ny + (b.iy + 1)) * NODE3;
-    b.x = ld3(n0);
-    if(prov) b.prov = (int32_t)prov[((size_t)b.ix * ny + b.iy) * NODEX + NX_PROV];
-    v3<real> s = b.x + ld3(n11);
-    b.xmid = V3(s.x * RL(0.5), s.y * RL(0.5), s.z * RL(0.5));
-    v2<real> tri_n = V(-(b.ymax - b.ymin), b.xmax - b.xmin);
-    tri_n = dv(tri_n, std::sqrt(dot(tri_n, tri_n)));
+        const real *n0 = bd + ((size_t)b.ix * ny + b.iy) * NODE3;
+        const real *n11 = bd + ((size_t)(b.ix + 1) * ny + (b.iy + 1)) * NODE3;
+        b.x = ld3(n0);
+        if(prov) b.prov = (int32_t)prov[((size_t)b.ix * ny + b.iy) * NODEX + NX_PROV];
+        v3<real> s = b.x + ld3(n11);
+        b.xmid = V3(s.x * RL(0.5), s.y * RL(0.5), s.z * RL(0.5));
+        const v2<real> tri_n = V(-(b.ymax - b.ymin), b.xmax - b.xmin);
+        b.tri = dv(tri_n, std::sqrt(dot(tri_n, tri_n)));
+    }
     v2<real> temp = V(x.x - b.xmid.x, x.y - b.xmid.y);
-    real over = dot(temp, tri_n);
+    real over = dot(temp, b.tri);
+    const bool was = b.side;
     b.onEdge = std::fabs(over) < TD3<real>::THRESH;
     if(!isInit && b.justSteppedTo) b.side = b.outgoingSide;
-    else if(!isInit && b.onEdge) b.side = dot(V(t.x, t.y), tri_n) >= RL(0.0);
+    else if(!isInit && b.onEdge) b.side = dot(V(t.x, t.y), b.tri) >= RL(0.0);
     else b.side = over >= RL(0.0);
     b.justSteppedTo = false;
-    b.n = ld3(n0 + (b.side ? N3_N2 : N3_N1));
+    if(!same || b.side != was) b.n = ld3(bd + ((size_t)b.ix * ny + b.iy) * NODE3 + (b.side ? N3_N2 : N3_N1));
     if(!std::isfinite(b.x.z) || !std::isfinite(b.n.x) || !std::isfinite(b.n.y) || !std::isfinite(b.n.z)) e.error(3);
 }
 
@@ -279,29 +321,48 @@ template<typename real> __host__ __device__ inline void set3(v3<real> &a, int d,
     else a.z = v;
 }
 
+// The limits of a step inside its cells: the depth layer (the top and bottom
+// layers extrapolate: infinite there) and the x and y segment of the boundary
+// grids and the sound speed grid together.
+template<typename real> struct StepLim3 {
+    real z0, z1, x0, x1, y0, y1;
+};
+template<typename real>
+__host__ __device__ inline StepLim3<real> step_limits3(const int iSeg0[3], const Trace3<real> &S, const Prob3D<real> &P)
+{
+    StepLim3<real> L;
+    const real *z = P.base + P.o_z3;
+    L.z0 = iSeg0[2] > 0 ? z[iSeg0[2]] : -RC<real>::MAXV;
+    L.z1 = iSeg0[2] + 1 < P.nz3 - 1 ? z[iSeg0[2] + 1] : RC<real>::MAXV;
+    L.x0 = rmax(S.top.xmin, S.bot.xmin);
+    L.x1 = rmin(S.top.xmax, S.bot.xmax);
+    L.y0 = rmax(S.top.ymin, S.bot.ymin);
+    L.y1 = rmin(S.top.ymax, S.bot.ymax);
+    if(P.ssp3 == 'H') {
+        const real *wx = P.base + P.o_hx + iSeg0[0], *wy = P.base + P.o_hy + iSeg0[1];
+        L.x0 = rmax(L.x0, wx[0]);
+        L.x1 = rmin(L.x1, wx[1]);
+        L.y0 = rmax(L.y0, wy[0]);
+        L.y1 = rmin(L.y1, wy[1]);
+    }
+    return L;
+}
+
+// (here and in TopBotSegCrossing3 one division serves both sides of the cell)
 template<typename real>
 __host__ __device__ inline void DepthInterfaceCrossing3(bool stepTo, real &hInt, v3<real> &x, v3<real> x0,
-                                                        v3<real> u, int iz, const Prob3D<real> &P,
-                                                        int *snap = nullptr)
-{ // step.hpp:41-80 (3D: the top and bottom layers extrapolate); snap: the
-  // snapDim of OceanToRayX (Nx2D), set where the step is cut
+                                                        v3<real> u, const StepLim3<real> &L, int *snap = nullptr)
+{ // step.hpp:41-80 (3D); snap: the snapDim of OceanToRayX (Nx2D), set where
+  // the step is cut
     if(!stepTo) hInt = RC<real>::MAXV;
-    if(std::fabs(u.z) > RC<real>::EPS) {
-        const real *z = P.base + P.o_z3;
-        if(z[iz] > x.z && iz > 0) {
-            hInt = (z[iz] - x0.z) / u.z;
-            if(stepTo) {
-                x = x0 + sc3(hInt, u);
-                x.z = z[iz];
-                if(snap) *snap = 2;
-            }
-        } else if(z[iz + 1] < x.z && iz + 1 < P.nz3 - 1) {
-            hInt = (z[iz + 1] - x0.z) / u.z;
-            if(stepTo) {
-                x = x0 + sc3(hInt, u);
-                x.z = z[iz + 1];
-                if(snap) *snap = 2;
-            }
+    const bool above = L.z0 > x.z;
+    if((above || L.z1 < x.z) && std::fabs(u.z) > RC<real>::EPS) {
+        const real zi = above ? L.z0 : L.z1;
+        hInt = (zi - x0.z) / u.z;
+        if(stepTo) {
+            x = x0 + sc3(hInt, u);
+            x.z = zi;
+            if(snap) *snap = 2;
         }
     }
 }
@@ -345,39 +406,23 @@ __host__ __device__ inline void TopBotCrossing3(bool stepTo, real &h, const BSta
 }
 
 template<typename real>
-__host__ __device__ inline void TopBotSegCrossing3(bool stepTo, bool isY, real &hSeg, const Trace3<real> &S,
-                                                   int iSeg, v3<real> &x, v3<real> x0, v3<real> u,
-                                                   const Prob3D<real> &P, bool &topRefl, bool &botRefl,
+__host__ __device__ inline void TopBotSegCrossing3(bool stepTo, bool isY, real &hSeg, const StepLim3<real> &L,
+                                                   v3<real> &x, v3<real> x0, v3<real> u, bool &topRefl, bool &botRefl,
                                                    int *snap = nullptr)
 { // step.hpp:157-207
-    real lmin = rmax(isY ? S.top.ymin : S.top.xmin, isY ? S.bot.ymin : S.bot.xmin);
-    real lmax = rmin(isY ? S.top.ymax : S.top.xmax, isY ? S.bot.ymax : S.bot.xmax);
-    if(P.ssp3 == 'H') {
-        const real *sw = P.base + (isY ? P.o_hy : P.o_hx);
-        lmin = rmax(lmin, sw[iSeg]);
-        lmax = rmin(lmax, sw[iSeg + 1]);
-    }
+    const real lmin = isY ? L.y0 : L.x0, lmax = isY ? L.y1 : L.x1;
     real xw = isY ? x.y : x.x, x0w = isY ? x0.y : x0.x, uw = isY ? u.y : u.x;
     if(!stepTo) hSeg = RC<real>::MAXV;
-    if(std::fabs(uw) > RC<real>::EPS) {
-        if(xw < lmin) {
-            hSeg = -(x0w - lmin) / uw;
-            if(stepTo) {
-                x = x0 + sc3(hSeg, u);
-                if(isY) x.y = lmin;
-                else x.x = lmin;
-                if(snap) *snap = isY ? 1 : 0;
-                topRefl = botRefl = false;
-            }
-        } else if(xw > lmax) {
-            hSeg = -(x0w - lmax) / uw;
-            if(stepTo) {
-                x = x0 + sc3(hSeg, u);
-                if(isY) x.y = lmax;
-                else x.x = lmax;
-                if(snap) *snap = isY ? 1 : 0;
-                topRefl = botRefl = false;
-            }
+    const bool low = xw < lmin;
+    if((low || xw > lmax) && std::fabs(uw) > RC<real>::EPS) {
+        const real li = low ? lmin : lmax;
+        hSeg = -(x0w - li) / uw;
+        if(stepTo) {
+            x = x0 + sc3(hSeg, u);
+            if(isY) x.y = li;
+            else x.x = li;
+            if(snap) *snap = isY ? 1 : 0;
+            topRefl = botRefl = false;
         }
     }
 }
@@ -389,14 +434,13 @@ __host__ __device__ inline void TriDiagCrossing(bool stepTo, real &h, BState3<re
 { // step.hpp:212-260
     if(!stepTo) h = RC<real>::MAXV;
     if(bd.onEdge) return;
-    v3<real> d = x - bd.xmid, d0 = x0 - bd.xmid;
-    v3<real> tri_n = V3(-(bd.ymax - bd.ymin), bd.xmax - bd.xmin, (real)RL(0.0));
-    tri_n = dv3(tri_n, len3(tri_n));
-    real over = dot3(d, tri_n);
+    // the diagonal's normal has no depth component
+    const v2<real> d = V(x.x - bd.xmid.x, x.y - bd.xmid.y), d0 = V(x0.x - bd.xmid.x, x0.y - bd.xmid.y);
+    real over = dot(d, bd.tri);
     bool newSide = over >= RL(0.0);
     if(newSide == bd.side) return;
     if(std::fabs(over) < TD3<real>::THRESH) return;
-    real hnew = -dot3(d0, tri_n) / dot3(u, tri_n);
+    real hnew = -dot(d0, bd.tri) / dot(V(u.x, u.y), bd.tri);
     if(hnew < RL(0.0)) {
         e.warning(9);
         h = RL(0.0);
@@ -414,20 +458,20 @@ __host__ __device__ inline void TriDiagCrossing(bool stepTo, real &h, BState3<re
 }
 
 template<typename real>
-__host__ __device__ inline void ReduceStep3(v3<real> x0, v3<real> u, const int iSeg0[3], Trace3<real> &S,
+__host__ __device__ inline void ReduceStep3(v3<real> x0, v3<real> u, const StepLim3<real> &L, Trace3<real> &S,
                                             const Prob3D<real> &P, Err &e, real &h)
 { // step.hpp:271-337
     real hInt, hBx, hBy, hBz, hTop, hBot, hxS, hyS, hTD, hBD;
     bool dummy = false;
     v3<real> x = x0 + sc3(h, u);
-    DepthInterfaceCrossing3(false, hInt, x, x0, u, iSeg0[2], P);
+    DepthInterfaceCrossing3(false, hInt, x, x0, u, L);
     BeamBoxCrossing3(false, 0, hBx, x, x0, u, P, S.xs);
     BeamBoxCrossing3(false, 1, hBy, x, x0, u, P, S.xs);
     BeamBoxCrossing3(false, 2, hBz, x, x0, u, P, S.xs);
     TopBotCrossing3(false, hTop, S.top, x, x0, u, dummy);
     TopBotCrossing3(false, hBot, S.bot, x, x0, u, dummy);
-    TopBotSegCrossing3(false, false, hxS, S, iSeg0[0], x, x0, u, P, dummy, dummy);
-    TopBotSegCrossing3(false, true, hyS, S, iSeg0[1], x, x0, u, P, dummy, dummy);
+    TopBotSegCrossing3(false, false, hxS, L, x, x0, u, dummy, dummy);
+    TopBotSegCrossing3(false, true, hyS, L, x, x0, u, dummy, dummy);
     TriDiagCrossing(false, hTD, S.top, x, x0, u, dummy, dummy, e);
     TriDiagCrossing(false, hBD, S.bot, x, x0, u, dummy, dummy, e);
     h = rmin(rmin(rmin(h, hInt), rmin(rmin(rmin(hBx, hBy), hBz), rmin(hTop, hBot))), rmin(rmin(hxS, hyS), rmin(hTD, hBD)));
@@ -442,22 +486,22 @@ __host__ __device__ inline void ReduceStep3(v3<real> x0, v3<real> u, const int i
 
 template<typename real>
 __host__ __device__ inline void StepToBdry3(v3<real> x0, v3<real> &x2, v3<real> u, real &h, bool &topRefl,
-                                            bool &botRefl, const int iSeg0[3], Trace3<real> &S, const Prob3D<real> &P,
+                                            bool &botRefl, const StepLim3<real> &L, Trace3<real> &S, const Prob3D<real> &P,
                                             Err &e, int *snapDim = nullptr)
 { // step.hpp:342-420; snapDim (Nx2D): which ocean coordinate the step end
   // was put on exactly (common_run.hpp:243-252)
     int snap = -1;
     int *sp = snapDim ? &snap : nullptr;
     x2 = x0 + sc3(h, u);
-    DepthInterfaceCrossing3(true, h, x2, x0, u, iSeg0[2], P, sp);
+    DepthInterfaceCrossing3(true, h, x2, x0, u, L, sp);
     BeamBoxCrossing3(true, 0, h, x2, x0, u, P, S.xs, sp);
     BeamBoxCrossing3(true, 1, h, x2, x0, u, P, S.xs, sp);
     BeamBoxCrossing3(true, 2, h, x2, x0, u, P, S.xs, sp);
     TopBotCrossing3(true, h, S.top, x2, x0, u, topRefl, sp);
     TopBotCrossing3(true, h, S.bot, x2, x0, u, botRefl, sp);
     if(botRefl) topRefl = false;
-    TopBotSegCrossing3(true, false, h, S, iSeg0[0], x2, x0, u, P, topRefl, botRefl, sp);
-    TopBotSegCrossing3(true, true, h, S, iSeg0[1], x2, x0, u, P, topRefl, botRefl, sp);
+    TopBotSegCrossing3(true, false, h, L, x2, x0, u, topRefl, botRefl, sp);
+    TopBotSegCrossing3(true, true, h, L, x2, x0, u, topRefl, botRefl, sp);
     TriDiagCrossing(true, h, S.top, x2, x0, u, topRefl, botRefl, e, sp);
     TriDiagCrossing(true, h, S.bot, x2, x0, u, topRefl, botRefl, e, sp);
     if(h < RC<real>::INF_STEP * P.deltas) {
@@ -537,6 +581,18 @@ template<typename real>
 __host__ __device__ inline PQ3<real> DeltaPQ3(const Ray3<real> &ray, const SSPOut3<real> &o)
 { // Get_c_partials + ComputeDeltaPQ, step.hpp:425-473 (3D)
     const real c = o.c.re;
+    PQ3<real> pq;
+    const real tt = ray.t.x * ray.t.x + ray.t.y * ray.t.y;
+    pq.phi = (FL(1.0) / c) * ray.t.z * (ray.t.y * o.gradc.x - ray.t.x * o.gradc.y) / tt;
+    pq.q = mscl(c, ray.p);
+    // No second derivatives (the hexahedral grid and piecewise-linear
+    // profiles): p does not change, whatever the ray normals are as long as
+    // they are numbers.
+    if(o.cxx == (real)0 && o.cyy == (real)0 && o.czz == (real)0 && o.cxy == (real)0 && o.cxz == (real)0
+       && o.cyz == (real)0 && tt > (real)0 && std::isfinite(ray.phi)) {
+        pq.p = M2((real)0, (real)0, (real)0, (real)0);
+        return pq;
+    }
     v3<real> e1, e2;
     RayNormal3(ray.t, ray.phi, false, c, e1, e2);
     real cnn = o.cxx * (e1.x * e1.x) + o.cyy * (e1.y * e1.y) + o.czz * (e1.z * e1.z) + FL(2.0) * o.cxy * e1.x * e1.y
@@ -545,12 +601,8 @@ __host__ __device__ inline PQ3<real> DeltaPQ3(const Ray3<real> &ray, const SSPOu
         + o.cxz * (e1.x * e2.z + e2.x * e1.z) + o.cyz * (e1.y * e2.z + e2.y * e1.z);
     real cmm = o.cxx * (e2.x * e2.x) + o.cyy * (e2.y * e2.y) + o.czz * (e2.z * e2.z) + FL(2.0) * o.cxy * e2.x * e2.y
         + FL(2.0) * o.cxz * e2.x * e2.z + FL(2.0) * o.cyz * e2.y * e2.z;
-    PQ3<real> pq;
-    pq.phi = (FL(1.0) / c) * ray.t.z * (ray.t.y * o.gradc.x - ray.t.x * o.gradc.y)
-        / (ray.t.x * ray.t.x + ray.t.y * ray.t.y);
     m2<real> cm = mscl(-RL(1.0) / (c * c), M2(cnn, cmn, cmn, cmm));
     pq.p = mmul(ray.q, mtr(cm));
-    pq.q = mscl(c, ray.p);
     return pq;
 }
 
@@ -633,13 +685,15 @@ __host__ __device__ inline void Step3(const Ray3<real> &ray0, Ray3<real> &ray2, 
 { // step.hpp:654-811 (3D)
     Ray3<real> ray1;
     SSPOut3<real> o0, o1, o2;
-    EvaluateSSP3(ray0.x, ray0.t, o0, P, S, e);
+    if(S.at.ok) o0 = carried3(S.at);
+    else EvaluateSSP3(ray0.x, ray0.t, o0, P, S, e);
     PQ3<real> pq0 = DeltaPQ3(ray0, o0);
     const int iSeg0[3] = {S.sx, S.sy, S.sz};
+    const StepLim3<real> L = step_limits3(iSeg0, S, P);
     real c0 = o0.c.re, csq0 = c0 * c0;
     v3<real> u0 = sc3(c0, ray0.t);
     real h = P.deltas;
-    ReduceStep3(ray0.x, u0, iSeg0, S, P, e, h);
+    ReduceStep3(ray0.x, u0, L, S, P, e, h);
     real halfh = FL(0.5) * h;
     ray1.x = ray0.x + sc3(halfh, u0);
     ray1.t = ray0.t - dv3(sc3(halfh, o0.gradc), csq0);
@@ -648,23 +702,25 @@ __host__ __device__ inline void Step3(const Ray3<real> &ray0, Ray3<real> &ray2, 
     PQ3<real> pq1 = DeltaPQ3(ray1, o1);
     real c1 = o1.c.re, csq1 = c1 * c1;
     v3<real> u1 = sc3(c1, ray1.t);
-    ReduceStep3(ray0.x, u1, iSeg0, S, P, e, h);
+    ReduceStep3(ray0.x, u1, L, S, P, e, h);
     real w1 = h / (RL(2.0) * halfh);
     real w0 = RL(1.0) - w1;
     v3<real> u2 = sc3(w0, u0) + sc3(w1, u1);
     v3<real> x2;
-    StepToBdry3(ray0.x, x2, u2, h, topRefl, botRefl, iSeg0, S, P, e);
+    StepToBdry3(ray0.x, x2, u2, h, topRefl, botRefl, L, S, P, e);
     ray2.x = x2;
     real hw0 = h * w0, hw1 = h * w1;
     ray2.t = (ray0.t - dv3(sc3(hw0, o0.gradc), csq0)) - dv3(sc3(hw1, o1.gradc), csq1);
-    ray2.tau = ray0.tau + realdiv(hw0, o0.c) + realdiv(hw1, o1.c);
+    ray2.tau = ray0.tau + slowness_term(hw0, o0.c) + slowness_term(hw1, o1.c);
     UpdatePQ3(ray2, ray0, hw0, pq0);
     UpdatePQ3(ray2, ray2, hw1, pq1);
     ray2.Amp = ray0.Amp;
     ray2.Phase = ray0.Phase;
     ray2.NumTopBnc = ray0.NumTopBnc;
     ray2.NumBotBnc = ray0.NumBotBnc;
+    const uint32_t seen = e.nerr + e.nwarn;
     EvaluateSSP3(ray2.x, ray2.t, o2, P, S, e);
+    carry3(S.at, o2, e.nerr + e.nwarn == seen);
     ray2.c = o2.c.re;
     if(S.sz != iSeg0[2] || S.sx != iSeg0[0] || S.sy != iSeg0[1])
         CurvCorrSSP3(ray2, o2.gradc - o0.gradc, S.sz != iSeg0[2], S.sx != iSeg0[0]);
@@ -801,7 +857,9 @@ __host__ __device__ inline void Reflect3(const Ray3<real> &oldp, Ray3<real> &new
     newp.x = oldp.x;
     newp.t = oldp.t - sc3(FL(2.0) * Th, nB);
     SSPOut3<real> o;
+    const uint32_t seen = e.nerr + e.nwarn;
     EvaluateSSP3(oldp.x, newp.t, o, P, S, e);
+    carry3(S.at, o, e.nerr + e.nwarn == seen);
     real c = o.c.re;
     newp.c = c;
     newp.tau = oldp.tau;
@@ -894,6 +952,7 @@ __host__ __device__ inline bool RayInit3(int ia, int ib, int isx, int isy, int i
     const real *G = P.base;
     real alpha = G[P.o_alpha + ia];
     real SrcDecl = (RL(180.0) / RC<real>::PI) * alpha;
+    S.at.ok = 0;
     S.sx = S.sy = S.sz = S.sr = 0;
     S.xs = V3(G[P.o_Sx + isx], G[P.o_Sy + isy], (real)P.Sz[isz]);
     SSPOut3<real> o;

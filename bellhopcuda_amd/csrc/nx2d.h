@@ -72,11 +72,8 @@ __host__ __device__ inline v2<real> OceanToRayX(v3<real> x, const OrgNx<real> &o
 // EvaluateSSP with O3D && !R3D (ssp.hpp:377-465): the 3D profile at the ocean
 // point, its gradient and second derivatives projected on the bearing.
 template<typename real>
-__host__ __device__ inline void EvaluateSSPNx(v2<real> x, v2<real> t, SSPOut<real> &o, const Prob3D<real> &N,
-                                              Trace3<real> &S, const OrgNx<real> &org, Err &e)
+__host__ __device__ inline void ProjectSSPNx(const SSPOut3<real> &p, SSPOut<real> &o, const OrgNx<real> &org)
 {
-    SSPOut3<real> p;
-    EvaluateSSP3(RayToOceanX(x, org), RayToOceanT(t, org), p, N, S, e);
     o.gradc.x = dot(org.tr, V(p.gradc.x, p.gradc.y));
     o.gradc.y = p.gradc.z;
     o.crz = org.tr.x * p.cxz + org.tr.y * p.cyz;
@@ -84,6 +81,17 @@ __host__ __device__ inline void EvaluateSSPNx(v2<real> x, v2<real> t, SSPOut<rea
     o.c = p.c;
     o.rho = p.rho;
     o.czz = p.czz;
+}
+// KEEP: the evaluation is the next step's, carried in S.at (SSPAt3).
+template<typename real, bool KEEP = false>
+__host__ __device__ inline void EvaluateSSPNx(v2<real> x, v2<real> t, SSPOut<real> &o, const Prob3D<real> &N,
+                                              Trace3<real> &S, const OrgNx<real> &org, Err &e)
+{
+    SSPOut3<real> p;
+    const uint32_t seen = e.nerr + e.nwarn;
+    EvaluateSSP3(RayToOceanX(x, org), RayToOceanT(t, org), p, N, S, e);
+    if(KEEP) carry3(S.at, p, e.nerr + e.nwarn == seen);
+    ProjectSSPNx(p, o, org);
 }
 
 // Step (step.hpp:654-811, O3D && !R3D): the 2D polygon integration in ray
@@ -97,16 +105,18 @@ __host__ __device__ inline void StepNx(const RayPt<real> &ray0, RayPt<real> &ray
                                        bool &botRefl)
 {
     SSPOut<real> o0, o1, o2;
-    EvaluateSSPNx(ray0.x, ray0.t, o0, N, S, org, e);
+    if(S.at.ok) ProjectSSPNx(carried3(S.at), o0, org);
+    else EvaluateSSPNx(ray0.x, ray0.t, o0, N, S, org, e);
     real c0 = o0.c.re;
     real cnn0 = o0.crr * (ray0.t.y * ray0.t.y) - FL(2.0) * o0.crz * ray0.t.x * ray0.t.y + o0.czz * (ray0.t.x * ray0.t.x);
     v2<real> pq0p = sc(-cnn0, ray0.q), pq0q = sc(c0, ray0.p);
     const int iSeg0[3] = {S.sx, S.sy, S.sz};
+    const StepLim3<real> L = step_limits3(iSeg0, S, N);
     real csq0 = c0 * c0;
     v2<real> u0 = sc(c0, ray0.t);
     real h = N.deltas;
     const v3<real> x_o = RayToOceanX(ray0.x, org);
-    ReduceStep3(x_o, RayToOceanT(u0, org), iSeg0, S, N, e, h);
+    ReduceStep3(x_o, RayToOceanT(u0, org), L, S, N, e, h);
     real halfh = FL(0.5) * h;
     RayPt<real> ray1;
     ray1.x = ray0.x + sc(halfh, u0);
@@ -120,18 +130,18 @@ __host__ __device__ inline void StepNx(const RayPt<real> &ray0, RayPt<real> &ray
     v2<real> pq1p = sc(-cnn1, ray1.q), pq1q = sc(c1, ray1.p);
     real csq1 = c1 * c1;
     v2<real> u1 = sc(c1, ray1.t);
-    ReduceStep3(x_o, RayToOceanT(u1, org), iSeg0, S, N, e, h);
+    ReduceStep3(x_o, RayToOceanT(u1, org), L, S, N, e, h);
 
     real w1 = h / (RL(2.0) * halfh);
     real w0 = RL(1.0) - w1;
     v2<real> u2 = sc(w0, u0) + sc(w1, u1);
     v3<real> x2_o;
     int snap = -1;
-    StepToBdry3(x_o, x2_o, RayToOceanT(u2, org), h, topRefl, botRefl, iSeg0, S, N, e, &snap);
+    StepToBdry3(x_o, x2_o, RayToOceanT(u2, org), h, topRefl, botRefl, L, S, N, e, &snap);
     ray2.x = OceanToRayX(x2_o, org, u2, snap, e);
     real hw0 = h * w0, hw1 = h * w1;
     ray2.t = (ray0.t - dv(sc(hw0, o0.gradc), csq0)) - dv(sc(hw1, o1.gradc), csq1);
-    ray2.tau = (ray0.tau + realdiv(hw0, o0.c)) + realdiv(hw1, o1.c);
+    ray2.tau = (ray0.tau + slowness_term(hw0, o0.c)) + slowness_term(hw1, o1.c);
     ray2.p = ray0.p + sc(hw0, pq0p);
     ray2.q = ray0.q + sc(hw0, pq0q);
     ray2.p = ray2.p + sc(hw1, pq1p);
@@ -141,7 +151,7 @@ __host__ __device__ inline void StepNx(const RayPt<real> &ray0, RayPt<real> &ray
     ray2.NumTopBnc = ray0.NumTopBnc;
     ray2.NumBotBnc = ray0.NumBotBnc;
 
-    EvaluateSSPNx(ray2.x, ray2.t, o2, N, S, org, e);
+    EvaluateSSPNx<real, true>(ray2.x, ray2.t, o2, N, S, org, e);
     ray2.c = o2.c.re;
     if(S.sz != iSeg0[2]) { // CurvatureCorrection, step.hpp:624-648 (crossing in depth)
         v2<real> gj = o2.gradc - o0.gradc;
@@ -178,7 +188,7 @@ __host__ __device__ inline void ReflectNx(const RayPt<real> &oldp, RayPt<real> &
     newp.x = oldp.x;
     newp.t = oldp.t - sc(FL(2.0) * Th, nB);
     SSPOut<real> o;
-    EvaluateSSPNx(oldp.x, newp.t, o, N, S, org, e);
+    EvaluateSSPNx<real, true>(oldp.x, newp.t, o, N, S, org, e);
     real c = o.c.re;
     newp.c = c;
     newp.tau = oldp.tau;
@@ -221,7 +231,10 @@ __host__ __device__ inline void ReflectNx(const RayPt<real> &oldp, RayPt<real> &
         } else {
             newp.Amp = aR * oldp.Amp;
             newp.Phase = oldp.Phase + std::atan2(Refl.im, Refl.re);
-            if(P.type3 == 'S') BeamShift(oldp, newp, hs, tB, o, omega);
+            if(P.type3 == 'S') {
+                BeamShift(oldp, newp, hs, tB, o, omega);
+                S.at.ok = 0;   // the point has moved
+            }
         }
     } else {
         e.error(4);
@@ -255,6 +268,7 @@ __host__ __device__ inline bool RayInitNx(int ia, int ib, int isx, int isy, int 
     real alpha = G[N.o_alpha + ia];
     I.alpha = alpha;
     I.SrcDeclAngle = (RL(180.0) / RC<real>::PI) * alpha;
+    S.at.ok = 0;
     S.sx = S.sy = S.sz = S.sr = 0;
     S.xs = V3(G[N.o_Sx + isx], G[N.o_Sy + isy], (real)N.Sz[isz]);
     SSPOut3<real> o;
