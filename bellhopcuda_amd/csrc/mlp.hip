@@ -10,15 +10,16 @@
 //   network (TL at one receiver); n_out = K (a multiple of 32, <= 256) gives
 //   the K coefficients of a field expanded in a fixed basis. Weights are kept
 //   in FP32 (master, Adam state) and as a BF16 copy that the matrix products
-//   read; hidden activations are stored in BF16, pre-activations in FP32.
+//   read; hidden activations are stored in BF16, the GELU's slopes in FP32.
 //
-// Matrix products use v_mfma_f32_32x32x16_bf16: a workgroup of 4 wavefronts
-// computes a 64 x 64 tile of C = A * B, each wavefront one 32 x 32 block, with
-// A and B staged through LDS 32 columns of K at a time (converted to BF16 on
-// the way in, B transposed so that every lane reads its 8 K values as one
-// 16-byte LDS load). Operand element (m, k) of A is A[m * sam + k * sak] and
-// (k, n) of B is B[k * sbk + n * sbn], so the backward products read the
-// forward tensors transposed without copies. Members are the grid's z axis.
+// The rows of a batch are independent through the whole network, so k_rows
+// takes 32 of them from the inputs to the outputs and, in training, back to the
+// first layer's gradient in one launch: activations pass from layer to layer in
+// LDS, weights are read from the L2 in the matrix cores' operand order, and
+// only the GELU's slopes go to memory, FP32, for the thread that made them.
+// What the weight gradients need (activations and layer gradients, BF16) is
+// written in operand order too, so that k_wgrad reads both operands of H^T dZ
+// straight into registers. A training step is k_rows, k_wgrad and k_adam.
 #include <hip/hip_runtime.h>
 #include <algorithm>
 #include <cmath>
@@ -30,6 +31,9 @@
 #include <vector>
 
 #include "../../include/bhc_hip.h"
+
+// hipMalloc that gives idle blocks of the library's contexts back before it gives up
+hipError_t bhc_device_malloc(void **p, size_t n);
 
 namespace {
 
@@ -52,7 +56,8 @@ int mfail(const char *fmt, ...)
 
 constexpr int D_IN = 16, N_FREQ = 32, D_FF = 2 * N_FREQ, WIDTH = 256, N_HID = 6;
 constexpr int N_FREQ_RAW = (D_FF - D_IN) / 2; // projections used by front 1
-constexpr int TILE = 64, KSTEP = 32;
+constexpr int ROWS = 32;           // batch rows per workgroup of k_rows
+constexpr int NT_W = WIDTH / 32;   // 32-column tiles of a hidden layer
 
 typedef uint16_t bf16_t;
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
@@ -81,253 +86,407 @@ __host__ __device__ inline float bf2f(bf16_t h)
     memcpy(&f, &u, 4);
     return f;
 }
-__device__ inline bf16_t to_bf(float v) { return f2bf(v); }
-__device__ inline bf16_t to_bf(bf16_t v) { return v; }
+// The same rounding by the hardware's conversion (one instruction for two values).
+__device__ inline bf16_t cvt_bf(float f) { return __builtin_bit_cast(bf16_t, (__bf16)f); }
+// GELU (erf form) of z from c = 1 + erf(z / sqrt 2), and its derivative.
+__device__ inline float gelu_c(float z) { return 1.0f + erff(z * 0.70710678118654752f); }
+__device__ inline float gelu(float z, float c) { return 0.5f * z * c; }
+__device__ inline float gelu_d(float z, float c) { return 0.5f * c + z * 0.39894228040143268f * expf(-0.5f * z * z); }
 
-__device__ inline float gelu(float z) { return 0.5f * z * (1.0f + erff(z * 0.70710678118654752f)); }
-__device__ inline float gelu_d(float z)
+// Operand order of a K x N matrix: blocks of 16 K values by 32 columns, K-major,
+// NT = N / 32 blocks across; a block holds 64 lanes' 8 values, lane l those of
+// column l % 32 at K = 8 (l / 32) .. + 7 (v_mfma_f32_32x32x16_bf16's A and B).
+__host__ __device__ inline size_t op_at(int k, int n, int NT)
 {
-    return 0.5f * (1.0f + erff(z * 0.70710678118654752f)) + z * 0.39894228040143268f * expf(-0.5f * z * z);
+    return (((size_t)(k >> 4) * NT + (n >> 5)) * 64 + (n & 31) + 32 * ((k >> 3) & 1)) * 8 + (k & 7);
 }
 
-enum : int { EPI_STORE = 0, EPI_BIAS_GELU = 1, EPI_ATOMIC = 2, EPI_BIAS = 3 };
-
-struct GemmArgs {
-    const void *A;
-    const void *B;
-    float *C;
-    long long sam, sak, sbk, sbn, ldc;
-    long long zA, zB, zC;     // member strides (elements)
-    int M, N, K;
-    const float *bias;        // EPI_BIAS_GELU, EPI_BIAS: bias[n] (member stride zbias)
-    long long zbias;
-    bf16_t *H;                // EPI_BIAS_GELU: GELU(C) as BF16, same layout as C
-    int ksplit;               // EPI_ATOMIC: K is split over ksplit slices (grid z = members x ksplit)
+struct RowArgs {
+    const float *X, *Y;        // inputs [.][16] and targets [.][n_out]; row b of the batch is idx[b] (b without idx)
+    const int32_t *idx;
+    int n, n_out, front;
+    const float *Bf;           // [N_FREQ][D_IN]
+    const bf16_t *Wf, *Wb;     // weights in operand order, for the forward and the backward products
+    const float *P;            // FP32 parameters (biases)
+    long long np, npf;         // parameters and BF16 copy's elements per member
+    float *out;                // [members][n][n_out] (prediction)
+    bf16_t *F;                 // operand order over the batch rows: features,
+    bf16_t *H[N_HID], *dZ[N_HID], *dO; // activations, layer gradients and output gradient [member]
+    long long zH, zO;          // elements per member of H / dZ and of dO
+    float *D[N_HID];           // GELU'(Z) [member][row block][16][512]: each thread's own values
+    int members;
+    float *G, *loss;
 };
 
-// C = A * B (FP32); EPI_BIAS: C = A * B + bias; EPI_BIAS_GELU: C = A * B + bias
-// and H = GELU(C); EPI_ATOMIC: C += A * B over K slices.
-// M, N arbitrary (guarded), K a multiple of 32.
-template<typename TA, typename TB, int EPI>
-__global__ void __launch_bounds__(256) k_gemm(GemmArgs g)
+typedef __attribute__((__vector_size__(4 * sizeof(uint16_t)))) uint16_t u16x4;
+
+// The weights of one 32 x 32 product: column block nt of W (operand order, KT
+// blocks deep), and the product of the rows of act (LDS) with them.
+template<int KT> __device__ inline void load_w(bf16x8 *b, const bf16_t *W, int NT, int nt, int lane)
 {
-    __shared__ __align__(16) bf16_t As[TILE][KSTEP + 8];
-    __shared__ __align__(16) bf16_t Bt[TILE][KSTEP + 8];
-    const int ks = EPI == EPI_ATOMIC ? (int)(blockIdx.z % g.ksplit) : 0;
-    const int z = EPI == EPI_ATOMIC ? (int)(blockIdx.z / g.ksplit) : (int)blockIdx.z;
-    const TA *A = static_cast<const TA *>(g.A) + z * g.zA;
-    const TB *B = static_cast<const TB *>(g.B) + z * g.zB;
-    float *C = g.C + z * g.zC;
-    const int m0 = blockIdx.y * TILE, n0 = blockIdx.x * TILE;
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
-    int kbeg = 0, kend = g.K;
-    if constexpr(EPI == EPI_ATOMIC) {
-        int per = (g.K / KSTEP + g.ksplit - 1) / g.ksplit * KSTEP;
-        kbeg = ks * per;
-        kend = min(g.K, kbeg + per);
-    }
-    f32x16 acc = {};
-    for(int k0 = kbeg; k0 < kend; k0 += KSTEP) {
-        // stage A[m0 .. m0+63][k0 .. k0+31] and B[k0 .. +31][n0 .. +63] (transposed)
-        for(int i = t; i < TILE * KSTEP; i += 256) {
-            int r = i / KSTEP, c = i % KSTEP;
-            int m = m0 + r;
-            As[r][c] = m < g.M ? to_bf(A[m * g.sam + (long long)(k0 + c) * g.sak]) : (bf16_t)0;
-        }
-        for(int i = t; i < TILE * KSTEP; i += 256) {
-            int kk, nn;
-            if(g.sbn == 1) { // consecutive threads along n: coalesced reads
-                kk = i / TILE;
-                nn = i % TILE;
-            } else {
-                nn = i / KSTEP;
-                kk = i % KSTEP;
-            }
-            int n = n0 + nn;
-            Bt[nn][kk] = n < g.N ? to_bf(B[(long long)(k0 + kk) * g.sbk + n * g.sbn]) : (bf16_t)0;
-        }
-        __syncthreads();
 #pragma unroll
-        for(int kk = 0; kk < KSTEP; kk += 16) {
-            const int kq = kk + 8 * (lane >> 5);
-            bf16x8 a = *reinterpret_cast<const bf16x8 *>(&As[wm + (lane & 31)][kq]);
-            bf16x8 b = *reinterpret_cast<const bf16x8 *>(&Bt[wn + (lane & 31)][kq]);
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
+    for(int kt = 0; kt < KT; ++kt)
+        b[kt] = *reinterpret_cast<const bf16x8 *>(W + (((size_t)kt * NT + nt) * 64 + lane) * 8);
+}
+template<int KT> __device__ inline f32x16 row_product(const bf16_t (*act)[WIDTH + 8], const bf16x8 *b, int lane)
+{
+    f32x16 acc = {};
+#pragma unroll
+    for(int kt = 0; kt < KT; ++kt) {
+        bf16x8 a = *reinterpret_cast<const bf16x8 *>(&act[lane & 31][kt * 16 + 8 * (lane >> 5)]);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b[kt], acc, 0, 0, 0);
+    }
+    return acc;
+}
+
+// Row of accumulator register r in a 32 x 32 product (column: lane % 32).
+__device__ inline int acc_row(int r, int lane) { return 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3); }
+
+// The 16 values of a lane's column as BF16: rows of the next product's
+// activations in LDS (act, if given) and operand order over the batch rows
+// (op, if given: block row rb * 2, nt of NT).
+__device__ inline void put_cols(const float *v, bf16_t (*act)[WIDTH + 8], bf16_t *op, int rb, int NT, int nt, int lane)
+{
+#pragma unroll
+    for(int g = 0; g < 4; ++g) {
+        u16x4 q;
+#pragma unroll
+        for(int i = 0; i < 4; ++i) {
+            q[i] = cvt_bf(v[4 * g + i]);
+            if(act) act[acc_row(4 * g + i, lane)][nt * 32 + (lane & 31)] = q[i];
         }
-        __syncthreads();
-    }
-    // D layout: lane -> column wn + lane % 32; register r -> row
-    // wm + 8 (r / 4) + 4 (lane / 32) + r % 4
-    const int n = n0 + wn + (lane & 31);
-    if(n >= g.N) return;
-    for(int r = 0; r < 16; ++r) {
-        int m = m0 + wm + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        if(m >= g.M) continue;
-        float v = acc[r];
-        if constexpr(EPI == EPI_BIAS_GELU || EPI == EPI_BIAS) v += g.bias[z * g.zbias + n];
-        if constexpr(EPI == EPI_BIAS_GELU) g.H[z * g.zC + m * g.ldc + n] = f2bf(gelu(v));
-        if constexpr(EPI == EPI_ATOMIC) unsafeAtomicAdd(C + m * g.ldc + n, v);
-        else C[m * g.ldc + n] = v;
+        if(op)
+            *reinterpret_cast<u16x4 *>(op + (((size_t)(rb * 2 + (g >> 1)) * NT + nt) * 64 + (lane & 31) + 32 * (g & 1)) * 8
+                                       + 4 * (lane >> 5)) = q;
     }
 }
 
-// Features of normalised inputs x[b][16], stored BF16 (shared by all members).
-// Front 0: F[b][2j] = sin(2 pi <B_j, x_b>), F[b][2j+1] = cos(...), j < 32.
-// Front 1: F[b][d] = x[b][d] for d < 16, then sin / cos of projections j < 24
-// at F[b][16 + 2j], F[b][17 + 2j]. One thread per (b, j), j < 32; under
-// front 1 threads j >= 24 copy two inputs each.
-__global__ void k_features(const float *x, int n, const float *Bf, int front, bf16_t *F)
+// Sum of a lane's column over the 32 rows, added to *to once per column.
+__device__ inline void add_col(const float *v, float *to, int lane)
 {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if(i >= n * N_FREQ) return;
-    int b = i / N_FREQ, j = i % N_FREQ;
-    if(front == 1 && j >= N_FREQ_RAW) {
-        int d = 2 * (j - N_FREQ_RAW);
-        F[b * D_FF + d] = f2bf(x[b * D_IN + d]);
-        F[b * D_FF + d + 1] = f2bf(x[b * D_IN + d + 1]);
-        return;
-    }
     float s = 0.f;
-    for(int d = 0; d < D_IN; ++d) s += Bf[j * D_IN + d] * x[b * D_IN + d];
-    float sn, cs;
-    sincospif(2.0f * s, &sn, &cs);
-    const int o = front == 1 ? D_IN : 0;
-    F[b * D_FF + o + 2 * j] = f2bf(sn);
-    F[b * D_FF + o + 2 * j + 1] = f2bf(cs);
+#pragma unroll
+    for(int r = 0; r < 16; ++r) s += v[r];
+    s += __shfl_xor(s, 32);
+    if(lane < 32) unsafeAtomicAdd(to, s);
 }
 
-// Single-output layer: out[e][b] = <H[e][b][:], Wout[e]> + bout[e] (BF16
-// operands, FP32 sum). np = parameters per member.
-__global__ void k_out_fwd(const bf16_t *H, const bf16_t *Wbf, const float *P, int n, long long zH, long long zO,
-                          long long np, float *out)
+// ROWS batch rows of one member through the network, and in training (TRAIN)
+// the loss, the output gradient and every layer's gradient dZ back to the
+// first layer. Eight wavefronts, one 32-column tile of each layer apiece: two
+// per SIMD. 2048 rows of 4 members are 256 workgroups, one per CU. The vector
+// ALU bounds it: 12.6 million GELUs a step, whose erf and exp take some 65
+// instructions, made once (the slope is kept, not the pre-activation). A
+// layer's weights (128 KB per workgroup, from the L2) are loaded while the
+// layer before goes through its GELU.
+// Replaces one launch per layer and direction with FP32 pre-activations and
+// gradients in memory: a training step of 2048 rows, 4 members, 128 outputs
+// took 1270 us in 36 launches (28 us of it at the matrix cores' rate).
+template<bool TRAIN> __global__ void __launch_bounds__(512) k_rows(RowArgs g)
 {
-    int e = blockIdx.y, b = blockIdx.x * blockDim.x + threadIdx.x;
-    if(b >= n) return;
-    const bf16_t *h = H + e * zH + (long long)b * WIDTH;
-    const bf16_t *w = Wbf + e * np + OFF_WOUT;
-    float s = 0.f;
-    for(int k = 0; k < WIDTH; ++k) s += bf2f(h[k]) * bf2f(w[k]);
-    out[(long long)e * zO + b] = s + P[e * np + off_bout(1)];
-}
-
-// Loss and single-output backward for a batch: dOut = 2 (out - y) / n,
-// dH5[e][b][k] = dOut * Wout[k] (FP32), loss[e] += sum (out - y)^2 / n.
-__global__ void k_out_bwd(const float *out, const float *y, int n, const bf16_t *Wbf, float *dH, long long zH,
-                          long long zO, long long np, float *dout, float *loss)
-{
-    int e = blockIdx.y, b = blockIdx.x;
-    if(b >= n) return;
-    float d = out[(long long)e * zO + b] - y[b];
-    float g = 2.0f * d / (float)n;
-    if(threadIdx.x == 0) {
-        dout[(long long)e * zO + b] = g;
-        atomicAdd(loss + e, d * d / (float)n);
+    __shared__ __align__(16) bf16_t act[2][ROWS][WIDTH + 8];
+    __shared__ float grow[ROWS];   // single output: its gradient per row
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int rb = blockIdx.x, e = blockIdx.y, r0 = rb * ROWS;
+    const float *P = g.P + e * g.np;
+    const bf16_t *Wf = g.Wf + e * g.npf, *Wb = g.Wb + e * g.npf;
+    float *G = TRAIN ? g.G + e * g.np : nullptr;
+    const int col = wave * 32 + (lane & 31);
+    // features of normalised inputs. Front 0: F[2j] = sin(2 pi <B_j, x>),
+    // F[2j + 1] = cos, j < 32. Front 1: F[d] = x[d], d < 16, then sin / cos of
+    // projections j < 24 at F[16 + 2j], F[17 + 2j].
+    for(int i = t; i < ROWS * N_FREQ; i += 512) {
+        const int row = i / N_FREQ, j = i % N_FREQ, b = r0 + row;
+        float v0 = 0.f, v1 = 0.f;
+        int o = 2 * j;
+        if(g.front == 1) o = j >= N_FREQ_RAW ? 2 * (j - N_FREQ_RAW) : D_IN + 2 * j;
+        if(b < g.n) {
+            const float *x = g.X + (size_t)(g.idx ? g.idx[b] : b) * D_IN;
+            if(g.front == 1 && j >= N_FREQ_RAW) {
+                v0 = x[o];
+                v1 = x[o + 1];
+            } else {
+                float s = 0.f;
+                for(int d = 0; d < D_IN; ++d) s += g.Bf[j * D_IN + d] * x[d];
+                sincospif(2.0f * s, &v0, &v1);
+            }
+        }
+        act[0][row][o] = f2bf(v0);
+        act[0][row][o + 1] = f2bf(v1);
     }
-    const bf16_t *w = Wbf + e * np + OFF_WOUT;
-    for(int k = threadIdx.x; k < WIDTH; k += blockDim.x) dH[e * zH + (long long)b * WIDTH + k] = g * bf2f(w[k]);
-}
-
-// Loss and output gradient of a multi-output batch (K outputs per point):
-// dOut = 2 (out - y) / (n K), loss[e] += sum (out - y)^2 / (n K). One block of
-// 256 threads per (chunk of 256 elements, member).
-__global__ void k_out_loss(const float *out, const float *y, int total, long long zO, float *dout, float *loss)
-{
-    __shared__ float red[256];
-    int e = blockIdx.y, i = blockIdx.x * blockDim.x + threadIdx.x;
-    float d2 = 0.f;
-    if(i < total) {
-        float d = out[e * zO + i] - y[i];
-        dout[e * zO + i] = 2.0f * d / (float)total;
-        d2 = d * d / (float)total;
-    }
-    red[threadIdx.x] = d2;
     __syncthreads();
-    for(int h = 128; h > 0; h >>= 1) {
-        if((int)threadIdx.x < h) red[threadIdx.x] += red[threadIdx.x + h];
+    if(TRAIN && e == 0 && t < 256) { // features in operand order over the rows
+        const int kt = t >> 7, nt = (t >> 6) & 1, c = nt * 32 + (lane & 31), k0 = kt * 16 + 8 * (lane >> 5);
+        alignas(16) bf16_t q[8];
+        for(int j = 0; j < 8; ++j) q[j] = act[0][k0 + j][c];
+        *reinterpret_cast<uint4 *>(g.F + (((size_t)(rb * 2 + kt) * 2 + nt) * 64 + lane) * 8) = *reinterpret_cast<uint4 *>(q);
+    }
+    // GELU' (FP32) of this lane's column, kept for the way back
+    const size_t ds = ((size_t)e * gridDim.x + rb) * 16 * 512 + t;
+    int cur = 0;
+    bf16x8 w[WIDTH / 16];
+    load_w<D_FF / 16>(w, Wf, NT_W, wave, lane);
+#pragma unroll 1
+    for(int l = 0; l < N_HID; ++l) {
+        const f32x16 acc = l == 0 ? row_product<D_FF / 16>(act[cur], w, lane) : row_product<WIDTH / 16>(act[cur], w, lane);
+        const float bias = P[off_b(l) + col];
+        if(l + 1 < N_HID) load_w<WIDTH / 16>(w, Wf + off_W(l + 1), NT_W, wave, lane);
+        float h[16];
+#pragma unroll
+        for(int r = 0; r < 16; ++r) {
+            const float z = acc[r] + bias, c = gelu_c(z);
+            if(TRAIN) g.D[l][ds + r * 512] = gelu_d(z, c);
+            h[r] = gelu(z, c);
+        }
+        put_cols(h, act[cur ^ 1], TRAIN ? g.H[l] + e * g.zH : nullptr, rb, NT_W, wave, lane);
+        cur ^= 1;
         __syncthreads();
     }
-    if(threadIdx.x == 0) atomicAdd(loss + e, red[0]);
-}
-
-constexpr int RCHUNK = 128; // batch rows per block of the column reductions
-
-// Single output: dWout[e][k] += sum over a chunk of b of H5[e][b][k] dOut[e][b];
-// dbout likewise (G's output-layer slots are zeroed first).
-__global__ void k_out_wgrad(const bf16_t *H, const float *dout, int n, long long zH, long long zO, long long np,
-                            float *G)
-{
-    int e = blockIdx.y, k = threadIdx.x;
-    int b0 = blockIdx.x * RCHUNK, b1 = min(n, b0 + RCHUNK);
-    float s = 0.f;
-    if(k < WIDTH) {
-        for(int b = b0; b < b1; ++b) s += bf2f(H[e * zH + (long long)b * WIDTH + k]) * dout[(long long)e * zO + b];
-        unsafeAtomicAdd(G + e * np + OFF_WOUT + k, s);
-    } else if(k == WIDTH) {
-        for(int b = b0; b < b1; ++b) s += dout[(long long)e * zO + b];
-        unsafeAtomicAdd(G + e * np + off_bout(1), s);
+    // output layer, and in training the loss and its gradient
+    float lsum = 0.f;
+    const float total = (float)(g.n * g.n_out);
+    if(g.n_out == 1) {
+        for(int k = 0; k < 4; ++k) {
+            const int row = wave * 4 + k;
+            float s = 0.f;
+            for(int j = 0; j < 4; ++j) s += bf2f(act[cur][row][lane * 4 + j]) * bf2f(Wf[OFF_WOUT + lane * 4 + j]);
+            for(int o = 32; o; o >>= 1) s += __shfl_xor(s, o);
+            s += P[off_bout(1)];
+            const int b = r0 + row;
+            if(lane == 0 && b < g.n) {
+                if(TRAIN) {
+                    const float d = s - g.Y[g.idx ? g.idx[b] : b];
+                    grow[row] = 2.0f * d / total;
+                    lsum += d * d / total;
+                } else {
+                    g.out[(size_t)e * g.n + b] = s;
+                }
+            }
+        }
+        if(!TRAIN) return;
+        __syncthreads();
+        if(t < WIDTH) {
+            float s = 0.f;
+            for(int r = 0; r < ROWS; ++r) s += bf2f(act[cur][r][t]) * grow[r];
+            unsafeAtomicAdd(G + OFF_WOUT + t, s);
+        } else if(t == WIDTH) {
+            float s = 0.f;
+            for(int r = 0; r < ROWS; ++r) s += grow[r];
+            unsafeAtomicAdd(G + off_bout(1), s);
+        }
+    } else {
+        const int NT = g.n_out / 32;
+        if(wave < NT) {
+            load_w<WIDTH / 16>(w, Wf + OFF_WOUT, NT, wave, lane);
+            const f32x16 acc = row_product<WIDTH / 16>(act[cur], w, lane);
+            const float bias = P[off_bout(g.n_out) + col];
+            float d[16];
+#pragma unroll
+            for(int r = 0; r < 16; ++r) {
+                const int b = r0 + acc_row(r, lane);
+                const float v = acc[r] + bias;
+                d[r] = 0.f;
+                if(b < g.n) {
+                    if(TRAIN) {
+                        const float df = v - g.Y[(size_t)(g.idx ? g.idx[b] : b) * g.n_out + col];
+                        lsum += df * df / total;
+                        d[r] = 2.0f * df / total;
+                    } else {
+                        g.out[((size_t)e * g.n + b) * g.n_out + col] = v;
+                    }
+                }
+            }
+            if(TRAIN) {
+                add_col(d, G + off_bout(g.n_out) + col, lane);
+                put_cols(d, act[cur ^ 1], g.dO + (size_t)e * g.zO, rb, NT, wave, lane);
+            }
+        }
+        if(!TRAIN) return;
+        cur ^= 1;
+        __syncthreads();
+    }
+    for(int o = 32; o; o >>= 1) lsum += __shfl_xor(lsum, o);
+    if(lane == 0) unsafeAtomicAdd(g.loss + e, lsum);
+    // back through the layers: dZ_l = (dZ_{l+1} W_{l+1}^T) GELU'(Z_l)
+#pragma unroll 1
+    for(int l = N_HID - 1; l >= 0; --l) {
+        float d[16], slope[16];
+#pragma unroll
+        for(int r = 0; r < 16; ++r) slope[r] = g.D[l][ds + r * 512];
+        if(l == N_HID - 1 && g.n_out == 1) {
+            const float wo = bf2f(Wf[OFF_WOUT + col]);
+#pragma unroll
+            for(int r = 0; r < 16; ++r) d[r] = grow[acc_row(r, lane)] * wo;
+        } else {
+            f32x16 acc = {};
+            if(l == N_HID - 1) {
+                const bf16_t *W = Wb + OFF_WOUT;
+                for(int kt = 0; kt < g.n_out / 16; ++kt) {
+                    bf16x8 b = *reinterpret_cast<const bf16x8 *>(W + (((size_t)kt * NT_W + wave) * 64 + lane) * 8);
+                    bf16x8 a = *reinterpret_cast<const bf16x8 *>(&act[cur][lane & 31][kt * 16 + 8 * (lane >> 5)]);
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
+                }
+            } else {
+                acc = row_product<WIDTH / 16>(act[cur], w, lane);
+            }
+#pragma unroll
+            for(int r = 0; r < 16; ++r) d[r] = acc[r];
+        }
+        if(l > 0) load_w<WIDTH / 16>(w, Wb + off_W(l), NT_W, wave, lane);
+#pragma unroll
+        for(int r = 0; r < 16; ++r) d[r] *= slope[r];
+        add_col(d, G + off_b(l) + col, lane);
+        put_cols(d, l > 0 ? act[cur ^ 1] : nullptr, g.dZ[l] + e * g.zH, rb, NT_W, wave, lane);
+        cur ^= 1;
+        __syncthreads();
     }
 }
 
-// zero the gradient slots that are accumulated by atomics: biases, output
-// layer, and the weights of the split-K products
+// Weight gradients dW = H^T dZ of every layer and member: one workgroup per
+// 64 x 32 tile, its four wavefronts splitting the batch rows; both operands
+// come in operand order, 16 bytes per lane, and the four partial tiles are
+// summed in LDS in a fixed order. A layer's tiles read the same two matrices
+// (2 MB at 2048 rows), so the workgroups of one (layer, member) are dealt to
+// one XCD (workgroups go to the eight XCDs in turn) and share its L2.
+constexpr int WG_TILES = (WIDTH / 64) * NT_W;
+__global__ void __launch_bounds__(256) k_wgrad(RowArgs g)
+{
+    const int n = g.n, n_out = g.n_out, members = g.members;
+    __shared__ float part[4][64 * 32];
+    const int nlayer = n_out > 1 ? N_HID + 1 : N_HID;
+    const int q = blockIdx.x >> 3, combo = (blockIdx.x & 7) + 8 * (q / WG_TILES), tile = q % WG_TILES;
+    if(combo >= nlayer * members) return;
+    const int l = combo % nlayer, e = combo / nlayer;
+    const int Kin = l == 0 ? D_FF : WIDTH, N = l == N_HID ? n_out : WIDTH;
+    const int NTa = Kin / 32, NTb = N / 32;
+    const int mp = tile / NTb, nt = tile % NTb;
+    if(mp >= Kin / 64) return;
+    const bf16_t *A = l == 0 ? g.F : g.H[l - 1] + e * g.zH;
+    const bf16_t *B = l == N_HID ? g.dO + e * g.zO : g.dZ[l] + e * g.zH;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int nk = n / 16, k0 = wave * nk / 4, k1 = (wave + 1) * nk / 4;
+    f32x16 c0 = {}, c1 = {};
+    for(int kt = k0; kt < k1; ++kt) {
+        const bf16_t *a = A + (((size_t)kt * NTa + 2 * mp) * 64 + lane) * 8;
+        bf16x8 a0 = *reinterpret_cast<const bf16x8 *>(a), a1 = *reinterpret_cast<const bf16x8 *>(a + 512);
+        bf16x8 b = *reinterpret_cast<const bf16x8 *>(B + (((size_t)kt * NTb + nt) * 64 + lane) * 8);
+        c0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, b, c0, 0, 0, 0);
+        c1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, b, c1, 0, 0, 0);
+    }
+    for(int r = 0; r < 16; ++r) {
+        part[wave][acc_row(r, lane) * 32 + (lane & 31)] = c0[r];
+        part[wave][(32 + acc_row(r, lane)) * 32 + (lane & 31)] = c1[r];
+    }
+    __syncthreads();
+    float *W = g.G + e * g.np + off_W(l);
+    for(int i = t; i < 64 * 32; i += 256)
+        W[(size_t)(mp * 64 + (i >> 5)) * N + nt * 32 + (i & 31)] = part[0][i] + part[1][i] + part[2][i] + part[3][i];
+}
+
+// Weight tiles of 32 x 32 in a member, layer by layer, K-major within a layer
+// (the output layer's only with several outputs).
+__host__ __device__ inline int n_tiles(int n_out)
+{
+    return (D_FF / 32 + (N_HID - 1) * NT_W) * NT_W + (n_out > 1 ? NT_W * (n_out / 32) : 0);
+}
+struct WTile {
+    size_t W;                  // the layer's first weight
+    int N, k0, n0, layer;
+};
+__device__ inline WTile w_tile(int q, int n_out)
+{
+    WTile t;
+    const int first = (D_FF / 32) * NT_W;
+    if(q < first) t.layer = 0;
+    else {
+        q -= first;
+        t.layer = 1 + min(q / (NT_W * NT_W), N_HID - 1);
+        q -= (t.layer - 1) * NT_W * NT_W;
+    }
+    t.W = off_W(t.layer);
+    t.N = t.layer == N_HID ? n_out : WIDTH;
+    t.k0 = q / (t.N / 32) * 32;
+    t.n0 = q % (t.N / 32) * 32;
+    return t;
+}
+
+// The BF16 copies of a tile (tile[k][n], by the 256 threads of a workgroup) in
+// operand order for both directions, 16 bytes per thread.
+__device__ inline void put_tile(const bf16_t (*tile)[34], const WTile &w, bf16_t *Wf, bf16_t *Wb)
+{
+    const int t = threadIdx.x & 127, kt = t >> 6, lane = t & 63, c = lane & 31, r0 = kt * 16 + 8 * (lane >> 5);
+    alignas(16) bf16_t q[8];
+    if(threadIdx.x < 128) { // K = row, N = column
+        for(int j = 0; j < 8; ++j) q[j] = tile[r0 + j][c];
+        *reinterpret_cast<uint4 *>(Wf + w.W + op_at(w.k0 + r0, w.n0 + c, w.N / 32)) = *reinterpret_cast<uint4 *>(q);
+    } else if(w.layer > 0) { // K = column, N = row
+        for(int j = 0; j < 8; ++j) q[j] = tile[c][r0 + j];
+        *reinterpret_cast<uint4 *>(Wb + w.W + op_at(w.n0 + r0, w.k0 + c, NT_W)) = *reinterpret_cast<uint4 *>(q);
+    }
+}
+
+// Parameter number j of those that are no tile's: the biases layer by layer,
+// then a single output's weights; -1 past the last.
+__device__ inline long long loose_param(int j, int n_out)
+{
+    if(j < N_HID * WIDTH) return (long long)off_b(j / WIDTH) + j % WIDTH;
+    j -= N_HID * WIDTH;
+    if(j < n_out) return (long long)off_bout(n_out) + j;
+    j -= n_out;
+    return n_out == 1 && j < WIDTH ? (long long)OFF_WOUT + j : -1;
+}
+__host__ __device__ inline int n_loose(int n_out) { return N_HID * WIDTH + n_out + (n_out == 1 ? WIDTH : 0); }
+
 __global__ void k_zero(float *p, long long n)
 {
     long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if(i < n) p[i] = 0.0f;
 }
 
-// dZ = dH * GELU'(Z) in place of dH (FP32).
-__global__ void k_gelu_bwd(float *dH, const float *Z, long long total)
+// Adam (FP32 master weights), the BF16 copies the products read, and zeros for
+// the next step's loss and for the gradients that k_rows adds to (biases, a
+// single output's weights). One workgroup per 32 x 32 tile of weights, which
+// goes through LDS so that both copies are stored 16 bytes at a time; the last
+// workgroups take the loose parameters. Member: blockIdx.y. STEP = false only
+// makes the copies.
+template<bool STEP>
+__global__ void __launch_bounds__(256) k_adam(float *Pm, float *M, float *V, float *Gm, bf16_t *Wf, bf16_t *Wb, long long np,
+                                              long long npf, int n_out, float lr, float b1, float b2, float eps, float c1,
+                                              float c2, float *next_loss)
 {
-    long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if(i < total) dH[i] *= gelu_d(Z[i]);
-}
-
-// db[e][c] += sum over a chunk of b of dZ[e][b][c], c < cols (one thread per
-// column, rows of `cols` values).
-__global__ void k_bias_grad(const float *dZ, int n, int cols, long long zZ, long long np, float *G, size_t off)
-{
-    int e = blockIdx.y, c = threadIdx.x;
-    int b0 = blockIdx.x * RCHUNK, b1 = min(n, b0 + RCHUNK);
-    if(c >= cols) return;
-    float s = 0.f;
-    for(int b = b0; b < b1; ++b) s += dZ[e * zZ + (long long)b * cols + c];
-    unsafeAtomicAdd(G + e * np + off + c, s);
-}
-
-// Adam (FP32 master weights) and the BF16 copy the products read.
-__global__ void k_adam(float *P, float *M, float *V, const float *G, bf16_t *Pbf, long long total, float lr,
-                       float b1, float b2, float eps, float c1, float c2)
-{
-    long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if(i >= total) return;
-    float g = G[i];
-    float m = b1 * M[i] + (1.0f - b1) * g;
-    float v = b2 * V[i] + (1.0f - b2) * g * g;
-    M[i] = m;
-    V[i] = v;
-    float p = P[i] - lr * (m / c1) / (sqrtf(v / c2) + eps);
-    P[i] = p;
-    Pbf[i] = f2bf(p);
-}
-
-__global__ void k_to_bf(const float *P, bf16_t *Pbf, long long total)
-{
-    long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if(i < total) Pbf[i] = f2bf(P[i]);
-}
-
-// Batch gather from the resident training set: idx[b] -> x[b][16], y[b][n_out].
-__global__ void k_gather(const float *X, const float *Y, const int32_t *idx, int n, int n_out, float *x, float *y)
-{
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int row = D_IN + n_out;
-    if(i >= n * row) return;
-    int b = i / row, d = i % row;
-    long long s = idx[b];
-    if(d < D_IN) x[b * D_IN + d] = X[s * D_IN + d];
-    else y[(long long)b * n_out + (d - D_IN)] = Y[s * n_out + (d - D_IN)];
+    __shared__ bf16_t tile[32][34];
+    const int e = blockIdx.y, t = threadIdx.x, nt = n_tiles(n_out);
+    float *P = Pm + e * np, *G = STEP ? Gm + e * np : nullptr;
+    Wf += e * npf;
+    Wb += e * npf;
+    auto step = [&](size_t i) {
+        float p = P[i];
+        if(STEP) {
+            const size_t s = e * np + i;
+            const float g = G[i];
+            const float m = b1 * M[s] + (1.0f - b1) * g;
+            const float v = b2 * V[s] + (1.0f - b2) * g * g;
+            M[s] = m;
+            V[s] = v;
+            p = p - lr * (m / c1) / (sqrtf(v / c2) + eps);
+            P[i] = p;
+        }
+        return p;
+    };
+    if((int)blockIdx.x < nt) {
+        const WTile w = w_tile((int)blockIdx.x, n_out);
+        for(int r = t >> 5; r < 32; r += 8) tile[r][t & 31] = cvt_bf(step(w.W + (size_t)(w.k0 + r) * w.N + w.n0 + (t & 31)));
+        __syncthreads();
+        put_tile(tile, w, Wf, Wb);
+        return;
+    }
+    const int j = ((int)blockIdx.x - nt) * 256 + t;
+    if(STEP && j == 0) next_loss[e] = 0.f;
+    const long long i = loose_param(j, n_out);
+    if(i < 0) return;
+    const float p = step((size_t)i);
+    if(STEP) G[i] = 0.f;
+    if(n_out == 1 && i >= (long long)OFF_WOUT && i < (long long)off_bout(1)) Wf[i] = cvt_bf(p);
 }
 
 } // namespace
@@ -337,17 +496,17 @@ struct bhc_mlp {
     hipStream_t stream;
     int members, max_batch;
     int n_out, front;          // outputs per point; feature front (0 Fourier, 1 inputs + Fourier)
-    long long np;              // parameters per member
+    long long np, npf;         // parameters per member; elements per member of a BF16 copy
     float *P, *Mo, *Vo, *G;    // [members][np]
-    bf16_t *Pbf;
+    bf16_t *Wf, *Wb;           // [members][npf]: weights in operand order, forward and backward
     float *Bf;                 // [N_FREQ][D_IN]
-    float *x, *y, *out, *dout, *loss; // y [max_batch][n_out], out and dout [members][max_batch][n_out]
-    bf16_t *F;                 // [max_batch][D_FF]
-    float *Z[N_HID];           // [members][max_batch][WIDTH]
-    bf16_t *H[N_HID];
-    float *dH, *dH2;           // [members][max_batch][WIDTH]
+    float *x, *y, *out, *loss; // x [max_batch][16], y [max_batch][n_out], out [members][max_batch][n_out], loss [2][16]
+    bf16_t *F;                 // features [max_batch][D_FF], operand order over the rows
+    bf16_t *H[N_HID], *dZ[N_HID]; // [members][max_batch][WIDTH], operand order over the rows
+    bf16_t *dO;                // [members][max_batch][n_out], operand order over the rows
+    float *D[N_HID];           // GELU'(Z) [members][max_batch / 32][16][512]
     float *X, *Y;              // resident training set: X [nset][16], Y [nset][n_out]
-    int32_t *idx;
+    int32_t *idx;              // batches of a chunk of steps
     long long nset;
     long long step;
     hipEvent_t e0, e1;
@@ -356,109 +515,68 @@ struct bhc_mlp {
 
 namespace {
 
-template<typename TA, typename TB, int EPI>
-void gemm(hipStream_t s, int members, const void *A, long long sam, long long sak, long long zA, const void *B,
-          long long sbk, long long sbn, long long zB, float *C, long long ldc, long long zC, int M, int N, int K,
-          const float *bias = nullptr, long long zbias = 0, bf16_t *H = nullptr, int ksplit = 1)
-{
-    GemmArgs g;
-    g.A = A;
-    g.B = B;
-    g.C = C;
-    g.sam = sam;
-    g.sak = sak;
-    g.sbk = sbk;
-    g.sbn = sbn;
-    g.ldc = ldc;
-    g.zA = zA;
-    g.zB = zB;
-    g.zC = zC;
-    g.M = M;
-    g.N = N;
-    g.K = K;
-    g.bias = bias;
-    g.zbias = zbias;
-    g.H = H;
-    g.ksplit = ksplit;
-    dim3 grid((N + TILE - 1) / TILE, (M + TILE - 1) / TILE, members * (EPI == EPI_ATOMIC ? ksplit : 1));
-    hipLaunchKernelGGL((k_gemm<TA, TB, EPI>), grid, dim3(256), 0, s, g);
-}
+constexpr int IDX_CHUNK = 8;   // training steps whose batches are drawn and copied at a time
 
-// forward of a batch already in m->x (n points): fills Z, H and out
-void forward(bhc_mlp *m, int n)
+RowArgs row_args(bhc_mlp *m, const float *X, const float *Y, const int32_t *idx, int n, float *loss)
 {
-    hipStream_t s = m->stream;
-    const int E = m->members;
-    const long long np = m->np;
-    const long long zH = (long long)m->max_batch * WIDTH, zO = (long long)m->max_batch * m->n_out;
-    hipLaunchKernelGGL(k_features, dim3((n * N_FREQ + 255) / 256), dim3(256), 0, s, m->x, n, m->Bf, m->front, m->F);
+    RowArgs g;
+    g.X = X;
+    g.Y = Y;
+    g.idx = idx;
+    g.n = n;
+    g.n_out = m->n_out;
+    g.front = m->front;
+    g.Bf = m->Bf;
+    g.Wf = m->Wf;
+    g.Wb = m->Wb;
+    g.P = m->P;
+    g.np = m->np;
+    g.npf = m->npf;
+    g.out = m->out;
+    g.F = m->F;
     for(int l = 0; l < N_HID; ++l) {
-        const int K = l == 0 ? D_FF : WIDTH;
-        const void *A = l == 0 ? (const void *)m->F : (const void *)m->H[l - 1];
-        const long long zA = l == 0 ? 0 : zH;
-        gemm<bf16_t, bf16_t, EPI_BIAS_GELU>(s, E, A, K, 1, zA, m->Pbf + off_W(l), WIDTH, 1, np, m->Z[l], WIDTH, zH, n,
-                                            WIDTH, K, m->P + off_b(l), np, m->H[l]);
+        g.H[l] = m->H[l];
+        g.dZ[l] = m->dZ[l];
+        g.D[l] = m->D[l];
     }
-    if(m->n_out == 1) {
-        hipLaunchKernelGGL(k_out_fwd, dim3((n + 255) / 256, E), dim3(256), 0, s, m->H[N_HID - 1], m->Pbf, m->P, n, zH,
-                           zO, np, m->out);
-    } else { // out = H5 Wout + bout: M = n, N = n_out, K = WIDTH
-        gemm<bf16_t, bf16_t, EPI_BIAS>(s, E, m->H[N_HID - 1], WIDTH, 1, zH, m->Pbf + OFF_WOUT, m->n_out, 1, np, m->out,
-                                       m->n_out, zO, n, m->n_out, WIDTH, m->P + off_bout(m->n_out), np);
-    }
+    g.dO = m->dO;
+    g.zH = (long long)m->max_batch * WIDTH;
+    g.zO = (long long)m->max_batch * m->n_out;
+    g.members = m->members;
+    g.G = m->G;
+    g.loss = loss;
+    return g;
 }
 
-// backward of the batch after forward(): gradients into m->G, loss into m->loss
-void backward(bhc_mlp *m, int n)
+// forward of n points X [n][16]: out [members][n][n_out]
+void forward(bhc_mlp *m, const float *X, int n)
 {
-    hipStream_t s = m->stream;
-    const int E = m->members, K_out = m->n_out;
-    const long long np = m->np;
-    const long long zH = (long long)m->max_batch * WIDTH, zO = (long long)m->max_batch * K_out;
-    const long long npt = (long long)E * np;
-    const int nchunk = (n + RCHUNK - 1) / RCHUNK;
-    const int ksplit = std::max(1, std::min(64, n / 512));
-    hipLaunchKernelGGL(k_zero, dim3((unsigned)((npt + 255) / 256)), dim3(256), 0, s, m->G, npt);
-    hipLaunchKernelGGL(k_zero, dim3(1), dim3(64), 0, s, m->loss, (long long)E);
-    if(K_out == 1) {
-        hipLaunchKernelGGL(k_out_bwd, dim3(n, E), dim3(256), 0, s, m->out, m->y, n, m->Pbf, m->dH, zH, zO, np, m->dout,
-                           m->loss);
-        hipLaunchKernelGGL(k_out_wgrad, dim3(nchunk, E), dim3(WIDTH + 64), 0, s, m->H[N_HID - 1], m->dout, n, zH, zO,
-                           np, m->G);
-    } else {
-        const int total = n * K_out;
-        hipLaunchKernelGGL(k_out_loss, dim3((total + 255) / 256, E), dim3(256), 0, s, m->out, m->y, total, zO,
-                           m->dout, m->loss);
-        // dWout = H5^T dOut : M = WIDTH, N = n_out, K = n
-        gemm<bf16_t, float, EPI_ATOMIC>(s, E, m->H[N_HID - 1], 1, WIDTH, zH, m->dout, K_out, 1, zO, m->G + OFF_WOUT,
-                                        K_out, np, WIDTH, K_out, n, nullptr, 0, nullptr, ksplit);
-        hipLaunchKernelGGL(k_bias_grad, dim3(nchunk, E), dim3(WIDTH), 0, s, m->dout, n, K_out, zO, np, m->G,
-                           off_bout(K_out));
-        // dH5 = dOut Wout^T : M = n, N = WIDTH, K = n_out
-        gemm<float, bf16_t, EPI_STORE>(s, E, m->dout, K_out, 1, zO, m->Pbf + OFF_WOUT, 1, K_out, np, m->dH, WIDTH, zH,
-                                       n, WIDTH, K_out);
-    }
-    float *dH = m->dH, *dHn = m->dH2;
-    for(int l = N_HID - 1; l >= 0; --l) {
-        const long long tot = (long long)E * zH;
-        hipLaunchKernelGGL(k_gelu_bwd, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, dH, m->Z[l], tot);
-        hipLaunchKernelGGL(k_bias_grad, dim3(nchunk, E), dim3(WIDTH), 0, s, dH, n, WIDTH, zH, np, m->G, off_b(l));
-        const int K_in = l == 0 ? D_FF : WIDTH;
-        // dW = Hprev^T dZ : M = K_in, N = WIDTH, K = n, split over K so that
-        // the 16 (or 4) output tiles per member still fill the GPU
-        const void *Hp = l == 0 ? (const void *)m->F : (const void *)m->H[l - 1];
-        const long long zHp = l == 0 ? 0 : zH;
-        gemm<bf16_t, float, EPI_ATOMIC>(s, E, Hp, 1, K_in, zHp, dH, WIDTH, 1, zH, m->G + off_W(l), WIDTH, np, K_in,
-                                        WIDTH, n, nullptr, 0, nullptr, ksplit);
-        if(l > 0) {
-            // dHprev = dZ W^T : M = n, N = WIDTH (K_in), K = WIDTH
-            gemm<float, bf16_t, EPI_STORE>(s, E, dH, WIDTH, 1, zH, m->Pbf + off_W(l), 1, WIDTH, np, dHn, WIDTH, zH, n,
-                                           K_in, WIDTH);
-            float *t = dH;
-            dH = dHn;
-            dHn = t;
-        }
-    }
+    hipLaunchKernelGGL(k_rows<false>, dim3((n + ROWS - 1) / ROWS, m->members), dim3(512), 0, m->stream,
+                       row_args(m, X, nullptr, nullptr, n, nullptr));
+}
+
+// forward and backward of a batch of n rows (a multiple of 32): gradients in
+// m->G (whose added slots are zero before), loss added to `loss`
+void forward_backward(bhc_mlp *m, const float *X, const float *Y, const int32_t *idx, int n, float *loss)
+{
+    const RowArgs g = row_args(m, X, Y, idx, n, loss);
+    hipLaunchKernelGGL(k_rows<true>, dim3(n / ROWS, m->members), dim3(512), 0, m->stream, g);
+    const int combos = (m->n_out > 1 ? N_HID + 1 : N_HID) * m->members;
+    hipLaunchKernelGGL(k_wgrad, dim3((unsigned)((combos + 7) / 8 * 8 * WG_TILES)), dim3(256), 0, m->stream, g);
+}
+
+void refresh_bf(bhc_mlp *m)
+{
+    hipLaunchKernelGGL(k_adam<false>, dim3(n_tiles(m->n_out) + (n_loose(m->n_out) + 255) / 256, m->members), dim3(256), 0,
+                       m->stream, m->P, nullptr, nullptr, nullptr, m->Wf, m->Wb, m->np, m->npf, m->n_out, 0.f, 0.f, 0.f,
+                       0.f, 0.f, 0.f, nullptr);
+}
+
+void zero_grads(bhc_mlp *m)
+{
+    const long long np = (long long)m->members * m->np;
+    hipLaunchKernelGGL(k_zero, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, m->stream, m->G, np);
+    hipLaunchKernelGGL(k_zero, dim3(1), dim3(64), 0, m->stream, m->loss, 32ll);
 }
 
 } // namespace
@@ -474,14 +592,13 @@ extern "C" void bhc_mlp_destroy(bhc_mlp *m)
     if(!m) return;
     (void)hipSetDevice(m->device);
     (void)hipStreamSynchronize(m->stream);
-    void *ptrs[] = {m->P, m->Mo, m->Vo, m->G, m->Pbf, m->Bf, m->x, m->y, m->out, m->dout, m->loss, m->F, m->dH,
-                    m->dH2, m->X, m->Y, m->idx};
+    void *ptrs[] = {m->P, m->Mo, m->Vo, m->G, m->Wf, m->Wb, m->Bf, m->x, m->y, m->out, m->loss, m->F, m->dO, m->X, m->Y,
+                    m->idx};
     for(void *p : ptrs)
         if(p) (void)hipFree(p);
-    for(int l = 0; l < N_HID; ++l) {
-        if(m->Z[l]) (void)hipFree(m->Z[l]);
-        if(m->H[l]) (void)hipFree(m->H[l]);
-    }
+    for(int l = 0; l < N_HID; ++l)
+        for(void *p : {(void *)m->H[l], (void *)m->D[l]})
+            if(p) (void)hipFree(p);
     (void)hipEventDestroy(m->e0);
     (void)hipEventDestroy(m->e1);
     (void)hipStreamDestroy(m->stream);
@@ -509,22 +626,26 @@ extern "C" int bhc_mlp_create_ex(int device, int members, int max_batch, int n_o
     m->n_out = n_out;
     m->front = front;
     m->np = (long long)n_param(n_out);
+    m->npf = (m->np + 63) / 64 * 64;
     MCHECK(hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking));
     MCHECK(hipEventCreate(&m->e0));
     MCHECK(hipEventCreate(&m->e1));
     size_t np = (size_t)members * m->np;
     size_t act = (size_t)members * max_batch * WIDTH;
     size_t outs = (size_t)max_batch * n_out;
-    bool bad = hipMalloc((void **)&m->P, np * 4) || hipMalloc((void **)&m->Mo, np * 4)
-        || hipMalloc((void **)&m->Vo, np * 4) || hipMalloc((void **)&m->G, np * 4)
-        || hipMalloc((void **)&m->Pbf, np * 2) || hipMalloc((void **)&m->Bf, N_FREQ * D_IN * 4)
-        || hipMalloc((void **)&m->x, (size_t)max_batch * D_IN * 4) || hipMalloc((void **)&m->y, outs * 4)
-        || hipMalloc((void **)&m->out, (size_t)members * outs * 4)
-        || hipMalloc((void **)&m->dout, (size_t)members * outs * 4) || hipMalloc((void **)&m->loss, 16 * 4)
-        || hipMalloc((void **)&m->F, (size_t)max_batch * D_FF * 2) || hipMalloc((void **)&m->dH, act * 4)
-        || hipMalloc((void **)&m->dH2, act * 4) || hipMalloc((void **)&m->idx, (size_t)max_batch * 4);
+    const size_t npf = (size_t)members * m->npf;
+    bool bad = bhc_device_malloc((void **)&m->P, np * 4) || bhc_device_malloc((void **)&m->Mo, np * 4)
+        || bhc_device_malloc((void **)&m->Vo, np * 4) || bhc_device_malloc((void **)&m->G, np * 4)
+        || bhc_device_malloc((void **)&m->Wf, npf * 2) || bhc_device_malloc((void **)&m->Wb, npf * 2)
+        || bhc_device_malloc((void **)&m->Bf, N_FREQ * D_IN * 4)
+        || bhc_device_malloc((void **)&m->x, (size_t)max_batch * D_IN * 4) || bhc_device_malloc((void **)&m->y, outs * 4)
+        || bhc_device_malloc((void **)&m->out, (size_t)members * outs * 4) || bhc_device_malloc((void **)&m->loss, 32 * 4)
+        || bhc_device_malloc((void **)&m->F, (size_t)max_batch * D_FF * 2)
+        || bhc_device_malloc((void **)&m->dO, (size_t)members * outs * 2)
+        || bhc_device_malloc((void **)&m->idx, IDX_CHUNK * (size_t)max_batch * 4);
     for(int l = 0; l < N_HID && !bad; ++l)
-        bad = hipMalloc((void **)&m->Z[l], act * 4) || hipMalloc((void **)&m->H[l], act * 2);
+        bad = bhc_device_malloc((void **)&m->H[l], act * 4) || bhc_device_malloc((void **)&m->D[l], act * 4);
+    for(int l = 0; l < N_HID && !bad; ++l) m->dZ[l] = m->H[l] + act; // second half of H's block
     if(bad) {
         bhc_mlp_destroy(m);
         return mfail("bhc_mlp_create: out of device memory");
@@ -548,8 +669,8 @@ extern "C" int bhc_mlp_create_ex(int device, int members, int max_batch, int n_o
     MCHECK(hipMemcpy(m->Bf, Bf.data(), Bf.size() * 4, hipMemcpyHostToDevice));
     MCHECK(hipMemset(m->Mo, 0, np * 4));
     MCHECK(hipMemset(m->Vo, 0, np * 4));
-    hipLaunchKernelGGL(k_to_bf, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, m->stream, m->P, m->Pbf,
-                       (long long)np);
+    refresh_bf(m);
+    MCHECK(hipGetLastError());
     MCHECK(hipStreamSynchronize(m->stream));
     *out = m;
     return 0;
@@ -585,8 +706,8 @@ extern "C" int bhc_mlp_set_params(bhc_mlp *m, const float *params)
     MCHECK(hipSetDevice(m->device));
     size_t np = (size_t)m->members * m->np;
     MCHECK(hipMemcpy(m->P, params, np * 4, hipMemcpyHostToDevice));
-    hipLaunchKernelGGL(k_to_bf, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, m->stream, m->P, m->Pbf,
-                       (long long)np);
+    refresh_bf(m);
+    MCHECK(hipGetLastError());
     MCHECK(hipStreamSynchronize(m->stream));
     return 0;
 }
@@ -596,16 +717,18 @@ extern "C" int bhc_mlp_predict(bhc_mlp *m, const float *x, long long n, float *o
 {
     MCHECK(hipSetDevice(m->device));
     const int K = m->n_out;
-    const long long zO = (long long)m->max_batch * K;
-    std::vector<float> tmp((size_t)m->members * zO);
     for(long long b0 = 0; b0 < n; b0 += m->max_batch) {
         int nb = (int)std::min<long long>(m->max_batch, n - b0);
         MCHECK(hipMemcpyAsync(m->x, x + b0 * D_IN, (size_t)nb * D_IN * 4, hipMemcpyHostToDevice, m->stream));
-        forward(m, nb);
-        MCHECK(hipMemcpyAsync(tmp.data(), m->out, (size_t)m->members * zO * 4, hipMemcpyDeviceToHost, m->stream));
+        forward(m, m->x, nb);
+        MCHECK(hipGetLastError());
+        // one copy where the members' results are adjacent in the caller's array too
+        const int parts = nb == n ? 1 : m->members;
+        const size_t len = (size_t)(nb == n ? m->members : 1) * nb * K;
+        for(int e = 0; e < parts; ++e)
+            MCHECK(hipMemcpyAsync(out + ((size_t)e * n + b0) * K, m->out + e * len, len * 4, hipMemcpyDeviceToHost,
+                                  m->stream));
         MCHECK(hipStreamSynchronize(m->stream));
-        for(int e = 0; e < m->members; ++e)
-            memcpy(out + ((size_t)e * n + b0) * K, tmp.data() + (size_t)e * zO, (size_t)nb * K * 4);
     }
     return 0;
 }
@@ -619,8 +742,8 @@ extern "C" int bhc_mlp_gradients(bhc_mlp *m, const float *x, const float *y, int
     MCHECK(hipSetDevice(m->device));
     MCHECK(hipMemcpyAsync(m->x, x, (size_t)n * D_IN * 4, hipMemcpyHostToDevice, m->stream));
     MCHECK(hipMemcpyAsync(m->y, y, (size_t)n * m->n_out * 4, hipMemcpyHostToDevice, m->stream));
-    forward(m, n);
-    backward(m, n);
+    zero_grads(m);
+    forward_backward(m, m->x, m->y, nullptr, n, m->loss);
     MCHECK(hipGetLastError());
     if(grads)
         MCHECK(hipMemcpyAsync(grads, m->G, (size_t)m->members * m->np * 4, hipMemcpyDeviceToHost, m->stream));
@@ -636,8 +759,8 @@ extern "C" int bhc_mlp_set_dataset(bhc_mlp *m, const float *X, const float *Y, l
     if(m->X) (void)hipFree(m->X);
     if(m->Y) (void)hipFree(m->Y);
     m->X = m->Y = nullptr;
-    MCHECK(hipMalloc((void **)&m->X, (size_t)n * D_IN * 4));
-    MCHECK(hipMalloc((void **)&m->Y, (size_t)n * m->n_out * 4));
+    MCHECK(bhc_device_malloc((void **)&m->X, (size_t)n * D_IN * 4));
+    MCHECK(bhc_device_malloc((void **)&m->Y, (size_t)n * m->n_out * 4));
     MCHECK(hipMemcpy(m->X, X, (size_t)n * D_IN * 4, hipMemcpyHostToDevice));
     MCHECK(hipMemcpy(m->Y, Y, (size_t)n * m->n_out * 4, hipMemcpyHostToDevice));
     m->nset = n;
@@ -654,32 +777,36 @@ extern "C" int bhc_mlp_train(bhc_mlp *m, int steps, int batch, float lr, unsigne
     MCHECK(hipSetDevice(m->device));
     std::mt19937_64 rng(seed);
     std::uniform_int_distribution<long long> ud(0, m->nset - 1);
-    std::vector<int32_t> idx((size_t)steps * batch);
-    for(auto &v : idx) v = (int32_t)ud(rng);
-    int32_t *d_idx = nullptr;
-    MCHECK(hipMalloc((void **)&d_idx, idx.size() * 4));
-    MCHECK(hipMemcpy(d_idx, idx.data(), idx.size() * 4, hipMemcpyHostToDevice));
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-    const long long np = (long long)m->members * m->np;
     MCHECK(hipEventRecord(m->e0, m->stream));
-    for(int s = 0; s < steps; ++s) {
-        hipLaunchKernelGGL(k_gather, dim3((batch * (D_IN + m->n_out) + 255) / 256), dim3(256), 0, m->stream, m->X,
-                           m->Y, d_idx + (size_t)s * batch, batch, m->n_out, m->x, m->y);
-        forward(m, batch);
-        backward(m, batch);
-        ++m->step;
-        float c1 = 1.0f - std::pow(b1, (float)m->step), c2 = 1.0f - std::pow(b2, (float)m->step);
-        hipLaunchKernelGGL(k_adam, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, m->stream, m->P, m->Mo, m->Vo,
-                           m->G, m->Pbf, np, lr, b1, b2, eps, c1, c2);
+    zero_grads(m);
+    // batches are drawn a chunk of steps at a time, while the GPU works on the
+    // chunk before; the copy follows that chunk's steps on the stream
+    std::vector<int32_t> idx((size_t)steps * batch);
+    for(int s0 = 0; s0 < steps; s0 += IDX_CHUNK) {
+        const int ns = std::min(IDX_CHUNK, steps - s0);
+        int32_t *chunk = idx.data() + (size_t)s0 * batch;
+        for(size_t i = 0; i < (size_t)ns * batch; ++i) chunk[i] = (int32_t)ud(rng);
+        MCHECK(hipMemcpyAsync(m->idx, chunk, (size_t)ns * batch * 4, hipMemcpyHostToDevice, m->stream));
+        for(int s = 0; s < ns; ++s) {
+            float *loss = m->loss + 16 * ((s0 + s) & 1), *next = m->loss + 16 * ((s0 + s + 1) & 1);
+            forward_backward(m, m->X, m->Y, m->idx + (size_t)s * batch, batch, loss);
+            ++m->step;
+            float c1 = 1.0f - std::pow(b1, (float)m->step), c2 = 1.0f - std::pow(b2, (float)m->step);
+            hipLaunchKernelGGL(k_adam<true>, dim3(n_tiles(m->n_out) + (n_loose(m->n_out) + 255) / 256, m->members),
+                               dim3(256), 0, m->stream, m->P, m->Mo, m->Vo, m->G, m->Wf, m->Wb, m->np, m->npf, m->n_out,
+                               lr, b1, b2, eps, c1, c2, next);
+        }
     }
     MCHECK(hipEventRecord(m->e1, m->stream));
     MCHECK(hipGetLastError());
-    if(loss_out) MCHECK(hipMemcpyAsync(loss_out, m->loss, (size_t)m->members * 4, hipMemcpyDeviceToHost, m->stream));
+    if(loss_out)
+        MCHECK(hipMemcpyAsync(loss_out, m->loss + 16 * ((steps - 1) & 1), (size_t)m->members * 4, hipMemcpyDeviceToHost,
+                              m->stream));
     MCHECK(hipStreamSynchronize(m->stream));
     float ms = 0.f;
     MCHECK(hipEventElapsedTime(&ms, m->e0, m->e1));
     m->last_ms = ms;
-    (void)hipFree(d_idx);
     return 0;
 }
 
