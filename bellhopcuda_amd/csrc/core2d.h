@@ -62,6 +62,13 @@ template<typename real> __host__ __device__ inline bool tiny_length(real d, real
     return d < RL(1.0e3) * spacing(x);
 }
 
+// d <= 1000 spacing(x), in the same way.
+template<typename real> __host__ __device__ inline bool small_length(real d, real x)
+{
+    if(d > RL(3.0e3) * RC<real>::EPS * std::fabs(x) + RL(1.0e4) * RC<real>::MINPOS) return false;
+    return d <= RL(1.0e3) * spacing(x);
+}
+
 // ---------------------------------------------------------------------------
 // Complex arithmetic as gcc lowers std::complex / C99 complex (no contraction)
 // ---------------------------------------------------------------------------

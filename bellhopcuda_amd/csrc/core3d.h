@@ -921,6 +921,7 @@ template<typename real> struct Infl3 {
     v3<real> xs;
     v3<real> rn1, rn2;     // ray-centred beams: the previous point's ray normals (c-scaled)
     v2<real> rbr;          // Cartesian: receiver ranges Rr[ir], Rr[ir + 1] (the walk's bracket)
+    real rA;               // Cartesian: range of the ray's current point
     int32_t ir;
 };
 
@@ -1000,6 +1001,7 @@ __host__ __device__ inline bool RayInit3(int ia, int ib, int isx, int isy, int i
     I.phase = FL(0.0);
     I.qOld = mdet(p0.q);
     I.xs = p0.x;
+    I.rA = RL(0.0);
     I.ir = BinarySearchGT(G + P.o_Rr, P.NRr, (real)RL(0.0));
     I.rbr = range_bracket(G + P.o_Rr, P.NRr, I.ir);
     I.rn1 = I.rn2 = V3((real)RL(0.0), (real)RL(0.0), (real)RL(0.0));
@@ -1007,21 +1009,35 @@ __host__ __device__ inline bool RayInit3(int ia, int ib, int isx, int isy, int i
     return true;
 }
 
+// RayUpdate (trace.hpp:274-381, 3D) in its two parts: the step to p1, which
+// reports the boundary it ends on (0 none, 1 top, 2 bottom), and the
+// reflection there.
 template<typename real>
-__host__ __device__ inline bool RayUpdate3(const Ray3<real> &p0, Ray3<real> &p1, Ray3<real> &p2, Trace3<real> &S,
-                                           const Prob3D<real> &P, Err &e, const real *tabs = nullptr)
-{ // trace.hpp:274-381 (3D, rectilinear boundaries)
+__host__ __device__ inline int RayStep3(const Ray3<real> &p0, Ray3<real> &p1, Trace3<real> &S, const Prob3D<real> &P,
+                                        Err &e)
+{
     bool topRefl = false, botRefl = false;
     Step3(p0, p1, S, P, e, topRefl, botRefl);
     GetBdrySeg3(p1.x, p1.t, S.top, P.base + P.o_ati, P.ati_nx, P.ati_ny, true, false, e, prov_of(P, true));
     GetBdrySeg3(p1.x, p1.t, S.bot, P.base + P.o_bty, P.bty_nx, P.bty_ny, false, false, e, prov_of(P, false));
-    if(topRefl || botRefl) {
-        ReflB3<real> r;
-        refl_bdry3(P, topRefl, topRefl ? S.top : S.bot, p1.x, r);
-        Reflect3(p1, p2, r.hs, topRefl, r.n, r.zxx, r.zxy, r.zyy, P, S, e, tabs);
-        return true;
-    }
-    return false;
+    return topRefl ? 1 : (botRefl ? 2 : 0);
+}
+template<typename real>
+__host__ __device__ inline void RayReflect3(const Ray3<real> &p1, Ray3<real> &p2, bool topRefl, Trace3<real> &S,
+                                            const Prob3D<real> &P, Err &e, const real *tabs = nullptr)
+{
+    ReflB3<real> r;
+    if(topRefl) refl_bdry3(P, true, S.top, p1.x, r);
+    else refl_bdry3(P, false, S.bot, p1.x, r);
+    Reflect3(p1, p2, r.hs, topRefl, r.n, r.zxx, r.zxy, r.zyy, P, S, e, tabs);
+}
+template<typename real>
+__host__ __device__ inline bool RayUpdate3(const Ray3<real> &p0, Ray3<real> &p1, Ray3<real> &p2, Trace3<real> &S,
+                                           const Prob3D<real> &P, Err &e, const real *tabs = nullptr)
+{
+    const int refl = RayStep3(p0, p1, S, P, e);
+    if(refl) RayReflect3(p1, p2, refl == 1, S, P, e, tabs);
+    return refl != 0;
 }
 
 // Returns true when the ray ends; nsteps is set as the reference sets Nsteps
@@ -1110,23 +1126,31 @@ template<typename real> struct Seg3D {
     int32_t job, is, ntop, nbot; // ray (job) number, step index, end point's bounce counts (arrivals, eigen hits)
 };
 
+// The update in two parts, as in 2D: seg3_begin applies the update of the
+// ray's influence state and tells whether the segment is handed to the
+// scatter, seg3_fill forms its descriptor.
+template<typename real> struct SegGeo3 {
+    v3<real> t;                 // step vector
+    real rlen, lo, hi;
+    int32_t first, ir;
+};
 template<typename real>
-__host__ __device__ inline void prelude3(Seg3D<real> &d, const Ray3<real> &p0, const Ray3<real> &p1, Infl3<real> &I,
-                                         int is, const Prob3D<real> &P, int isz, int isx, int isy)
+__host__ __device__ inline bool seg3_begin(SegGeo3<real> &g, const Ray3<real> &p0, const Ray3<real> &p1,
+                                           Infl3<real> &I, int is, const Prob3D<real> &P)
 {
-    d.nitems = 0;
     const real *Rr = P.base + P.o_Rr;
-    real dax = p0.x.x - I.xs.x, day = p0.x.y - I.xs.y, dbx = p1.x.x - I.xs.x, dby = p1.x.y - I.xs.y;
-    real rA = std::sqrt(dax * dax + day * day);
-    real rB = std::sqrt(dbx * dbx + dby * dby);
-    if(std::fabs(rA - rB) <= RL(1.0e3) * spacing(rA)) return; // IsDuplicatePoint
+    const real dbx = p1.x.x - I.xs.x, dby = p1.x.y - I.xs.y;
+    const real rA = I.rA;       // the range of p0, which ended the step before
+    const real rB = std::sqrt(dbx * dbx + dby * dby);
+    I.rA = rB;
+    if(small_length(std::fabs(rA - rB), rA)) return false; // IsDuplicatePoint
     if(is == 0) {
         I.ir = (rB > rA) ? 0 : P.NRr - 1;
         I.rbr = range_bracket(Rr, P.NRr, I.ir);
     }
-    v3<real> rayt = p1.x - p0.x;
-    real rlen = len3(rayt);
-    if(rlen <= RL(1.0e3) * spacing(p1.x.x)) return;
+    g.t = p1.x - p0.x;
+    g.rlen = len3(g.t);
+    if(small_length(g.rlen, p1.x.x)) return false;
     real phaseq = mdet(p0.q);
     if((phaseq <= RL(0.0) && I.qOld > RL(0.0)) || (phaseq >= RL(0.0) && I.qOld < RL(0.0)))
         I.phase += RC<real>::PI / FL(2.0);
@@ -1134,7 +1158,8 @@ __host__ __device__ inline void prelude3(Seg3D<real> &d, const Ray3<real> &p0, c
     // receiver walk: the visited ranges are contiguous; the bracket
     // (Rr[ir], Rr[ir + 1]) travels with the ray, so a step that crosses no
     // receiver range reads none (the comparisons are the walk's)
-    int ir = I.ir, first = I.ir;
+    int ir = I.ir;
+    g.first = ir;
     real rlo = I.rbr.x, rhi = I.rbr.y;
     const real rfirst = rlo;    // Rr[first]
     for(;;) {
@@ -1157,13 +1182,25 @@ __host__ __device__ inline void prelude3(Seg3D<real> &d, const Ray3<real> &p0, c
     }
     I.ir = ir;
     I.rbr = V(rlo, rhi);
-    d.lo = rmin(rA, rB);
-    d.hi = rmax(rA, rB);
+    g.ir = ir;
+    g.lo = rmin(rA, rB);
+    g.hi = rmax(rA, rB);
     // a step that crosses no receiver range has the one range Rr[first]:
     // outside [lo, hi) the scatter's row test accepts none of its receivers
-    if(ir == first && !(rfirst >= d.lo && rfirst < d.hi)) return;
+    return !(ir == g.first && !(rfirst >= g.lo && rfirst < g.hi));
+}
+
+template<typename real>
+__host__ __device__ inline void seg3_fill(Seg3D<real> &d, const SegGeo3<real> &g, const Ray3<real> &p0,
+                                          const Ray3<real> &p1, const Infl3<real> &I, int is, const Prob3D<real> &P,
+                                          int isz, int isx, int isy)
+{
+    d.lo = g.lo;
+    d.hi = g.hi;
+    const int first = g.first, ir = g.ir;
+    const real rlen = g.rlen;
     // the beam's frame and reach: only for steps handed to the scatter
-    rayt = dv3(rayt, rlen);
+    const v3<real> rayt = dv3(g.t, rlen);
     v3<real> e1, e2;
     RayNormal3(rayt, p1.phi, true, (real)RL(1.0), e1, e2);
     real a0 = p0.q.a00 * I.rcp_q0, b0 = p0.q.a10 * I.rcp_q0, a1 = p1.q.a00 * I.rcp_q0, b1 = p1.q.a10 * I.rcp_q0;
@@ -1208,6 +1245,15 @@ __host__ __device__ inline void prelude3(Seg3D<real> &d, const Ray3<real> &p0, c
     d.ntop = p1.NumTopBnc;
     d.nbot = p1.NumBotBnc;
     d.nitems = ((ir >= first ? ir - first : first - ir) + 1) * P.Ntheta;
+}
+
+template<typename real>
+__host__ __device__ inline void prelude3(Seg3D<real> &d, const Ray3<real> &p0, const Ray3<real> &p1, Infl3<real> &I,
+                                         int is, const Prob3D<real> &P, int isz, int isx, int isy)
+{
+    SegGeo3<real> g;
+    d.nitems = 0;
+    if(seg3_begin(g, p0, p1, I, is, P)) seg3_fill(d, g, p0, p1, I, is, P, isz, isx, isy);
 }
 
 // One (range, bearing) row of a segment: the row tests of the reference and

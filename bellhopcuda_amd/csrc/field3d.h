@@ -111,13 +111,12 @@ template<typename real, bool RCEN = false> __device__ inline void seal3(const Se
     }
 }
 
-template<typename real, typename Desc, bool RCEN = false>
-__device__ inline void append3(const Desc &d, int lane, const DevOut3 &O, SegBlock &B)
+// A slot of the segment buffer for this lane (if has), called by all lanes.
+template<typename real, bool RCEN> __device__ inline uint32_t reserve3(bool has, int lane, const DevOut3 &O, SegBlock &B)
 {
-    bool has = d.nitems > 0;
-    unsigned long long m = __ballot(has);
-    if(!m) return;
-    uint32_t cnt = (uint32_t)__popcll(m);
+    const unsigned long long m = __ballot(has);
+    if(!m) return 0xFFFFFFFFu;
+    const uint32_t cnt = (uint32_t)__popcll(m);
     if(B.used + cnt > B.cap) {
         seal3<real, RCEN>(B, lane, O);
         uint32_t base = 0;
@@ -126,17 +125,32 @@ __device__ inline void append3(const Desc &d, int lane, const DevOut3 &O, SegBlo
         B.used = 0;
         B.cap = SEG_BLOCK;
     }
-    if(has) {
-        uint32_t slot = B.base + B.used + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
-        if(slot < O.seg_cap) reinterpret_cast<SegSlot3<real, RCEN> *>(O.segs)[slot].d = d;
-        else atomicOr(O.overflow, 1u);
-    }
+    const uint32_t slot = B.base + B.used + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
     B.used += cnt;
+    return slot;
+}
+
+template<typename real, bool RCEN, typename Desc> __device__ inline void store3(const Desc &d, uint32_t slot, const DevOut3 &O)
+{
+    if(slot < O.seg_cap) reinterpret_cast<SegSlot3<real, RCEN> *>(O.segs)[slot].d = d;
+    else atomicOr(O.overflow, 1u);
 }
 
 // Trace kernel: the ray loop of MainFieldModes (src/trace.hpp:525-589), 3D.
 // Reflection tables staged in LDS up to this many reals (top and bottom together).
 constexpr int REFL_LDS = 768;
+// A wavefront's reflections are made when 1 / REFLECT_SHARE of its rays wait.
+constexpr int REFLECT_SHARE = 16;
+
+// Whether the wavefront's pending reflections are made now: once a sixteenth of
+// its rays wait for one, or none can step. The whole wavefront walks through a
+// reflection for however few of its rays, and in 3D that (curvature matrices,
+// ray normals, halfspace coefficient) is most of a step's work.
+__device__ inline bool reflect_now(bool active, bool pending)
+{
+    const int np = __popcll(__ballot(pending)), na = __popcll(__ballot(active));
+    return np > 0 && REFLECT_SHARE * np >= na;
+}
 
 template<typename real, bool RCEN = false> __global__ void __launch_bounds__(64) k_trace3d(Prob3D<real> P, DevOut3 O)
 {
@@ -148,7 +162,7 @@ template<typename real, bool RCEN = false> __global__ void __launch_bounds__(64)
     Ray3<real> p0;
     Trace3<real> S;
     Infl3<real> I;
-    int job = 0, ia = 0, ib = 0, isx = 0, isy = 0, isz = 0, is = 0;
+    int job = 0, ia = 0, ib = 0, isx = 0, isy = 0, isz = 0, is = 0, pend = 0;
     bool active = false, exhausted = false, init_fail = false;
     unsigned long long steps = 0;
     SegBlock blk{0u, 0u, 0u};
@@ -196,31 +210,60 @@ template<typename real, bool RCEN = false> __global__ void __launch_bounds__(64)
                 continue;
             }
         }
-        Ray3<real> p1, p2;
-        std::conditional_t<RCEN, Seg3R<real>, Seg3D<real>> d;
-        d.nitems = 0;
-        bool two = false;
-        if(active) {
-            two = RayUpdate3(p0, p1, p2, S, P, e, tabs);
-            if constexpr(RCEN) prelude3rc(d, p0, p1, I, is, P, isz, isx, isy);
-            else prelude3(d, p0, p1, I, is, P, isz, isx, isy);
-            d.job = job;
-            ++is;
-        }
-        append3<real, decltype(d), RCEN>(d, lane, O, blk);
-        if(__any(two)) {
-            d.nitems = 0;
-            if(active && two) {
-                if constexpr(RCEN) prelude3rc(d, p1, p2, I, is, P, isz, isx, isy);
-                else prelude3(d, p1, p2, I, is, P, isz, isx, isy);
-                d.job = job;
-                ++is;
+        // the step, its segment, and the reflections once enough of the
+        // wavefront's rays wait for one (reflect_now), as in the 2D trace; the
+        // reflected point's segment has no length: only ray-centred beams
+        // update their influence state there
+        Ray3<real> p1;
+        bool go = active && !pend;
+        int refl = 0;
+        if(go) refl = RayStep3(p0, p1, S, P, e);
+#pragma unroll 1
+        for(;;) {
+            if constexpr(RCEN) {
+                Seg3R<real> d;
+                d.nitems = 0;
+                if(go) {
+                    prelude3rc(d, p0, p1, I, is, P, isz, isx, isy);
+                    d.job = job;
+                }
+                const bool has = d.nitems > 0;
+                const uint32_t slot = reserve3<real, RCEN>(has, lane, O, blk);
+                if(has) store3<real, RCEN>(d, slot, O);
+            } else {
+                SegGeo3<real> g;
+                const bool has = go && seg3_begin(g, p0, p1, I, is, P);
+                const uint32_t slot = reserve3<real, RCEN>(has, lane, O, blk);
+                if(has) {
+                    Seg3D<real> d;
+                    seg3_fill(d, g, p0, p1, I, is, P, isz, isx, isy);
+                    d.job = job;
+                    store3<real, RCEN>(d, slot, O);
+                }
             }
-            append3<real, decltype(d), RCEN>(d, lane, O, blk);
+            if(go) {
+                ++is;
+                p0 = p1;
+                go = false;
+            }
+            if(refl) {
+                pend = refl;
+                refl = 0;
+            }
+            if(!reflect_now(active, pend != 0)) break;
+            if(pend) {
+                RayReflect3(p0, p1, pend == 1, S, P, e, tabs);
+                pend = 0;
+                go = RCEN;
+                if(!go) {
+                    ++is;
+                    p0 = p1;
+                }
+            }
+            if(!__any(go)) break;
         }
         bool fin = false;
-        if(active) {
-            p0 = two ? p2 : p1;
+        if(active && !pend) {
             if(RayTerminate3(p0, is, S, P, e)) {
                 active = false;
                 fin = true;

@@ -330,24 +330,38 @@ __host__ __device__ inline bool RayInitNx(int ia, int ib, int isx, int isy, int 
     return true;
 }
 
-// RayUpdate (trace.hpp:274-381, O3D && !R3D).
+// RayUpdate (trace.hpp:274-381, O3D && !R3D) in its two parts: the step to p1,
+// which reports the boundary it ends on (0 none, 1 top, 2 bottom), and the
+// reflection there.
 template<typename real>
-__host__ __device__ inline bool RayUpdateNx(const RayPt<real> &p0, RayPt<real> &p1, RayPt<real> &p2, Trace3<real> &S,
-                                            const OrgNx<real> &org, const Prob3D<real> &N, const Prob2D<real> &P,
-                                            Err &e, const real *tabs = nullptr)
+__host__ __device__ inline int RayStepNx(const RayPt<real> &p0, RayPt<real> &p1, Trace3<real> &S,
+                                         const OrgNx<real> &org, const Prob3D<real> &N, Err &e)
 {
     bool topRefl = false, botRefl = false;
     StepNx(p0, p1, S, org, N, e, topRefl, botRefl);
     const v3<real> x_o = RayToOceanX(p1.x, org), t_o = RayToOceanT(p1.t, org);
     GetBdrySeg3(x_o, t_o, S.top, N.base + N.o_ati, N.ati_nx, N.ati_ny, true, false, e, prov_of(N, true));
     GetBdrySeg3(x_o, t_o, S.bot, N.base + N.o_bty, N.bty_nx, N.bty_ny, false, false, e, prov_of(N, false));
-    if(topRefl || botRefl) {
-        ReflB3<real> r;
-        refl_bdry3(N, topRefl, topRefl ? S.top : S.bot, x_o, r);
-        ReflectNx(p1, p2, r.hs, topRefl, r.n, r.kxx, r.kxy, r.kyy, org, N, P, S, e, tabs);
-        return true;
-    }
-    return false;
+    return topRefl ? 1 : (botRefl ? 2 : 0);
+}
+template<typename real>
+__host__ __device__ inline void RayReflectNx(const RayPt<real> &p1, RayPt<real> &p2, bool topRefl, Trace3<real> &S,
+                                             const OrgNx<real> &org, const Prob3D<real> &N, const Prob2D<real> &P,
+                                             Err &e, const real *tabs = nullptr)
+{
+    ReflB3<real> r;
+    if(topRefl) refl_bdry3(N, true, S.top, RayToOceanX(p1.x, org), r);
+    else refl_bdry3(N, false, S.bot, RayToOceanX(p1.x, org), r);
+    ReflectNx(p1, p2, r.hs, topRefl, r.n, r.kxx, r.kxy, r.kyy, org, N, P, S, e, tabs);
+}
+template<typename real>
+__host__ __device__ inline bool RayUpdateNx(const RayPt<real> &p0, RayPt<real> &p1, RayPt<real> &p2, Trace3<real> &S,
+                                            const OrgNx<real> &org, const Prob3D<real> &N, const Prob2D<real> &P,
+                                            Err &e, const real *tabs = nullptr)
+{
+    const int refl = RayStepNx(p0, p1, S, org, N, e);
+    if(refl) RayReflectNx(p1, p2, refl == 1, S, org, N, P, e, tabs);
+    return refl != 0;
 }
 
 // RayTerminate (trace.hpp:391-477, O3D && !R3D): the 3D tests on the ocean

@@ -140,7 +140,7 @@ struct DevOut {
     const int32_t *job_sz;
     const int32_t *nsteps_in;   // eigen re-trace limits (or null)
     int32_t *nsteps_out;
-    unsigned long long *counters; // [0] steps, [1] contributions
+    unsigned long long *counters; // [0] steps, [1] contributions, [2] candidate receivers (single problems)
     uint32_t *errw;             // err, warn, nerr, nwarn
     int32_t *work;              // ray work counter (relative to job_begin)
     int32_t job_begin, job_end; // ray range of this trace pass
@@ -357,14 +357,6 @@ __device__ inline void store_seg(const SegDesc<real> &d, uint32_t slot, const De
     }
 }
 
-template<typename real>
-__device__ inline void append_seg(const SegDesc<real> &d, int lane, const DevOut &O, SegBlock &B, bool full)
-{
-    const bool has = d.nitems > 0;
-    const uint32_t slot = reserve_seg<real>(has, lane, O, B);
-    if(has) store_seg(d, slot, O, full);
-}
-
 // Exclusive prefix sum of cnt over the wavefront; returns the total.
 __device__ inline int wave_excl_scan(int cnt, int lane, int &excl)
 {
@@ -389,6 +381,7 @@ __device__ inline int wave_owner(int excl, int t)
     return own;
 }
 
+constexpr int RAYCEN_DIRECT = 6;
 // Scatter one segment's receivers with the 64 lanes of a wavefront (d is
 // wavefront-uniform). Both geometries have rows of different lengths --
 // Cartesian range columns with their depth bands, ray-centred depths with
@@ -422,6 +415,11 @@ __device__ inline void scatter_seg(const SegDesc<real> &d, const Prob2D<real> &P
         int blo = 0, bhi = -1;
         if(g + lane < d.nz && !raycen_range(d, iz, P, Rr, P.Rz, nA, rA, nB, rB, blo, bhi)) bhi = blo - 1;
         const int cnt = bhi - blo + 1;
+        if(!__any(cnt > RAYCEN_DIRECT)) {
+            for(int k = 0; __any(k < cnt); ++k)
+                if(k < cnt) raycen_one<real, RT, Sink, FAST>(d, blo + k, iz, nA, rA, nB, rB, P, Rr, sink);
+            continue;
+        }
         int excl;
         const int total = wave_excl_scan(cnt, lane, excl);
         for(int t0 = 0; t0 < total; t0 += WAVE) {
@@ -436,22 +434,24 @@ __device__ inline void scatter_seg(const SegDesc<real> &d, const Prob2D<real> &P
 
 // One step of the wavefront's rays (RayUpdate and both influence updates of
 // the ray loop, src/trace.hpp:525-589): p0 moves to the step's end, or past the
-// reflection there. reserve(has) is called by all lanes and gives the lanes
-// with a segment its slot; out(d, slot) takes the descriptor. The reflected
-// point's segment has no length on Cartesian beams unless the beam is shifted:
-// its influence update then changes nothing and is left out. Both segments run
-// through one copy of the code, the descriptor is formed where it is stored,
-// and the reflection is made after that, so that descriptor, reflection and
-// the points between are not held in registers side by side.
-template<typename real, char ST, bool WINDOW, typename Reserve, typename Out>
-__device__ inline void step_ray(bool active, RayPt<real> &p0, Trace<real> &S, Infl<real> &I, int &is,
-                                const Prob2D<real> &P, const real *B, const real *G, int isz, int ia, Err &e,
+// reflection there. step(p0, p1) (which tells the boundary it ends on: 1 top, 2
+// bottom) and reflect(p0, p1, top) are the ray's own; reserve(has) is called by
+// all lanes and gives the lanes with a segment its slot; out(d, slot) takes the
+// descriptor. The reflected point's segment has no length on Cartesian beams
+// unless the beam is shifted: its influence update then changes nothing and is
+// left out. Both segments run through one copy of the code, the descriptor is
+// formed where it is stored, and the reflection is made after that, so that
+// descriptor, reflection and the points between are not held in registers side
+// by side.
+template<typename real, bool WINDOW, typename StepF, typename ReflF, typename Reserve, typename Out>
+__device__ inline void step_ray(bool active, RayPt<real> &p0, Infl<real> &I, int &is, const Prob2D<real> &P,
+                                const real *RzT, const real *G, int isz, int ia, StepF step, ReflF reflect,
                                 Reserve reserve, Out out)
 {
     RayPt<real> p1;
-    int refl = 0;
     bool go = active;
-    if(active) refl = RayStep<real, ST>(p0, p1, S, P, B, e);
+    int refl = 0;
+    if(go) refl = step(p0, p1);
 #pragma unroll 1
     for(;;) {
         SegGeo<real> g;
@@ -462,17 +462,17 @@ __device__ inline void step_ray(bool active, RayPt<real> &p0, Trace<real> &S, In
             SegDesc<real> d;
             d.lo = lo;
             d.hi = hi;
-            seg_fill<real, WINDOW>(d, g, p0, p1, I, is, P, B + P.o_rzs, isz, ia);
+            seg_fill<real, WINDOW>(d, g, p0, p1, I, is, P, RzT, isz, ia);
             out(d, slot);
         }
         if(go) {
             seg_end(g, p1, I, P);
             ++is;
             p0 = p1;
+            go = false;
         }
-        go = false;
         if(refl) {
-            RayReflect<real, ST>(p0, p1, refl == 1, S, P, B, G, e);
+            reflect(p0, p1, refl == 1);
             refl = 0;
             go = P.isRayCen || p1.x.x != p0.x.x || p1.x.y != p0.x.y;
             if(!go) {
@@ -482,6 +482,15 @@ __device__ inline void step_ray(bool active, RayPt<real> &p0, Trace<real> &S, In
         }
         if(!__any(go)) break;
     }
+}
+
+// Receivers that a segment's descriptor brackets, about (ray-centred: its
+// depths by the ranges it spans).
+template<typename real> __device__ inline unsigned candidates(const SegDesc<real> &d, const Prob2D<real> &P)
+{
+    if(!P.isRayCen) return (unsigned)d.nitems;
+    const float span = fabsf((float)(d.xb.x - d.xa.x)) / (float)P.Delta_r;
+    return (unsigned)((float)d.nitems * (1.0f + fminf(span, (float)P.NRr)));
 }
 
 // Trace kernel of the field modes (TL / arrivals / eigen): the ray loop of
@@ -515,7 +524,7 @@ __global__ void __launch_bounds__(WAVE) k_trace2d(Prob2D<real> P, DevOut O)
     Infl<real> I;
     int job = 0, isz = 0, ia = 0, is = 0;
     bool active = false, exhausted = false;
-    unsigned long long steps = 0;
+    unsigned long long steps = 0, cand = 0;
     SegBlock blk{0u, 0u, 0u};
     for(int iter = 0;; ++iter) {
         if(!exhausted) {
@@ -564,9 +573,15 @@ __global__ void __launch_bounds__(WAVE) k_trace2d(Prob2D<real> P, DevOut O)
                 continue;
             }
         }
-        step_ray<real, ST, true>(active, p0, S, I, is, P, B, G, isz, ia, e,
-                                 [&](bool has) { return reserve_seg<real>(has, lane, O, blk); },
-                                 [&](const SegDesc<real> &d, uint32_t slot) { store_seg(d, slot, O, full); });
+        step_ray<real, true>(
+            active, p0, I, is, P, B + P.o_rzs, G, isz, ia,
+            [&](const RayPt<real> &a, RayPt<real> &b) { return RayStep<real, ST>(a, b, S, P, B, e); },
+            [&](const RayPt<real> &a, RayPt<real> &b, bool top) { RayReflect<real, ST>(a, b, top, S, P, B, G, e); },
+            [&](bool has) { return reserve_seg<real>(has, lane, O, blk); },
+            [&](const SegDesc<real> &d, uint32_t slot) {
+                cand += candidates(d, P);
+                store_seg(d, slot, O, full);
+            });
         bool fin = false;
         if(active) {
             int t = RayTerminate(p0, is, S, MAXN, P, e);
@@ -587,8 +602,14 @@ __global__ void __launch_bounds__(WAVE) k_trace2d(Prob2D<real> P, DevOut O)
     }
     seal_block<real>(blk, lane, O);
     flush_err(e, O);
-    for(int off = WAVE / 2; off > 0; off >>= 1) steps += __shfl_xor(steps, off);
-    if(lane == 0) atomicAdd(O.counters + 0, steps);
+    for(int off = WAVE / 2; off > 0; off >>= 1) {
+        steps += __shfl_xor(steps, off);
+        cand += __shfl_xor(cand, off);
+    }
+    if(lane == 0) {
+        atomicAdd(O.counters + 0, steps);
+        atomicAdd(O.counters + 2, cand);
+    }
 }
 
 // Scatter kernel: one wavefront per segment; the descriptor is wavefront-
@@ -649,9 +670,12 @@ __global__ void __launch_bounds__(256) k_scatter2d_lanes(Prob2D<real> P, DevOut 
 enum : int { SCATTER_AUTO = 0, SCATTER_TILED = 1, SCATTER_WAVE = 2, SCATTER_LANES = 3 };
 
 struct BinCfg {
-    int32_t nbins, bin_w, tile_w, tile_lo_off; // tile columns = [b*bin_w - tile_lo_off, + tile_w)
-    int32_t chunk;                              // segments per workgroup
-    int32_t *counts, *offsets, *cursor, *chunk_start;
+    int32_t nbins;              // range bins of one source; source isz's bins are isz nbins ..
+    int32_t total;              // bins of all sources
+    int32_t bin_w, tile_w, tile_lo_off; // tile columns of range bin b = [b*bin_w - tile_lo_off, + tile_w)
+    int32_t chunk;              // segments per workgroup
+    int32_t *counts, *offsets, *cursor;
+    int32_t *chunk_bin, *chunk_pos; // per chunk: its bin and its first position in idx
     uint32_t *idx;
     int32_t *nchunks;
 };
@@ -668,7 +692,7 @@ template<typename real> __device__ inline int seg_bin(const SegDesc<real> &d, co
         col = (d.ir0 + d.ir1) / 2;
     }
     col = imax(0, imin(col, P.NRr - 1));
-    return imin(col / C.bin_w, C.nbins - 1);
+    return d.isz * C.nbins + imin(col / C.bin_w, C.nbins - 1);
 }
 
 // The bin of stored segment s (its rest read for ray-centred segments only).
@@ -690,51 +714,56 @@ template<typename real> __global__ void __launch_bounds__(256) k_bin_count(Prob2
     if(n > O.seg_cap) n = O.seg_cap;
     uint32_t per = (n + gridDim.x - 1) / gridDim.x;
     uint32_t s0 = blockIdx.x * per, s1 = min(n, s0 + per);
-    for(int b = threadIdx.x; b < C.nbins; b += blockDim.x) h[b] = 0;
+    for(int b = threadIdx.x; b < C.total; b += blockDim.x) h[b] = 0;
     __syncthreads();
     for(uint32_t s = s0 + threadIdx.x; s < s1; s += blockDim.x)
         if(seg_nitems<real>(O, s) > 0) atomicAdd(h + seg_bin_at(O, s, P, C), 1);
     __syncthreads();
-    for(int b = threadIdx.x; b < C.nbins; b += blockDim.x)
+    for(int b = threadIdx.x; b < C.total; b += blockDim.x)
         if(h[b]) atomicAdd(C.counts + b, h[b]);
 }
 
 // Exclusive scan of the bin counts and of the per-bin chunk counts (one workgroup).
 __global__ void __launch_bounds__(1024) k_bin_scan(BinCfg C)
 {
-    __shared__ int32_t part_s[1024], part_c[1024];
-    int t = threadIdx.x, nb = C.nbins;
-    int per = (nb + 1023) / 1024;
-    int b0 = t * per, b1 = min(nb, b0 + per);
+    __shared__ int32_t wave_s[16], wave_c[16];
+    const int t = threadIdx.x, lane = t & (WAVE - 1), w = t / WAVE, nb = C.total;
+    const int per = (nb + 1023) / 1024;
+    const int b0 = min(nb, t * per), b1 = min(nb, b0 + per);
     int ss = 0, sc = 0;
     for(int b = b0; b < b1; ++b) {
         ss += C.counts[b];
         sc += (C.counts[b] + C.chunk - 1) / C.chunk;
     }
-    part_s[t] = ss;
-    part_c[t] = sc;
-    __syncthreads();
-    if(t == 0) {
-        int a = 0, c = 0;
-        for(int i = 0; i < 1024; ++i) {
-            int x = part_s[i], y = part_c[i];
-            part_s[i] = a;
-            part_c[i] = c;
-            a += x;
-            c += y;
+    int is = ss, ic = sc; // inclusive over the wavefront
+    for(int o = 1; o < WAVE; o <<= 1) {
+        const int a = __shfl_up(is, o), c = __shfl_up(ic, o);
+        if(lane >= o) {
+            is += a;
+            ic += c;
         }
-        *C.nchunks = c;
+    }
+    if(lane == WAVE - 1) {
+        wave_s[w] = is;
+        wave_c[w] = ic;
     }
     __syncthreads();
-    ss = part_s[t];
-    sc = part_c[t];
+    int ps = is - ss, pc = ic - sc;
+    for(int k = 0; k < w; ++k) {
+        ps += wave_s[k];
+        pc += wave_c[k];
+    }
+    if(t == 1023) *C.nchunks = pc + sc;
     for(int b = b0; b < b1; ++b) {
-        C.offsets[b] = ss;
-        C.cursor[b] = ss;
-        int nc = (C.counts[b] + C.chunk - 1) / C.chunk;
-        for(int k = 0; k < nc; ++k) C.chunk_start[sc + k] = b; // chunk -> bin
-        ss += C.counts[b];
-        sc += nc;
+        C.offsets[b] = ps;
+        C.cursor[b] = ps;
+        const int nc = (C.counts[b] + C.chunk - 1) / C.chunk;
+        for(int k = 0; k < nc; ++k) {
+            C.chunk_bin[pc + k] = b;
+            C.chunk_pos[pc + k] = ps + k * C.chunk;
+        }
+        ps += C.counts[b];
+        pc += nc;
     }
 }
 
@@ -748,12 +777,12 @@ template<typename real> __global__ void __launch_bounds__(256) k_bin_fill(Prob2D
     if(n > O.seg_cap) n = O.seg_cap;
     uint32_t per = (n + gridDim.x - 1) / gridDim.x;
     uint32_t s0 = blockIdx.x * per, s1 = min(n, s0 + per);
-    for(int b = threadIdx.x; b < C.nbins; b += blockDim.x) h[b] = 0;
+    for(int b = threadIdx.x; b < C.total; b += blockDim.x) h[b] = 0;
     __syncthreads();
     for(uint32_t s = s0 + threadIdx.x; s < s1; s += blockDim.x)
         if(seg_nitems<real>(O, s) > 0) atomicAdd(h + seg_bin_at(O, s, P, C), 1);
     __syncthreads();
-    for(int b = threadIdx.x; b < C.nbins; b += blockDim.x)
+    for(int b = threadIdx.x; b < C.total; b += blockDim.x)
         if(h[b]) h[b] = atomicAdd(C.cursor + b, h[b]);
     __syncthreads();
     for(uint32_t s = s0 + threadIdx.x; s < s1; s += blockDim.x) {
@@ -764,15 +793,15 @@ template<typename real> __global__ void __launch_bounds__(256) k_bin_fill(Prob2D
 }
 
 template<typename real> struct TileSink {
-    float *tile;          // LDS [tile_w][nz] complex
-    int col0, tile_w, nz, nrr;
+    float *tile;          // LDS [tile_w][nz] complex, of source isz0
+    int col0, tile_w, nz, nrr, isz0;
     unsigned long long nc;
     // (the cell, not its index: an index would have to be divided back into
     // range and depth, several hundred instructions of 64-bit division)
     __device__ void add_cell(const Prob2D<real> &Pp, int isz, int iz, int ir, float re, float im)
     {
         const int c = ir - col0;
-        if(c >= 0 && c < tile_w && isz == 0) {
+        if(c >= 0 && c < tile_w && isz == isz0) {
             int k = c * nz + iz; // real parts first, then imaginary parts (bank-conflict free)
             atomicAdd(tile + k, re);
             atomicAdd(tile + tile_w * nz + k, im);
@@ -788,48 +817,67 @@ template<typename real> struct TileSink {
     __device__ void mark() {}
 };
 
-// One workgroup per (bin, chunk); the field of source isz lives at
-// P.field + isz * plane, so the tile is per source: segments of other
-// sources fall back to global atomics (single-source runs are the common case).
+// One workgroup per chunk of a (source, range) bin, one wavefront per segment
+// at a time. Latency bounds it (on the 20001-ray seamount field the SIMDs
+// issue vector instructions in 45 % of their cycles), so the wavefront's next
+// descriptor is on its way while it works on the current one: 64 segment
+// numbers are read at a time, lane k loads word k of the next descriptor (one
+// load instruction for all its words), and the words reach every lane through
+// LDS.
 constexpr int TILE_THREADS = 512;
+constexpr int TILE_STAGE = (TILE_THREADS / WAVE) * SEG_NW<double> * 16; // bytes beside the tile
 
 template<typename real, bool FAST>
 __global__ void __launch_bounds__(TILE_THREADS, 4) k_scatter_tile(Prob2D<real> P, DevOut O, BinCfg C)
 {
     extern __shared__ __align__(16) unsigned char lds_raw[];
+    __shared__ uint4 stage_all[TILE_THREADS / WAVE][SEG_NW<real>];
     float *tile = reinterpret_cast<float *>(lds_raw);
-    int nchunks = *C.nchunks;
+    const int nchunks = *C.nchunks;
     const int lane = threadIdx.x & (WAVE - 1);
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));
     const int nw = blockDim.x / WAVE;
     const int nz = P.NRz_per_range;
+    const int words = seg_full(P) ? SEG_NW<real> : SEG_NC<real>;
+    uint4 *stage = stage_all[wave];
     unsigned long long total = 0;
     for(int ch = blockIdx.x; ch < nchunks; ch += gridDim.x) {
-        int b = C.chunk_start[ch];
-        int first_chunk = ch;
-        while(first_chunk > 0 && C.chunk_start[first_chunk - 1] == b) --first_chunk; // chunk index within bin
-        int k0 = C.offsets[b] + (ch - first_chunk) * C.chunk;
-        int k1 = min(C.offsets[b] + C.counts[b], k0 + C.chunk);
-        int col0 = b * C.bin_w - C.tile_lo_off;
-        int ncol = C.tile_w;
+        const int b = C.chunk_bin[ch], k0 = C.chunk_pos[ch];
+        const int k1 = min(C.offsets[b] + C.counts[b], k0 + C.chunk);
+        const int isz = b / C.nbins;
+        const int col0 = (b - isz * C.nbins) * C.bin_w - C.tile_lo_off;
+        const int ncol = C.tile_w;
         for(int i = threadIdx.x; i < 2 * ncol * nz; i += blockDim.x) tile[i] = 0.f;
         __syncthreads();
-        TileSink<real> sink{tile, col0, ncol, nz, P.NRr, 0};
-        for(int k = k0 + wave; k < k1; k += nw) {
-            uint32_t si = __builtin_amdgcn_readfirstlane(C.idx[k]);
-            SegDesc<real> d;
-            load_seg_core(O, si, d);
-            if(seg_full(P)) load_seg_rest(O, si, d);
-            if(d.isz != 0) {
-                DevSink<real> gs{&O, &P, 0};
-                scatter_seg<real, RT_TL, FAST>(d, P, gs, lane);
-                sink.nc += gs.nc;
-                continue;
-            }
-            scatter_seg<real, RT_TL, FAST>(d, P, sink, lane);
+        TileSink<real> sink{tile, col0, ncol, nz, P.NRr, isz, 0};
+        // this wavefront's segments: positions k0 + wave, + nw, ...
+        const int mine = k1 - k0 - wave > 0 ? (k1 - k0 - wave + nw - 1) / nw : 0;
+        uint32_t nums = 0;
+        uint4 next = make_uint4(0u, 0u, 0u, 0u);
+        auto fetch = [&](int j) { // the words of segment j, one per lane
+            if((j & (WAVE - 1)) == 0) nums = C.idx[k0 + wave + nw * min(j + lane, mine - 1)];
+            const uint32_t si = (uint32_t)__builtin_amdgcn_readlane((int)nums, j & (WAVE - 1));
+            if(lane < words) next = *reinterpret_cast<const uint4 *>(seg_word(O, lane, si));
+        };
+        if(mine > 0) fetch(0);
+        for(int j = 0; j < mine; ++j) {
+            if(lane < words) stage[lane] = next;
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            SegWords<real> u;
+            if(words == SEG_NW<real>) __builtin_memcpy(&u, stage, SEG_NW<real> * 16);
+            else __builtin_memcpy(&u, stage, SEG_NC<real> * 16);
+            if(j + 1 < mine) fetch(j + 1);
+            scatter_seg<real, RT_TL, FAST>(u.d, P, sink, lane);
+            // the stage is rewritten for the next segment
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         }
         __syncthreads();
-        // flush: tile column c, depth iz -> field (isz 0)
+        // flush: tile column c, depth iz -> the source's field
+        float *field = P.field + 2 * (size_t)isz * nz * P.NRr;
         for(int i = threadIdx.x; i < ncol * nz; i += blockDim.x) {
             int c = i / nz, iz = i - c * nz;
             int ir = col0 + c;
@@ -837,8 +885,8 @@ __global__ void __launch_bounds__(TILE_THREADS, 4) k_scatter_tile(Prob2D<real> P
             float re = tile[i], im = tile[ncol * nz + i];
             if(re != 0.f || im != 0.f) {
                 size_t idx = (size_t)iz * P.NRr + ir;
-                unsafeAtomicAdd(P.field + 2 * idx, re);
-                unsafeAtomicAdd(P.field + 2 * idx + 1, im);
+                unsafeAtomicAdd(field + 2 * idx, re);
+                unsafeAtomicAdd(field + 2 * idx + 1, im);
             }
         }
         __syncthreads();
@@ -945,8 +993,9 @@ __global__ void __launch_bounds__(64) k_tracenx2d(Prob2D<real> P, bhc3d::Prob3D<
     OrgNx<real> org;
     Infl<real> I;
     int job = 0, isf = 0, ia = 0, is = 0;
+    const bool full = seg_full(P);
     bool active = false, exhausted = false, init_fail = false;
-    unsigned long long steps = 0;
+    unsigned long long steps = 0, cand = 0;
     SegBlock blk{0u, 0u, 0u};
     for(int iter = 0;; ++iter) {
         if(!exhausted) {
@@ -994,27 +1043,17 @@ __global__ void __launch_bounds__(64) k_tracenx2d(Prob2D<real> P, bhc3d::Prob3D<
                 continue;
             }
         }
-        RayPt<real> p1, p2;
-        SegDesc<real> d;
-        d.nitems = 0;
-        bool two = false;
-        if(active) {
-            two = bhc3d::RayUpdateNx(p0, p1, p2, S, org, N, P, e, tabs);
-            prelude(d, p0, p1, I, is, P, G, G + P.o_rzs, isf, ia);
-            ++is;
-        }
-        append_seg(d, lane, O, blk, seg_full(P));
-        if(__any(two)) {
-            d.nitems = 0;
-            if(active && two) {
-                prelude(d, p1, p2, I, is, P, G, G + P.o_rzs, isf, ia);
-                ++is;
-            }
-            append_seg(d, lane, O, blk, seg_full(P));
-        }
+        step_ray<real, true>(
+            active, p0, I, is, P, G + P.o_rzs, G, isf, ia,
+            [&](const RayPt<real> &a, RayPt<real> &b) { return bhc3d::RayStepNx(a, b, S, org, N, e); },
+            [&](const RayPt<real> &a, RayPt<real> &b, bool top) { bhc3d::RayReflectNx(a, b, top, S, org, N, P, e, tabs); },
+            [&](bool has) { return reserve_seg<real>(has, lane, O, blk); },
+            [&](const SegDesc<real> &d, uint32_t slot) {
+                cand += candidates(d, P);
+                store_seg(d, slot, O, full);
+            });
         bool fin = false;
         if(active) {
-            p0 = two ? p2 : p1;
             if(bhc3d::RayTerminateNx(p0, is, S, org, N, e, MAXN)) {
                 active = false;
                 fin = true;
@@ -1034,8 +1073,14 @@ __global__ void __launch_bounds__(64) k_tracenx2d(Prob2D<real> P, bhc3d::Prob3D<
     }
     seal_block<real>(blk, lane, O);
     flush_err(e, O);
-    for(int off = WAVE / 2; off > 0; off >>= 1) steps += __shfl_xor(steps, off);
-    if(lane == 0) atomicAdd(O.counters + 0, steps);
+    for(int off = WAVE / 2; off > 0; off >>= 1) {
+        steps += __shfl_xor(steps, off);
+        cand += __shfl_xor(cand, off);
+    }
+    if(lane == 0) {
+        atomicAdd(O.counters + 0, steps);
+        atomicAdd(O.counters + 2, cand);
+    }
 }
 
 // Nx2D ray run type: MainRayMode (src/trace.hpp:482-520) with O3D && !R3D.
@@ -1383,7 +1428,7 @@ struct bhc_dev_problem {
     int32_t *d_work;
     double freq0;
     // range bins of the tiled TL scatter
-    int nbins, bin_w, tile_w, tile_lo_off, chunk, max_chunks;
+    int nbins, total_bins, bin_w, tile_w, tile_lo_off, chunk, max_chunks;
     int scatter_mode;           // SCATTER_AUTO / _TILED / _WAVE / _LANES
     int32_t *d_bins;            // counts | offsets | cursor | chunk_start | nchunks
     // Nx2D runs: the 3D environment the trace kernel reads (P64 / P32 then view
@@ -1707,7 +1752,7 @@ extern "C" int bhc_problem_upload2d(bhc_ctx *ctx, const bhc_problem2d *prob, con
     }
     dp->P64.base = (const double *)dp->d_blob;
     dp->P32.base = (const float *)dp->d_blob;
-    if(palloc(ctx, &dp->d_Rz, prob->NRz) || palloc(ctx, &dp->d_Sz, prob->NSz) || palloc(ctx, &dp->d_counters, 2)
+    if(palloc(ctx, &dp->d_Rz, prob->NRz) || palloc(ctx, &dp->d_Sz, prob->NSz) || palloc(ctx, &dp->d_counters, 3)
        || palloc(ctx, &dp->d_errw, 4) || palloc(ctx, &dp->d_work, 1)) {
         bhc_problem_release(dp);
         return -1;
@@ -1733,9 +1778,11 @@ extern "C" int bhc_problem_upload2d(bhc_ctx *ctx, const bhc_problem2d *prob, con
     if(tl && prob->NRr > 1 && prob->Delta_r > 0) {
         // LDS tile of 64 KiB: tile_w range columns x all depths, complex float
         int nz = prob->NRz_per_range;
-        int tile_w = (int)(65536 / ((size_t)nz * 2 * sizeof(float)));
+        int tile_w = (int)((65536 - TILE_STAGE) / ((size_t)nz * 2 * sizeof(float)));
         int margin = (int)std::ceil(prob->deltas / (2.0 * prob->Delta_r)) + 2;
-        if(tile_w >= 6 && (prob->NRr + std::max(1, tile_w - 2 * margin) - 1) / std::max(1, tile_w - 2 * margin) <= 16384) {
+        if(tile_w >= 6
+           && (long long)prob->NSz * ((prob->NRr + std::max(1, tile_w - 2 * margin) - 1) / std::max(1, tile_w - 2 * margin))
+               <= 16384) {
             int bin_w = std::max(1, tile_w - 2 * margin);
             if(bin_w == 1) margin = (tile_w - 1) / 2;
             dp->tile_w = tile_w;
@@ -1743,13 +1790,17 @@ extern "C" int bhc_problem_upload2d(bhc_ctx *ctx, const bhc_problem2d *prob, con
             dp->tile_lo_off = margin;
             dp->nbins = (prob->NRr + bin_w - 1) / bin_w;
             dp->chunk = 2048;
+            dp->total_bins = dp->nbins * prob->NSz;
             if(ensure_segs(ctx)) {
                 bhc_problem_release(dp);
                 return -1;
             }
             size_t cap = ctx->seg_bytes / sizeof(Seg<float>);
-            dp->max_chunks = (int)std::min<size_t>(cap / dp->chunk + dp->nbins + 1, 0x7FFFFFFF);
-            if(palloc(ctx, &dp->d_bins, 3 * (size_t)dp->nbins + 1 + dp->max_chunks)) {
+            // chunks hold dp->chunk segments, or fewer when there are less than
+            // two full ones per CU (run_passes): at most that many either way
+            dp->max_chunks = (int)std::min<size_t>(
+                std::max<size_t>(cap / dp->chunk, 2 * (size_t)ctx->num_cus) + dp->total_bins + 2, 0x3FFFFFFF);
+            if(palloc(ctx, &dp->d_bins, 3 * (size_t)dp->total_bins + 1 + 2 * (size_t)dp->max_chunks)) {
                 bhc_problem_release(dp);
                 return -1;
             }
@@ -1841,6 +1892,16 @@ int fan_lanes(int nrays, int num_cus)
     return std::min(WAVE, std::max(1, (nrays + simds - 1) / simds));
 }
 
+// The scatter mapping that a problem without a chosen one gets, per pass, from
+// the candidate receivers its segments bracket per step (counted by the
+// trace): below this many, one lane walks a segment alone, which for a few
+// receivers costs less than a wavefront per segment, or range bins and tiles
+// (2001 hat beams, 1.8 contributions per step: 0.28 ms against 0.71 and 0.68).
+// Above, tiles (at 8.5 contributions per step 4.4 ms against 7.2 for lanes and
+// 10.5 for wavefronts). A hat beam's bracket holds about three times the
+// receivers that it reaches, a Gaussian's hardly more than those.
+double sparse_items(bool gaussian) { return gaussian ? 6.0 : 16.0; }
+
 template<typename real> const bhc3d::Prob3D<real> &nx_of(const bhc_dev_problem *dp);
 template<> const bhc3d::Prob3D<double> &nx_of<double>(const bhc_dev_problem *dp) { return dp->N64; }
 template<> const bhc3d::Prob3D<float> &nx_of<float>(const bhc_dev_problem *dp) { return dp->N32; }
@@ -1868,7 +1929,7 @@ int run_passes(bhc_dev_problem *dp, const Prob2D<real> &P, DevOut O, void *segbu
     c->passes = 0;
     c->ph_trace_ms = c->ph_scatter_ms = 0.0;
     bool first = true;
-    unsigned long long steps_done = 0;
+    unsigned long long steps_done = 0, cand_done = 0;
     while(!todo.empty()) {
         auto r = todo.back();
         todo.pop_back();
@@ -1912,11 +1973,14 @@ int run_passes(bhc_dev_problem *dp, const Prob2D<real> &P, DevOut O, void *segbu
         }
         HIPCHECK(hipGetLastError());
         HIPCHECK(hipEventRecord(c->pb, s));
-        uint32_t of = 0;
-        unsigned long long steps_now = 0;
+        uint32_t of = 0, nseg = 0;
+        unsigned long long cnt[3] = {0, 0, 0};
         HIPCHECK(hipMemcpyAsync(&of, c->d_overflow, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-        HIPCHECK(hipMemcpyAsync(&steps_now, dp->d_counters, sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
+        HIPCHECK(hipMemcpyAsync(&nseg, c->d_seg_count, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+        HIPCHECK(hipMemcpyAsync(cnt, dp->d_counters, sizeof(cnt), hipMemcpyDeviceToHost, s));
         HIPCHECK(hipStreamSynchronize(s));
+        const unsigned long long steps_now = cnt[0];
+        nseg = std::min(nseg, O.seg_cap);
         if(phase_add(c, &c->ph_trace_ms)) return -1;
         if(of) {
             if(nj <= 1) return fail("segment buffer too small for a single ray (raise BHC_SEG_BUFFER_MB)");
@@ -1928,16 +1992,20 @@ int run_passes(bhc_dev_problem *dp, const Prob2D<real> &P, DevOut O, void *segbu
             // statistics; the counter and the words go back to the completed
             // passes' values, so that the retried rays' warnings count once
             HIPCHECK(hipMemcpyAsync(dp->d_counters, &steps_done, sizeof(unsigned long long), hipMemcpyHostToDevice, s));
+            HIPCHECK(hipMemcpyAsync(dp->d_counters + 2, &cand_done, sizeof(unsigned long long), hipMemcpyHostToDevice, s));
             HIPCHECK(hipMemcpyAsync(dp->d_errw, ew_start, sizeof(ew_start), hipMemcpyHostToDevice, s));
             HIPCHECK(hipMemcpyAsync(c->d_prog, &prog_start, sizeof(prog_start), hipMemcpyHostToDevice, s));
             HIPCHECK(hipStreamSynchronize(s));
             continue;
         }
+        const bool sparse = (double)(cnt[2] - cand_done) < sparse_items(P.isGaussian != 0) * (double)(steps_now - steps_done);
         steps_done = steps_now;
+        cand_done = cnt[2];
         if(first) HIPCHECK(hipEventRecord(c->evm, s));
         HIPCHECK(hipEventRecord(c->pa, s));
         int mode = dp->scatter_mode;
-        if(mode == SCATTER_AUTO) mode = (RT == RT_TL && c->use_tiles && dp->nbins > 0) ? SCATTER_TILED : SCATTER_WAVE;
+        if(mode == SCATTER_AUTO)
+            mode = sparse ? SCATTER_LANES : (RT == RT_TL && c->use_tiles && dp->nbins > 0) ? SCATTER_TILED : SCATTER_WAVE;
         if(mode == SCATTER_TILED && (!(RT == RT_TL && dp->nbins > 0) || own_buffer)) mode = SCATTER_WAVE;
         if(mode == SCATTER_LANES) {
             int sblocks = c->num_cus * 8;
@@ -1948,19 +2016,22 @@ int run_passes(bhc_dev_problem *dp, const Prob2D<real> &P, DevOut O, void *segbu
         } else if(mode == SCATTER_TILED) {
             BinCfg B;
             B.nbins = dp->nbins;
+            B.total = dp->total_bins;
             B.bin_w = dp->bin_w;
             B.tile_w = dp->tile_w;
             B.tile_lo_off = dp->tile_lo_off;
-            B.chunk = dp->chunk;
+            // two chunks per CU, of at most dp->chunk segments
+            B.chunk = (int)std::min<long long>(dp->chunk, std::max(64ll, (long long)nseg / (2 * c->num_cus) + 1));
             B.counts = dp->d_bins;
-            B.offsets = B.counts + dp->nbins;
-            B.cursor = B.offsets + dp->nbins;
-            B.nchunks = B.cursor + dp->nbins;
-            B.chunk_start = B.nchunks + 1;
+            B.offsets = B.counts + dp->total_bins;
+            B.cursor = B.offsets + dp->total_bins;
+            B.nchunks = B.cursor + dp->total_bins;
+            B.chunk_bin = B.nchunks + 1;
+            B.chunk_pos = B.chunk_bin + dp->max_chunks;
             B.idx = c->d_bin_idx;
-            HIPCHECK(hipMemsetAsync(B.counts, 0, dp->nbins * sizeof(int32_t), s));
+            HIPCHECK(hipMemsetAsync(B.counts, 0, dp->total_bins * sizeof(int32_t), s));
             int gb = c->num_cus * 4;
-            size_t hl = (size_t)dp->nbins * sizeof(int32_t);
+            size_t hl = (size_t)dp->total_bins * sizeof(int32_t);
             hipLaunchKernelGGL((k_bin_count<real>), dim3(gb), dim3(256), hl, s, P, O, B);
             hipLaunchKernelGGL(k_bin_scan, dim3(1), dim3(1024), 0, s, B);
             hipLaunchKernelGGL((k_bin_fill<real>), dim3(gb), dim3(256), hl, s, P, O, B);
@@ -2001,7 +2072,7 @@ int field_launch(bhc_ctx *ctx, bhc_dev_problem *dp, void *segbuf, size_t segbyte
     if(dp->d_ncand) HIPCHECK(hipMemsetAsync(dp->d_ncand, 0, dp->nrcv * sizeof(int32_t), s));
     if(dp->d_narr) HIPCHECK(hipMemsetAsync(dp->d_narr, 0, dp->nrcv * sizeof(int32_t), s));
     if(dp->d_neigen) HIPCHECK(hipMemsetAsync(dp->d_neigen, 0, sizeof(int32_t), s));
-    HIPCHECK(hipMemsetAsync(dp->d_counters, 0, 2 * sizeof(unsigned long long), s));
+    HIPCHECK(hipMemsetAsync(dp->d_counters, 0, 3 * sizeof(unsigned long long), s));
     HIPCHECK(hipMemsetAsync(dp->d_errw, 0, 4 * sizeof(uint32_t), s));
     DevOut O = make_out(dp);
     char r0 = dp->run0;
@@ -2625,8 +2696,10 @@ __device__ __attribute__((noinline)) int run_problem(const BatchDev<real> &Bdref
                 break;
             }
         }
-        step_ray<real, ST, MODE != TRACE_DESC>(
-            active, p0, S, I, is, P, B, G, isz, ia, e,
+        step_ray<real, MODE != TRACE_DESC>(
+            active, p0, I, is, P, B + P.o_rzs, G, isz, ia,
+            [&](const RayPt<real> &a, RayPt<real> &b) { return RayStep<real, ST>(a, b, S, P, B, e); },
+            [&](const RayPt<real> &a, RayPt<real> &b, bool top) { RayReflect<real, ST>(a, b, top, S, P, B, G, e); },
             [&](bool has) {
                 if constexpr(MODE == TRACE_DESC) return reserve_seg<real>(has, lane, O, blk);
                 else return 0u;
