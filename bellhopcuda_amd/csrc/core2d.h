@@ -167,10 +167,12 @@ enum : int { RT_TL = 0, RT_ARR = 1, RT_EIG = 2, RT_RAY = 3 };
 __host__ __device__ inline bool tl_run(char run0) { return run0 == 'C' || run0 == 'S' || run0 == 'I'; }
 
 // Boundary node record in the blob (BdryPtFull<false> subset). Straight-segment
-// boundaries with one set of geoacoustics use the first NODE_SHORT reals of a
-// node; curvilinear ('C') or per-node geoacoustics ('L') use all NODE_FULL.
+// boundaries with one set of geoacoustics use the first NODE_LINE reals of a
+// node, where the tangent is the normal turned by a quarter and the curvature
+// is zero (pack checks it), else NODE_SHORT; curvilinear ('C') or per-node
+// geoacoustics ('L') use all NODE_FULL.
 enum : int {
-    BN_XX = 0, BN_XY, BN_TX, BN_TY, BN_NX, BN_NY, BN_LEN, BN_KAPPA, NODE_SHORT,
+    BN_XX = 0, BN_XY, BN_NX, BN_NY, NODE_LINE, BN_TX = NODE_LINE, BN_TY, BN_LEN, BN_KAPPA, NODE_SHORT,
     BN_NDNX = NODE_SHORT, BN_NDNY, BN_NDTX, BN_NDTY, BN_CPR, BN_CPI, BN_CSR, BN_CSI, BN_RHO, BN_PAD, NODE_FULL
 };
 
@@ -1007,15 +1009,17 @@ __host__ __device__ inline void RayReflect(const RayPt<real> &p1, RayPt<real> &p
         tI = sc(FL(1.0) - sss, V(b0[BN_NDTX], b0[BN_NDTY])) + sc(sss, V(b1[BN_NDTX], b1[BN_NDTY]));
     } else {
         nI = V(b0[BN_NX], b0[BN_NY]);
-        tI = V(b0[BN_TX], b0[BN_TY]);
+        if(P.node == NODE_LINE) tI = topRefl ? V(-nI.y, nI.x) : V(nI.y, -nI.x);
+        else tI = V(b0[BN_TX], b0[BN_TY]);
     }
+    const real kappa = P.node == NODE_LINE ? RL(0.0) : b0[BN_KAPPA];
     HSd<real> hs = topRefl ? P.top : P.bot;
     if((topRefl ? P.ati_long : P.bty_long) == 'L') { // the segment's own geoacoustics
         hs.cP = C(b0[BN_CPR], b0[BN_CPI]);
         hs.cS = C(b0[BN_CSR], b0[BN_CSI]);
         hs.rho = b0[BN_RHO];
     }
-    Reflect<real, ST>(p1, p2, hs, topRefl, tI, nI, b0[BN_KAPPA], P, B, G, S, e);
+    Reflect<real, ST>(p1, p2, hs, topRefl, tI, nI, kappa, P, B, G, S, e);
     CarrySSP<real, ST>(p1.x, p2.x, p2.t, S, P, B);
     Distances(p2.x, S, S.DistEndTop, S.DistEndBot);
 }

@@ -34,8 +34,10 @@ template<typename real> int pack(const bhc_problem2d *p, std::vector<real> &blob
     P.Nr = p->ssp_nr;
     P.o_z = put(p->ssp_z, N);
     P.o_rho = put(p->ssp_rho, N);
-    P.o_c = put(p->ssp_c, 2 * (size_t)N);
-    P.o_cz = put(p->ssp_cz, 2 * (size_t)N);
+    if(p->ssp_type != 'S' && p->ssp_type != 'P') { // (splines read their coefficients only)
+        P.o_c = put(p->ssp_c, 2 * (size_t)N);
+        P.o_cz = put(p->ssp_cz, 2 * (size_t)N);
+    }
     if(p->ssp_type == 'N') {
         P.o_n2 = put(p->ssp_n2, 2 * (size_t)N);
         P.o_n2z = put(p->ssp_n2z, 2 * (size_t)N);
@@ -48,13 +50,25 @@ template<typename real> int pack(const bhc_problem2d *p, std::vector<real> &blob
     }
     // node record: compact unless a boundary is curvilinear or long format
     bool full = p->ati_type[0] == 'C' || p->bty_type[0] == 'C' || p->ati_type[1] == 'L' || p->bty_type[1] == 'L';
-    P.node = full ? NODE_FULL : NODE_SHORT;
+    // straight segments whose tangent follows from the normal (by its sign: n =
+    // (t_z, -t_r) above, (-t_z, t_r) below) and whose curvature is zero need
+    // position and normal only
+    auto line = [](const bhc_bdry_node2d *nodes, int n, bool top) {
+        for(int i = 0; i + 1 < n; ++i) {
+            const bhc_bdry_node2d &b = nodes[i];
+            const double t[2] = {top ? -b.n[1] : b.n[1], top ? b.n[0] : -b.n[0]};
+            if(b.kappa != 0.0 || memcmp(t, b.t, sizeof(t)) != 0) return false;
+        }
+        return true;
+    };
+    P.node = full ? NODE_FULL
+        : line(p->ati, p->ati_npts, true) && line(p->bty, p->bty_npts, false) ? NODE_LINE : NODE_SHORT;
     auto put_bdry = [&](const bhc_bdry_node2d *nodes, int n) {
         int32_t off = (int32_t)blob.size();
         for(int i = 0; i < n; ++i) {
             const bhc_bdry_node2d &b = nodes[i];
-            real rec[NODE_FULL] = {(real)b.x[0],     (real)b.x[1],     (real)b.t[0],     (real)b.t[1],
-                                   (real)b.n[0],     (real)b.n[1],     (real)b.Len,      (real)b.kappa,
+            real rec[NODE_FULL] = {(real)b.x[0],     (real)b.x[1],     (real)b.n[0],     (real)b.n[1],
+                                   (real)b.t[0],     (real)b.t[1],     (real)b.Len,      (real)b.kappa,
                                    (real)b.Noden[0], (real)b.Noden[1], (real)b.Nodet[0], (real)b.Nodet[1],
                                    (real)b.cP[0],    (real)b.cP[1],    (real)b.cS[0],    (real)b.cS[1],
                                    (real)b.rho,      (real)0};

@@ -148,6 +148,7 @@ struct DevOut {
     void *segs;                 // segment buffer: seg_cap descriptor cores, then seg_cap rests (seg_core / seg_rest)
     uint32_t *seg_count;
     uint32_t seg_cap;
+    int32_t seg_words;          // words of a descriptor that the buffer has rows for: SEG_NW, or SEG_NC (seg_slots)
     uint32_t *overflow;
     Progress prog;
 };
@@ -381,6 +382,9 @@ __device__ inline int wave_owner(int excl, int t)
     return own;
 }
 
+// Ray-centred rows of up to this many receivers are walked by the row's own
+// lane, without the prefix sum and the search per item: on a 400-ray seamount
+// field whose rows hold 1-6 receivers the scatter went from 86 to 77 ms.
 constexpr int RAYCEN_DIRECT = 6;
 // Scatter one segment's receivers with the 64 lanes of a wavefront (d is
 // wavefront-uniform). Both geometries have rows of different lengths --
@@ -1868,6 +1872,17 @@ DevOut make_out(bhc_dev_problem *dp)
     return O;
 }
 
+// Slots of a segment buffer of `bytes`. A sweep that stores descriptor cores
+// alone (full false) has slots of a core, so a pass holds 1.4 times as many and
+// two wavefronts per SIMD leave it as many passes as one did; a single field
+// fits in one or two passes either way. Never more than the binned order has
+// entries (ensure_segs).
+template<typename real> uint32_t seg_slots(size_t bytes, bool full)
+{
+    const size_t slot = std::max(full ? sizeof(Seg<real>) : (size_t)SEG_NC<real> * 16, sizeof(Seg<float>));
+    return (uint32_t)std::min(bytes / slot, SEG_CAP_MAX);
+}
+
 size_t seg_size(int precision) { return precision == 64 ? sizeof(Seg<double>) : sizeof(Seg<float>); }
 
 // Segment buffer: BHC_SEG_BUFFER_MB (default 16384 MiB) of HBM, allocated once per context.
@@ -1924,7 +1939,8 @@ int run_passes(bhc_dev_problem *dp, const Prob2D<real> &P, DevOut O, void *segbu
     O.segs = segbuf;
     O.seg_count = c->d_seg_count;
     O.overflow = c->d_overflow;
-    O.seg_cap = (uint32_t)std::min<size_t>(segbytes / sizeof(Seg<real>), SEG_CAP_MAX);
+    O.seg_cap = seg_slots<real>(segbytes, true);
+    O.seg_words = SEG_NW<real>;
     std::vector<std::pair<int, int>> todo{{0, dp->njobs}};
     c->passes = 0;
     c->ph_trace_ms = c->ph_scatter_ms = 0.0;
@@ -2529,7 +2545,9 @@ template<typename real> struct BatchDev {
     int32_t nprob;
     int32_t lds_cap;               // reals of LDS per workgroup for staging
     int32_t *ray_next;             // [nprob] next unclaimed ray
-    int32_t *pcursor;              // lowest problem that may have unclaimed rays
+    const int32_t *order;          // the launch's problems, those with the longest rays first
+    int32_t nlong;                 // of these, the first whose rays are much longer than the rest (long_problems)
+    int32_t *pcursor;              // first place in order whose problem may have unclaimed rays
     uint32_t *perr;                // [nprob][4] err, warn, nerr, nwarn
     unsigned long long *psteps;    // [nprob] steps
     const RaySave<real> *save_in;  // [*nsave_in][64]
@@ -2542,6 +2560,25 @@ template<typename real> struct BatchDev {
     int32_t *more;                 // set when a wavefront stopped taking new problems
     uint32_t suspend_at;           // segment count at which wavefronts suspend
 };
+
+// A copy of a structure that is the same for the whole wavefront, word by word
+// through the scalar registers: the compiler then keeps its fields there
+// instead of in a register of every lane.
+template<typename T> __device__ inline T uniform_copy(const T &src)
+{
+    static_assert(sizeof(T) % 4 == 0, "whole words");
+    int w[sizeof(T) / 4];
+    __builtin_memcpy(w, &src, sizeof(T));
+#pragma unroll
+    for(size_t i = 0; i < sizeof(T) / 4; ++i) w[i] = __builtin_amdgcn_readfirstlane(w[i]);
+    T t;
+    __builtin_memcpy(&t, w, sizeof(T));
+    return t;
+}
+
+// Rays per wavefront of a launch's longest problems: fewer rays meet fewer
+// different cases in a step, so each step is shorter.
+constexpr int LONG_LANES = 16;
 
 template<typename real> __device__ inline const real *stage_problem(const Prob2D<real> &P, int lds_cap,
                                                                     unsigned char *lds)
@@ -2579,7 +2616,7 @@ enum { TRACE_DESC = 0, TRACE_FUSED_FAST = 1, TRACE_FUSED_EXACT = 2 };
 // the descriptor stores in flight); 2, global memory known to be global; 0,
 // either, through a generic pointer (the fused mappings).
 template<typename real, char ST, int MODE, int STAGE>
-__device__ __attribute__((noinline)) int run_problem(const BatchDev<real> &Bdref, const DevOut &Oref, int pid,
+__device__ __attribute__((noinline)) int run_problem(const BatchDev<real> &Bdref, const DevOut &Oref, int pid, int lanes,
                                                      const RaySave<real> *resume, SegBlock &blk_io, unsigned char *lds,
                                                      unsigned long long &all_steps, unsigned long long &all_contrib)
 {
@@ -2587,13 +2624,14 @@ __device__ __attribute__((noinline)) int run_problem(const BatchDev<real> &Bdref
     // references their fields would be reloaded after every descriptor store;
     // the segment block in registers (through its reference, every append
     // would read it back from memory and wait for the stores in flight)
-    const DevOut O = Oref;
-    SegBlock blk = blk_io;
-    const BatchDev<real> Bd = Bdref;
+    const DevOut O = uniform_copy(Oref);
+    SegBlock blk = uniform_copy(blk_io);
+    const BatchDev<real> Bd = uniform_copy(Bdref);
+    pid = __builtin_amdgcn_readfirstlane(pid);
     const int lane = threadIdx.x;
     // a copy: through a reference the problem's fields would be reloaded after
     // every descriptor store (they might alias)
-    Prob2D<real> P = Bd.probs[pid];
+    Prob2D<real> P = uniform_copy(Bd.probs[pid]);
     const real *G = STAGE == 0 ? P.base : as_global(P.base);
     const real *B;
     if constexpr(STAGE == 1) {
@@ -2636,7 +2674,8 @@ __device__ __attribute__((noinline)) int run_problem(const BatchDev<real> &Bdref
     }
     for(int iter = 0;; ++iter) {
         if(!pexh) {
-            unsigned long long need = __ballot(!active);
+            const bool want = !active && lane < lanes;
+            unsigned long long need = __ballot(want);
             if(need) {
                 int cnt = __popcll(need);
                 int leader = __ffsll((unsigned long long)need) - 1;
@@ -2644,7 +2683,7 @@ __device__ __attribute__((noinline)) int run_problem(const BatchDev<real> &Bdref
                 if(lane == leader) base = atomicAdd(Bd.ray_next + pid, cnt);
                 base = __shfl(base, leader);
                 if(base + cnt >= nr) pexh = true;
-                if(!active) {
+                if(want) {
                     int my = base + __popcll(need & ((1ull << lane) - 1ull));
                     if(my < nr) {
                         job = my;
@@ -2697,7 +2736,7 @@ __device__ __attribute__((noinline)) int run_problem(const BatchDev<real> &Bdref
             }
         }
         step_ray<real, MODE != TRACE_DESC>(
-            active, p0, I, is, P, B + P.o_rzs, G, isz, ia,
+            active, p0, I, is, P, G + P.o_rzs, G, isz, ia,
             [&](const RayPt<real> &a, RayPt<real> &b) { return RayStep<real, ST>(a, b, S, P, B, e); },
             [&](const RayPt<real> &a, RayPt<real> &b, bool top) { RayReflect<real, ST>(a, b, top, S, P, B, G, e); },
             [&](bool has) {
@@ -2742,7 +2781,7 @@ __device__ __attribute__((noinline)) int run_problem(const BatchDev<real> &Bdref
 }
 
 template<typename real, int MODE>
-__device__ inline int run_problem_any(const BatchDev<real> &Bd, const DevOut &O, int pid, const RaySave<real> *resume,
+__device__ inline int run_problem_any(const BatchDev<real> &Bd, const DevOut &O, int pid, int lanes, const RaySave<real> *resume,
                                       SegBlock &blk, unsigned char *lds, unsigned long long &all_steps,
                                       unsigned long long &all_contrib)
 {
@@ -2750,10 +2789,10 @@ __device__ inline int run_problem_any(const BatchDev<real> &Bd, const DevOut &O,
     const bool lds_fits = Pp.staged_reals > 0 && Pp.staged_reals <= Bd.lds_cap;
 #define BHC_RUN(ST)                                                                                                   \
     if constexpr(MODE == TRACE_DESC) {                                                                                \
-        if(lds_fits) return run_problem<real, ST, MODE, 1>(Bd, O, pid, resume, blk, lds, all_steps, all_contrib);    \
-        return run_problem<real, ST, MODE, 2>(Bd, O, pid, resume, blk, lds, all_steps, all_contrib);                 \
+        if(lds_fits) return run_problem<real, ST, MODE, 1>(Bd, O, pid, lanes, resume, blk, lds, all_steps, all_contrib);    \
+        return run_problem<real, ST, MODE, 2>(Bd, O, pid, lanes, resume, blk, lds, all_steps, all_contrib);                 \
     } else {                                                                                                          \
-        return run_problem<real, ST, MODE, 0>(Bd, O, pid, resume, blk, lds, all_steps, all_contrib);                 \
+        return run_problem<real, ST, MODE, 0>(Bd, O, pid, lanes, resume, blk, lds, all_steps, all_contrib);                 \
     }
     switch(Pp.ssp_type) {
     case 'C': BHC_RUN('C')
@@ -2766,8 +2805,12 @@ __device__ inline int run_problem_any(const BatchDev<real> &Bd, const DevOut &O,
 #undef BHC_RUN
 }
 
+// Two wavefronts per SIMD (at most 256 registers, which run_problem fits
+// without spilling now that the launch's structures are scalar): a single one
+// waits for memory and for its own dependent FP64 operations in half of its
+// cycles. Each gets half of the LDS (sweep_waves).
 template<typename real, int MODE>
-__global__ void __launch_bounds__(64) k_trace_batch(BatchDev<real> Bd, DevOut O)
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) k_trace_batch(BatchDev<real> Bd, DevOut O)
 {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     const int lane = threadIdx.x;
@@ -2783,7 +2826,7 @@ __global__ void __launch_bounds__(64) k_trace_batch(BatchDev<real> Bd, DevOut O)
         }
         if(u >= 0 && u < nsave_in) {
             int pid = __builtin_amdgcn_readfirstlane(Bd.save_in_pid[u]);
-            if(run_problem_any<real, MODE>(Bd, O, pid, Bd.save_in + (size_t)u * WAVE, blk, lds_raw, all_steps,
+            if(run_problem_any<real, MODE>(Bd, O, pid, WAVE, Bd.save_in + (size_t)u * WAVE, blk, lds_raw, all_steps,
                                            all_contrib))
                 break;
             continue;
@@ -2795,19 +2838,26 @@ __global__ void __launch_bounds__(64) k_trace_batch(BatchDev<real> Bd, DevOut O)
             if(lane == 0) atomicOr(Bd.more, 1);
             break;
         }
-        int p = 0;
+        int p = 0, lanes = WAVE;
         if(lane == 0) {
             p = __hip_atomic_load(Bd.pcursor, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             while(p < Bd.nprob
-                  && __hip_atomic_load(Bd.ray_next + p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                      >= Bd.probs[p].njobs) {
+                  && __hip_atomic_load(Bd.ray_next + Bd.order[p], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                      >= Bd.probs[Bd.order[p]].njobs) {
                 atomicMax(Bd.pcursor, p + 1);
                 ++p;
             }
+            if(p < Bd.nlong) lanes = LONG_LANES;
+            p = p < Bd.nprob ? Bd.order[p] : -1;
         }
         p = __builtin_amdgcn_readfirstlane(__shfl(p, 0));
-        if(p >= Bd.nprob) break;
-        if(run_problem_any<real, MODE>(Bd, O, p, nullptr, blk, lds_raw, all_steps, all_contrib)) break;
+        lanes = __builtin_amdgcn_readfirstlane(__shfl(lanes, 0));
+        if(p < 0) break;
+        // the launch ends with its longest rays: their wavefronts go first
+        // where two share a SIMD
+        if(lanes < WAVE) __builtin_amdgcn_s_setprio(3);
+        else __builtin_amdgcn_s_setprio(0);
+        if(run_problem_any<real, MODE>(Bd, O, p, lanes, nullptr, blk, lds_raw, all_steps, all_contrib)) break;
     }
     seal_block<real>(blk, lane, O);
     for(int off = WAVE / 2; off > 0; off >>= 1) {
@@ -2915,7 +2965,7 @@ __global__ void __launch_bounds__(128) k_scatter_flat(BatchDev<real> Bd, DevOut 
         const int cnt = (int)min((uint32_t)WAVE, n - base);
         // word k of the descriptors base .. base + cnt - 1 (consecutive lanes,
         // consecutive slots) into the stage's records
-        for(int t = lane; t < cnt * SEG_NW<real>; t += WAVE) {
+        for(int t = lane; t < cnt * O.seg_words; t += WAVE) {
             const int k = t / cnt, i = t - k * cnt;
             stage[w][(size_t)i * W16 + k] = *reinterpret_cast<const uint4 *>(seg_word(O, k, base + i));
         }
@@ -2992,6 +3042,7 @@ struct bhc_sweep {
     bhc_ctx *ctx;
     int precision, nprob;
     int with_stats;
+    bool any_full;              // some problem's segments need the descriptor's rest
     std::vector<int> njobs, nrz, nrr, nsz;
     std::vector<size_t> field_off, stats_off;   // in floats / rays
     size_t field_floats, total_rays;
@@ -3001,6 +3052,10 @@ struct bhc_sweep {
     float *d_fields;
     int32_t *d_stats;
     double *d_xend;
+    std::vector<double> est;    // steps of a ray, about (the order of the problems)
+    int32_t *d_order;           // of the range order_p0, order_p1
+    int order_p0, order_p1;
+    int nlong;                  // its first problems that LONG_LANES rays per wavefront trace
     int32_t *d_ray_next, *d_pcursor, *d_resume, *d_nsave, *d_more;   // d_nsave: [2], one per parity
     uint32_t *d_perr;
     unsigned long long *d_psteps, *d_counters;
@@ -3026,7 +3081,7 @@ extern "C" void bhc_sweep_release(bhc_sweep *sw)
     (void)hipSetDevice(sw->ctx->device);
     (void)hipStreamSynchronize(sw->ctx->stream);
     void *ptrs[] = {sw->d_blobs, sw->d_probs, sw->d_rzsz,  sw->d_fields,   sw->d_stats,  sw->d_xend,
-                    sw->d_ray_next, sw->d_pcursor, sw->d_resume, sw->d_nsave, sw->d_more, sw->d_perr, sw->d_psteps,
+                    sw->d_order, sw->d_ray_next, sw->d_pcursor, sw->d_resume, sw->d_nsave, sw->d_more, sw->d_perr, sw->d_psteps,
                     sw->d_counters, sw->d_save[0], sw->d_save[1], sw->d_save_pid[0], sw->d_save_pid[1]};
     for(void *p : ptrs)
         if(p) (void)hipFree(p);
@@ -3036,6 +3091,20 @@ extern "C" void bhc_sweep_release(bhc_sweep *sw)
 }
 
 namespace {
+
+constexpr int SWEEP_LDS2 = 20480;   // LDS per trace wavefront that leaves room for two per SIMD
+
+// Segments that the sweep's wavefronts may add between two polls: 2 per lane
+// per step, 32 steps apart, plus one partly used slot block each.
+size_t sweep_margin(int waves) { return (size_t)waves * (2 * 32 * WAVE + 2 * SEG_BLOCK); }
+
+// Wavefronts of a sweep's trace: two per SIMD where the LDS budget and the
+// segment buffer (which must hold their margin twice over) allow it, else one.
+int sweep_waves(const bhc_sweep *sw, size_t seg_cap)
+{
+    const bool two = sw->lds_bytes <= SWEEP_LDS2 && 2 * sweep_margin(sw->max_waves) < seg_cap;
+    return two ? sw->max_waves : sw->max_waves / 2;
+}
 
 template<typename real>
 int sweep_upload(bhc_sweep *sw, const bhc_problem2d *const *probs)
@@ -3060,11 +3129,17 @@ int sweep_upload(bhc_sweep *sw, const bhc_problem2d *const *probs)
         boff[i] = blobs.size();
         blobs.insert(blobs.end(), blob.begin(), blob.end());
         while(blobs.size() % 32) blobs.push_back((real)0);
+        sw->any_full = sw->any_full || seg_full(P[i]);
+        P[i].staged_reals = P[i].o_rzs;   // (the depths are read by the fused mappings only, from global memory)
         max_staged = std::max(max_staged, (size_t)P[i].staged_reals);
         rzoff[i] = rzsz.size();
         rzsz.insert(rzsz.end(), p->Rz, p->Rz + p->NRz);
         szoff[i] = rzsz.size();
         rzsz.insert(rzsz.end(), p->Sz, p->Sz + p->NSz);
+        // steps of a ray, about: one per step length, boundary node and profile
+        // knot passed on a zigzag at 15 degrees
+        const double depth = std::max(1e-3, p->bot_hs.depth > 0 ? p->bot_hs.depth : p->box_z);
+        sw->est.push_back(p->box_r / p->deltas + p->bty_npts + p->ati_npts + 0.27 * p->box_r / depth * p->ssp_npts);
         sw->njobs.push_back((p->iSingle_alpha >= 1 ? 1 : p->Nalpha) * p->NSz);
         sw->nsz.push_back(p->NSz);
         sw->nrz.push_back(p->NRz_per_range);
@@ -3075,15 +3150,17 @@ int sweep_upload(bhc_sweep *sw, const bhc_problem2d *const *probs)
         sw->stats_off[i] = sw->total_rays;
         sw->total_rays += sw->njobs.back();
     }
-    // LDS per workgroup: up to 40 KiB, so that four single-wavefront
-    // workgroups fit a CU's 160 KiB; larger tables stay in global memory
+    // LDS per workgroup: by default at most 20 KiB, so that eight
+    // single-wavefront workgroups (two per SIMD) fit a CU's 160 KiB; up to
+    // 40 KiB can be set, which leaves one per SIMD. Larger tables stay in
+    // global memory
     size_t cap_reals = std::min<size_t>((size_t)40960, (size_t)ctx->lds_max) / sizeof(real);
     size_t lds_reals = std::min(max_staged, cap_reals);
-    sw->lds_bytes = (int)(lds_reals * sizeof(real));
-    sw->lds_bytes_max = sw->lds_bytes;
+    sw->lds_bytes_max = (int)(lds_reals * sizeof(real));
+    sw->lds_bytes = std::min(sw->lds_bytes_max, SWEEP_LDS2);
     if(dalloc((real **)&sw->d_blobs, blobs.size()) || dalloc(&sw->d_rzsz, rzsz.size())
        || dalloc(&sw->d_fields, sw->field_floats) || dalloc((Prob2D<real> **)&sw->d_probs, (size_t)n)
-       || dalloc(&sw->d_ray_next, (size_t)n) || dalloc(&sw->d_pcursor, 1) || dalloc(&sw->d_resume, 1)
+       || dalloc(&sw->d_order, (size_t)n) || dalloc(&sw->d_ray_next, (size_t)n) || dalloc(&sw->d_pcursor, 1) || dalloc(&sw->d_resume, 1)
        || dalloc(&sw->d_nsave, 2) || dalloc(&sw->d_more, 1) || dalloc(&sw->d_perr, 4 * (size_t)n)
        || dalloc(&sw->d_psteps, (size_t)n)
        || dalloc(&sw->d_counters, 2))
@@ -3106,9 +3183,7 @@ int sweep_upload(bhc_sweep *sw, const bhc_problem2d *const *probs)
         }
     }
     HIPCHECK(hipMemcpy(sw->d_probs, P.data(), n * sizeof(Prob2D<real>), hipMemcpyHostToDevice));
-    // one single-wavefront workgroup per SIMD: the trace kernel runs at one
-    // wavefront per SIMD (register bound), and 4 x 40 KiB of LDS fill a CU
-    sw->max_waves = ctx->num_cus * 4;
+    sw->max_waves = ctx->num_cus * 8;   // two per SIMD
     size_t save_units = (size_t)sw->max_waves;
     for(int k = 0; k < 2; ++k)
         if(dalloc((RaySave<real> **)&sw->d_save[k], save_units * WAVE) || dalloc(&sw->d_save_pid[k], save_units))
@@ -3127,6 +3202,7 @@ template<typename real> BatchDev<real> batch_dev(bhc_sweep *sw, int p0, int p1)
     Bd.probs = (const Prob2D<real> *)sw->d_probs + p0;
     Bd.nprob = p1 - p0;
     Bd.lds_cap = sw->lds_bytes / (int)sizeof(real);
+    Bd.order = sw->d_order;
     Bd.ray_next = sw->d_ray_next + p0;
     Bd.pcursor = sw->d_pcursor;
     Bd.perr = sw->d_perr + 4 * (size_t)p0;
@@ -3145,7 +3221,8 @@ template<typename real> DevOut batch_out(bhc_sweep *sw)
     O.segs = c->segs;
     O.seg_count = c->d_seg_count;
     O.overflow = c->d_overflow;
-    O.seg_cap = (uint32_t)std::min<size_t>(c->seg_bytes / sizeof(Seg<real>), SEG_CAP_MAX);
+    O.seg_cap = seg_slots<real>(c->seg_bytes, sw->any_full);
+    O.seg_words = sw->any_full ? SEG_NW<real> : SEG_NC<real>;
     O.prog = prog_of(c);
     return O;
 }
@@ -3162,20 +3239,21 @@ template<typename real> void enqueue_pass(bhc_sweep *sw, BatchDev<real> Bd, cons
     Bd.save_out = (RaySave<real> *)sw->d_save[1 - cur];
     Bd.save_out_pid = sw->d_save_pid[1 - cur];
     Bd.nsave_out = sw->d_nsave + (1 - cur);
+    const int waves = sweep_waves(sw, O.seg_cap);
     hipLaunchKernelGGL(k_pass_reset, dim3(1), dim3(64), 0, s, c->d_seg_count, c->d_overflow, sw->d_resume,
                        sw->d_nsave + (1 - cur), sw->d_more);
     if(sw->scatter_lanes == 3) {
         // fused: the trace evaluates every step's receivers itself
         if(c->exact_phasor)
-            hipLaunchKernelGGL((k_trace_batch<real, TRACE_FUSED_EXACT>), dim3(sw->max_waves), dim3(WAVE), sw->lds_bytes,
+            hipLaunchKernelGGL((k_trace_batch<real, TRACE_FUSED_EXACT>), dim3(waves), dim3(WAVE), sw->lds_bytes,
                                s, Bd, O);
         else
-            hipLaunchKernelGGL((k_trace_batch<real, TRACE_FUSED_FAST>), dim3(sw->max_waves), dim3(WAVE), sw->lds_bytes,
+            hipLaunchKernelGGL((k_trace_batch<real, TRACE_FUSED_FAST>), dim3(waves), dim3(WAVE), sw->lds_bytes,
                                s, Bd, O);
         if(e_mid) (void)hipEventRecord(e_mid, s);
         return;
     }
-    hipLaunchKernelGGL((k_trace_batch<real, TRACE_DESC>), dim3(sw->max_waves), dim3(WAVE), sw->lds_bytes, s, Bd, O);
+    hipLaunchKernelGGL((k_trace_batch<real, TRACE_DESC>), dim3(waves), dim3(WAVE), sw->lds_bytes, s, Bd, O);
     if(e_mid) (void)hipEventRecord(e_mid, s);
     if(sw->scatter_lanes == 2) {
         if(c->exact_phasor)
@@ -3206,9 +3284,7 @@ template<typename real> int sweep_core(bhc_sweep *sw, int p0, int p1, bool graph
     if(ensure_segs(c)) return -1;
     BatchDev<real> Bd = batch_dev<real>(sw, p0, p1);
     DevOut O = batch_out<real>(sw);
-    // every wavefront may add 2 segments per lane per step between two polls
-    // (32 steps apart) plus one partly used slot block
-    size_t margin = (size_t)sw->max_waves * (2 * 32 * WAVE + 2 * SEG_BLOCK);
+    size_t margin = sweep_margin(sweep_waves(sw, O.seg_cap));
     if(margin * 2 >= O.seg_cap) return fail("segment buffer too small for a batched sweep (raise BHC_SEG_BUFFER_MB)");
     Bd.suspend_at = (uint32_t)(O.seg_cap - margin);
     const int np = p1 - p0;
@@ -3217,6 +3293,32 @@ template<typename real> int sweep_core(bhc_sweep *sw, int p0, int p1, bool graph
         for(int i = p0; i < p1; ++i) rays += sw->njobs[i];
         if(prog_begin(c, rays)) return -1;
     }
+    // The problems with the longest rays go first: a launch ends with its
+    // longest ray, and one of 17800 steps among 1700 on average, started last,
+    // would run alone at the end.
+    if(sw->order_p0 != p0 || sw->order_p1 != p1) {
+        std::vector<int32_t> order(np);
+        for(int i = 0; i < np; ++i) order[i] = i;
+        std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return sw->est[p0 + a] > sw->est[p0 + b]; });
+        // much longer than the mean over the rays, and together on at most a
+        // quarter of the wavefronts
+        double rays = 0, steps = 0;
+        for(int i = p0; i < p1; ++i) {
+            rays += sw->njobs[i];
+            steps += sw->njobs[i] * sw->est[i];
+        }
+        long long waves = 0;
+        for(sw->nlong = 0; sw->nlong < np; ++sw->nlong) {
+            const int q = p0 + order[sw->nlong];
+            waves += (sw->njobs[q] + LONG_LANES - 1) / LONG_LANES;
+            if(!(sw->est[q] > 1.5 * steps / rays) || waves > sw->max_waves / 4) break;
+        }
+        HIPCHECK(hipStreamSynchronize(s));
+        HIPCHECK(hipMemcpy(sw->d_order, order.data(), np * sizeof(int32_t), hipMemcpyHostToDevice));
+        sw->order_p0 = p0;
+        sw->order_p1 = p1;
+    }
+    Bd.nlong = sw->nlong;
     const size_t f0 = sw->field_off[p0], f1 = p1 == sw->nprob ? sw->field_floats : sw->field_off[p1];
     HIPCHECK(hipMemsetAsync(sw->d_fields + f0, 0, (f1 - f0) * sizeof(float), s));
     HIPCHECK(hipMemsetAsync(sw->d_ray_next + p0, 0, np * sizeof(int32_t), s));
@@ -3318,11 +3420,10 @@ template<typename real> int sweep_tune(bhc_sweep *sw)
     int nsub = std::min(sw->nprob, 64);
     int cus = sw->ctx->num_cus;
     const int grids[3] = {cus * 4, cus * 8, cus * 16};
-    // staging budgets: the full one (one wavefront per SIMD), half of it (two
-    // wavefronts per SIMD, problems with larger tables unstaged) and none
-    const int rsz = (int)(sw->precision == 64 ? sizeof(double) : sizeof(float));
-    const int half = (sw->lds_bytes_max / 2) / rsz * rsz;
-    const int ldss[3] = {sw->lds_bytes_max, half, 0};
+    // staging budgets: the default (two wavefronts per SIMD, problems with
+    // larger tables unstaged), the largest table's (one wavefront per SIMD where
+    // it is over the default) and none
+    const int ldss[3] = {std::min(sw->lds_bytes_max, SWEEP_LDS2), sw->lds_bytes_max, 0};
     auto timed = [&](int mode, int blocks, int lds, double &t) -> int {
         sw->scatter_lanes = mode;
         sw->scatter_blocks = blocks;
@@ -3334,7 +3435,7 @@ template<typename real> int sweep_tune(bhc_sweep *sw)
         return 0;
     };
     // the staging budget acts on the trace and the mapping / grid on the
-    // scatter: choose the scatter's at the full budget, then the budget
+    // scatter: choose the scatter's at the default budget, then the budget
     int best_blocks = grids[0], best_lanes = 1, best_lds = ldss[0];
     double best = 1e300, t = 0.0;
     for(int mode = 0; mode < 4; ++mode)
@@ -3346,7 +3447,8 @@ template<typename real> int sweep_tune(bhc_sweep *sw)
                 best_lanes = mode;
             }
         }
-    for(int li = 1; li < (sw->lds_bytes_max > 0 ? 3 : 1); ++li) {
+    for(int li = 1; li < 3; ++li) {
+        if(ldss[li] == ldss[li - 1]) continue;
         if(timed(best_lanes, best_blocks, ldss[li], t)) return -1;
         if(t < best) {
             best = t;
@@ -3429,10 +3531,11 @@ extern "C" int bhc_sweep_set_launch(bhc_sweep *sw, int scatter_blocks, int lds_b
     if(!sw) return fail("bhc_sweep_set_launch: null sweep");
     const int rsz = sw->precision == 64 ? (int)sizeof(double) : (int)sizeof(float);
     if(scatter_blocks < 1 || scatter_blocks > (1 << 20)) return fail("bhc_sweep_set_launch: scatter_blocks out of range");
-    if(lds_bytes < 0 || lds_bytes > sw->lds_bytes_max || lds_bytes % rsz)
-        return fail("bhc_sweep_set_launch: lds_bytes must be a multiple of %d in [0, %d]", rsz, sw->lds_bytes_max);
+    const int most = std::max(sw->lds_bytes_max, std::min(2 * SWEEP_LDS2, sw->ctx->lds_max));
+    if(lds_bytes < 0 || lds_bytes > most || lds_bytes % rsz)
+        return fail("bhc_sweep_set_launch: lds_bytes must be a multiple of %d in [0, %d]", rsz, most);
     sw->scatter_blocks = scatter_blocks;
-    sw->lds_bytes = lds_bytes;
+    sw->lds_bytes = std::min(lds_bytes, sw->lds_bytes_max);
     sw->tuned = true;
     return 0;
 }
