@@ -255,16 +255,6 @@ template<typename real> struct DevSink {
     __device__ void mark() {}
 };
 
-template<typename real> __device__ inline const real *stage(const Prob2D<real> &P, unsigned char *lds)
-{
-    const real *G = P.base;
-    if(P.staged_reals <= 0) return G;
-    real *L = reinterpret_cast<real *>(lds);
-    for(int i = threadIdx.x; i < P.staged_reals; i += blockDim.x) L[i] = G[i];
-    __syncthreads();
-    return L;
-}
-
 __device__ inline void flush_err(const Err &e, const DevOut &O)
 {
     if(e.err) atomicOr(O.errw + 0, e.err);
@@ -922,15 +912,29 @@ template<typename real> __device__ inline void store_pt(bhc_ray_pt2d *d, const R
 }
 
 // Ray run type and eigenray re-trace: MainRayMode, src/trace.hpp:482-520.
-template<typename real>
-__global__ void __launch_bounds__(256) k_ray2d(Prob2D<real> P, DevOut O)
+// Bound by the serial chain of a ray's steps. A plot's few rays are spread over
+// the wavefronts (O.lanes, as the field trace's), and the tables are read as
+// there (STAGED, ST): 101 rays of a
+// Munk fan with all their points, the call from 4.6 to 3.3 ms.
+template<typename real, char ST, bool STAGED>
+__global__ void __launch_bounds__(WAVE) k_ray2d(Prob2D<real> P, DevOut O)
 {
     extern __shared__ __align__(16) unsigned char lds_raw[];
-    const real *B = stage(P, lds_raw);
-    const real *G = P.base;
+    const real *G = as_global(P.base);
+    const real *B;
+    if constexpr(STAGED) {
+        real *L = reinterpret_cast<real *>(lds_raw);
+        for(int i = threadIdx.x; i < P.staged_reals; i += WAVE) L[i] = G[i];
+        __syncthreads();
+        B = L;
+    } else {
+        B = G;
+    }
+    bhc_ray_pt2d *const points = as_global(O.points);
+    const int first = threadIdx.x < O.lanes ? (int)(blockIdx.x * O.lanes + threadIdx.x) : O.job_end;
     Err e = {0, 0, 0, 0};
     const int M = O.max_points;
-    for(int job = blockIdx.x * blockDim.x + threadIdx.x; job < O.job_end; job += gridDim.x * blockDim.x) {
+    for(int job = first; job < O.job_end; job += gridDim.x * O.lanes) {
         int isz, ia;
         if(O.job_alpha) {
             ia = O.job_alpha[job];
@@ -938,12 +942,12 @@ __global__ void __launch_bounds__(256) k_ray2d(Prob2D<real> P, DevOut O)
         } else {
             JobIndices(job, P, isz, ia);
         }
-        bhc_ray_pt2d *ray = O.points + (size_t)job * M;
+        bhc_ray_pt2d *ray = points + (size_t)job * M;
         RayPt<real> p0, p1, p2;
         Trace<real> S;
         Infl<real> I;
         int Nsteps = O.nsteps_in ? O.nsteps_in[job] : -1;
-        bool ok = RayInit(isz, ia, p0, S, I, P, B, G, e);
+        bool ok = RayInit<real, ST>(isz, ia, p0, S, I, P, B, G, e);
         store_pt(ray, p0);
         if(!ok) {
             O.nsteps_out[job] = 1;
@@ -952,7 +956,7 @@ __global__ void __launch_bounds__(256) k_ray2d(Prob2D<real> P, DevOut O)
         int is = 0;
         for(;;) {
             if(e.err) break;
-            bool two = RayUpdate(p0, p1, p2, S, P, B, G, e);
+            bool two = RayUpdate<real, ST>(p0, p1, p2, S, P, B, G, e);
             store_pt(ray + is + 1, p1);
             if(two) store_pt(ray + is + 2, p2);
             if(Nsteps >= 0 && is >= Nsteps) {
@@ -2233,6 +2237,26 @@ extern "C" int bhc_field_run2d(bhc_ctx *ctx, const bhc_problem2d *prob, bhc_fiel
     return rc;
 }
 
+namespace {
+template<typename real> void launch_rays(bhc_dev_problem *dp, const Prob2D<real> &P, const DevOut &O, int blocks)
+{
+    hipStream_t s = dp->ctx->stream;
+#define BHC_RAYS(ST)                                                                                                   \
+    if(dp->lds_bytes) hipLaunchKernelGGL((k_ray2d<real, ST, true>), dim3(blocks), dim3(WAVE), dp->lds_bytes, s, P, O); \
+    else hipLaunchKernelGGL((k_ray2d<real, ST, false>), dim3(blocks), dim3(WAVE), 0, s, P, O);                         \
+    break;
+    switch(P.ssp_type) {
+    case 'C': BHC_RAYS('C')
+    case 'S': BHC_RAYS('S')
+    case 'P': BHC_RAYS('P')
+    case 'N': BHC_RAYS('N')
+    case 'Q': BHC_RAYS('Q')
+    default: BHC_RAYS('A')
+    }
+#undef BHC_RAYS
+}
+} // namespace
+
 extern "C" int bhc_ray_run2d(bhc_ctx *ctx, const bhc_problem2d *prob, bhc_ray_out *out)
 {
     return bhc_ray_run2d_list(ctx, prob, out, nullptr, nullptr, nullptr, -1);
@@ -2284,11 +2308,10 @@ extern "C" int bhc_ray_run2d_list(bhc_ctx *ctx, const bhc_problem2d *prob, bhc_r
         O.nsteps_out = d_nout;
         hipMemsetAsync(dp->d_errw, 0, 4 * sizeof(uint32_t), ctx->stream);
         hipMemsetAsync(d_pts, 0, npts * sizeof(bhc_ray_pt2d), ctx->stream);
-        int blocks = std::max(1, std::min((njobs + 255) / 256, ctx->num_cus * ctx->bpc));
-        if(dp->precision == 64)
-            hipLaunchKernelGGL(k_ray2d<double>, dim3(blocks), dim3(256), dp->lds_bytes, ctx->stream, dp->P64, O);
-        else
-            hipLaunchKernelGGL(k_ray2d<float>, dim3(blocks), dim3(256), dp->lds_bytes, ctx->stream, dp->P32, O);
+        O.lanes = fan_lanes(njobs, ctx->num_cus);
+        const int blocks = std::min((njobs + O.lanes - 1) / O.lanes, ctx->num_cus * 4 * ctx->bpc);
+        if(dp->precision == 64) launch_rays(dp, dp->P64, O, blocks);
+        else launch_rays(dp, dp->P32, O, blocks);
         if(hipGetLastError() != hipSuccess || hipStreamSynchronize(ctx->stream) != hipSuccess) {
             rc = fail("ray kernel failed");
         } else {

@@ -183,3 +183,22 @@ def test_network_tiles(n, n_out, front):
             assert np.array_equal(m.predict(x[:k]), whole[:, :k])
     finally:
         m.close()
+
+
+@pytest.mark.parametrize("nodes", [2, 3000])
+@pytest.mark.parametrize("ssp_type", ["C", "N", "S", "P"])
+@pytest.mark.parametrize("nbeams", [2, 65, 1100])
+def test_ray_paths_spread_over_wavefronts(nbeams, ssp_type, nodes, gpu_ctx):
+    """Every point of every ray, bit for bit, for fans below and above one ray
+    per SIMD and tables in the LDS and in memory."""
+    _announce("ray_paths_%d_%s_%d" % (nbeams, ssp_type, nodes))
+    e = munk_env(nbeams=nbeams, run_type="RG", ssp_type=ssp_type, r_max_km=20.0)
+    r = np.linspace(0.0, 21.0, nodes)
+    e.bty = Boundary("LS", r_km=r, z=4600.0 - 300.0 * np.sin(r / 3.0))
+    e.box_r_km = 21.0
+    po, no, _ = oracle.ray_run(e, max_points=600)
+    pg, ng, _ = bh.ray_run(e, ctx=gpu_ctx, max_points=600)
+    assert np.array_equal(no, ng)
+    for k in range(len(no)):
+        for f in ("x", "t", "NumTopBnc", "NumBotBnc"):
+            assert np.array_equal(po[k, :no[k]][f], pg[k, :no[k]][f]), (k, f)
