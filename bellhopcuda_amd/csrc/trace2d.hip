@@ -3447,12 +3447,12 @@ template<typename real> int sweep_tune(bhc_sweep *sw)
     // larger tables unstaged), the largest table's (one wavefront per SIMD where
     // it is over the default) and none
     const int ldss[3] = {std::min(sw->lds_bytes_max, SWEEP_LDS2), sw->lds_bytes_max, 0};
-    auto timed = [&](int mode, int blocks, int lds, double &t) -> int {
+    auto timed = [&](int mode, int blocks, int lds, int n, double &t) -> int {
         sw->scatter_lanes = mode;
         sw->scatter_blocks = blocks;
         sw->lds_bytes = lds;
         for(int rep = 0; rep < 2; ++rep) {
-            if(sweep_core<real>(sw, 0, nsub, false)) return -1;
+            if(sweep_core<real>(sw, 0, n, false)) return -1;
             if(rep == 1) t = sw->trace_ms + sw->scatter_ms;
         }
         return 0;
@@ -3463,16 +3463,23 @@ template<typename real> int sweep_tune(bhc_sweep *sw)
     double best = 1e300, t = 0.0;
     for(int mode = 0; mode < 4; ++mode)
         for(int gi = 0; gi < (mode == 3 ? 1 : 3); ++gi) {   // the fused mode launches no scatter
-            if(timed(mode, grids[gi], ldss[0], t)) return -1;
+            if(timed(mode, grids[gi], ldss[0], nsub, t)) return -1;
             if(t < best) {
                 best = t;
                 best_blocks = grids[gi];
                 best_lanes = mode;
             }
         }
-    for(int li = 1; li < 3; ++li) {
-        if(ldss[li] == ldss[li - 1]) continue;
-        if(timed(best_lanes, best_blocks, ldss[li], t)) return -1;
+    // the budget acts on how well the trace hides its waits, which shows once
+    // there is work for every wavefront: 64 problems end with a few long rays on
+    // an idle chip, where one wavefront per SIMD is the faster (of 4096 unlike
+    // environments, 303 fields/s with the budget that 64 chose, 363 with two
+    // wavefronts per SIMD)
+    const int nlds = std::min(sw->nprob, 256);
+    best = 1e300;
+    for(int li = 0; li < 3; ++li) {
+        if(li > 0 && ldss[li] == ldss[li - 1]) continue;
+        if(timed(best_lanes, best_blocks, ldss[li], nlds, t)) return -1;
         if(t < best) {
             best = t;
             best_lds = ldss[li];
