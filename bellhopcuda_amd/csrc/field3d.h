@@ -803,7 +803,8 @@ int ray3d(bhc_ctx *c, const bhc_problem3d *p, bhc_ray_out3d *out, const bhc_eige
     if(hipMemcpyAsync(d_blob, blob.data(), blob.size() * sizeof(real), hipMemcpyHostToDevice, s) != hipSuccess
        || hipMemcpyAsync(d_Rz, p->Rz, p->NRz * sizeof(float), hipMemcpyHostToDevice, s) != hipSuccess
        || hipMemcpyAsync(d_Sz, p->Sz, p->NSz * sizeof(float), hipMemcpyHostToDevice, s) != hipSuccess
-       || hipMemsetAsync(d_errw, 0, 4 * sizeof(uint32_t), s) != hipSuccess) {
+       || hipMemsetAsync(d_errw, 0, 4 * sizeof(uint32_t), s) != hipSuccess
+       || (njobs > 0 && hipMemsetAsync(d_pts, 0, (size_t)njobs * M * sizeof(bhc_ray_pt3d), s) != hipSuccess)) {
         cleanup();
         return fail("bhc_ray_run3d: upload failed");
     }
@@ -894,6 +895,8 @@ template<typename real> int run3d(bhc_ctx *c, const bhc_problem3d *p, bhc_field_
     if(out->ray_nsteps) {
         TRY(palloc(c, &d_stats, 3 * (size_t)njobs));
         TRY(palloc(c, &d_xend, 3 * (size_t)njobs));
+        HTRY(hipMemsetAsync(d_stats, 0, 3 * (size_t)njobs * sizeof(int32_t), s));
+        HTRY(hipMemsetAsync(d_xend, 0, 3 * (size_t)njobs * sizeof(double), s));
     }
     HTRY(hipMemcpyAsync(d_blob, blob.data(), blob.size() * sizeof(real), hipMemcpyHostToDevice, s));
     HTRY(hipMemcpyAsync(d_Rz, p->Rz, p->NRz * sizeof(float), hipMemcpyHostToDevice, s));
@@ -916,6 +919,8 @@ template<typename real> int run3d(bhc_ctx *c, const bhc_problem3d *p, bhc_field_
         TRY(palloc(c, &d_arr, nrcv * (size_t)out->max_narr));
         TRY(palloc(c, &d_narr, nrcv));
         HTRY(hipMemsetAsync(d_ncand, 0, nrcv * sizeof(int32_t), s));
+        // (the merge writes a receiver's arrivals, not the slots past them)
+        HTRY(hipMemsetAsync(d_arr, 0, nrcv * (size_t)out->max_narr * sizeof(bhc_arrival), s));
     }
     if(hits_too) {
         TRY(palloc(c, &d_hits, (size_t)out->eigen_memsize));

@@ -1434,6 +1434,7 @@ struct bhc_dev_problem {
     unsigned long long *d_counters;
     uint32_t *d_errw;
     int32_t *d_work;
+    int cleared;                // the outputs hold zeros or a launch's results (clear_outputs)
     double freq0;
     // range bins of the tiled TL scatter
     int nbins, total_bins, bin_w, tile_w, tile_lo_off, chunk, max_chunks;
@@ -2083,17 +2084,30 @@ int run_passes(bhc_dev_problem *dp, const Prob2D<real> &P, DevOut O, void *segbu
 extern "C" int bhc_problem_autotune(bhc_ctx *ctx, bhc_dev_problem *dp, int *mode_out);
 
 namespace {
+// Zeros in every output of a problem that reaches the caller: its blocks may
+// have served another run, and a launch need not write all of them (arrival
+// slots past a receiver's count, rays that an error stopped).
+int clear_outputs(bhc_dev_problem *dp, hipStream_t s)
+{
+    if(dp->d_field) HIPCHECK(hipMemsetAsync(dp->d_field, 0, 2 * dp->nrcv * sizeof(float), s));
+    if(dp->d_ncand) HIPCHECK(hipMemsetAsync(dp->d_ncand, 0, dp->nrcv * sizeof(int32_t), s));
+    if(dp->d_arr) HIPCHECK(hipMemsetAsync(dp->d_arr, 0, dp->nrcv * dp->max_narr * sizeof(bhc_arrival), s));
+    if(dp->d_narr) HIPCHECK(hipMemsetAsync(dp->d_narr, 0, dp->nrcv * sizeof(int32_t), s));
+    if(dp->d_neigen) HIPCHECK(hipMemsetAsync(dp->d_neigen, 0, sizeof(int32_t), s));
+    if(dp->d_stats) HIPCHECK(hipMemsetAsync(dp->d_stats, 0, 3 * (size_t)dp->njobs * sizeof(int32_t), s));
+    if(dp->d_xend) HIPCHECK(hipMemsetAsync(dp->d_xend, 0, (size_t)dp->xend_dim * dp->njobs * sizeof(double), s));
+    HIPCHECK(hipMemsetAsync(dp->d_counters, 0, 3 * sizeof(unsigned long long), s));
+    HIPCHECK(hipMemsetAsync(dp->d_errw, 0, 4 * sizeof(uint32_t), s));
+    dp->cleared = 1;
+    return 0;
+}
+
 int field_launch(bhc_ctx *ctx, bhc_dev_problem *dp, void *segbuf, size_t segbytes)
 {
     HIPCHECK(hipSetDevice(ctx->device));
     hipStream_t s = ctx->stream;
     if(prog_begin(ctx, dp->njobs)) return -1;
-    if(dp->d_field) HIPCHECK(hipMemsetAsync(dp->d_field, 0, 2 * dp->nrcv * sizeof(float), s));
-    if(dp->d_ncand) HIPCHECK(hipMemsetAsync(dp->d_ncand, 0, dp->nrcv * sizeof(int32_t), s));
-    if(dp->d_narr) HIPCHECK(hipMemsetAsync(dp->d_narr, 0, dp->nrcv * sizeof(int32_t), s));
-    if(dp->d_neigen) HIPCHECK(hipMemsetAsync(dp->d_neigen, 0, sizeof(int32_t), s));
-    HIPCHECK(hipMemsetAsync(dp->d_counters, 0, 3 * sizeof(unsigned long long), s));
-    HIPCHECK(hipMemsetAsync(dp->d_errw, 0, 4 * sizeof(uint32_t), s));
+    if(clear_outputs(dp, s)) return -1;
     DevOut O = make_out(dp);
     char r0 = dp->run0;
     int rt = (r0 == 'C' || r0 == 'S' || r0 == 'I') ? RT_TL : (r0 == 'E') ? RT_EIG : RT_ARR;
@@ -2186,6 +2200,7 @@ extern "C" int bhc_problem_autotune(bhc_ctx *ctx, bhc_dev_problem *dp, int *mode
 extern "C" int bhc_field_download(bhc_ctx *ctx, bhc_dev_problem *dp, bhc_field_out *out)
 {
     HIPCHECK(hipSetDevice(ctx->device));
+    if(!dp->cleared && clear_outputs(dp, ctx->stream)) return -1;   // not launched yet
     HIPCHECK(hipStreamSynchronize(ctx->stream));
     if(out->field && dp->d_field)
         HIPCHECK(hipMemcpy(out->field, dp->d_field, 2 * dp->nrcv * sizeof(float), hipMemcpyDeviceToHost));
