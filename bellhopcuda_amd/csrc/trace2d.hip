@@ -1906,10 +1906,17 @@ int ensure_segs(bhc_ctx *c)
 // wavefronts. A wavefront walks the code of every case that one of its lanes
 // meets in a step (reflection, profile knot, receiver range, refill), so
 // fewer rays per wavefront make each step shorter.
-int fan_lanes(int nrays, int num_cus)
+// Every wavefront takes a slot block of its own, so a small segment buffer
+// (slots; 0: none) bounds their number: together they may leave an eighth of it
+// in partly used blocks. 2001 rays on 1001 wavefronts overflow the
+// allocation-free launch's 64 MiB whatever they trace: over 5 km 2.75 ms in four
+// passes, against 0.67 ms in one on the 113 wavefronts of this bound and 0.85 on
+// 32 full ones.
+int fan_lanes(int nrays, int num_cus, size_t slots)
 {
-    const int simds = std::max(1, 4 * num_cus);
-    return std::min(WAVE, std::max(1, (nrays + simds - 1) / simds));
+    size_t waves = std::max(1, 4 * num_cus);
+    if(slots) waves = std::min(waves, std::max<size_t>(1, slots / (8 * (size_t)SEG_BLOCK)));
+    return (int)std::min<size_t>(WAVE, std::max<size_t>(1, ((size_t)nrays + waves - 1) / waves));
 }
 
 // The scatter mapping that a problem without a chosen one gets, per pass, from
@@ -1960,7 +1967,7 @@ int run_passes(bhc_dev_problem *dp, const Prob2D<real> &P, DevOut O, void *segbu
         HIPCHECK(hipMemsetAsync(c->d_overflow, 0, sizeof(uint32_t), s));
         HIPCHECK(hipMemsetAsync(dp->d_work, 0, sizeof(int32_t), s));
         int nj = r.second - r.first;
-        O.lanes = fan_lanes(nj, c->num_cus);
+        O.lanes = fan_lanes(nj, c->num_cus, O.seg_cap);
         // one wavefront per workgroup spreads the rays over all CUs (the trace
         // kernel is register-bound at one wavefront per SIMD)
         int tblocks = std::max(1, std::min((nj + O.lanes - 1) / O.lanes, c->num_cus * 4 * c->bpc));
@@ -2323,7 +2330,7 @@ extern "C" int bhc_ray_run2d_list(bhc_ctx *ctx, const bhc_problem2d *prob, bhc_r
         O.nsteps_out = d_nout;
         hipMemsetAsync(dp->d_errw, 0, 4 * sizeof(uint32_t), ctx->stream);
         hipMemsetAsync(d_pts, 0, npts * sizeof(bhc_ray_pt2d), ctx->stream);
-        O.lanes = fan_lanes(njobs, ctx->num_cus);
+        O.lanes = fan_lanes(njobs, ctx->num_cus, 0);
         const int blocks = std::min((njobs + O.lanes - 1) / O.lanes, ctx->num_cus * 4 * ctx->bpc);
         if(dp->precision == 64) launch_rays(dp, dp->P64, O, blocks);
         else launch_rays(dp, dp->P32, O, blocks);
