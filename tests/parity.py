@@ -14,6 +14,15 @@ def tl_db(field):
         return -20.0 * np.log10(np.maximum(a, 1e-300))
 
 
+def tl_err(a, b):
+    """Largest TL difference in dB over the receivers where either field is above
+    the 120 dB floor, so that a receiver that one of them leaves out counts;
+    infinite where there is none."""
+    ta, tb = tl_db(a), tl_db(b)
+    m = (ta < 120) | (tb < 120)
+    return float(np.max(np.abs(ta - tb)[m])) if m.any() else np.inf
+
+
 def compare_field(o, g, scaled_o, scaled_g, fp64=True, min_exact=0.999, path_rtol=1e-9, tl_tol=0.1):
     rep = {}
     rep["steps_exact"] = float(np.mean(o.nsteps == g.nsteps))

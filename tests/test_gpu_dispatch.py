@@ -13,7 +13,7 @@ from bellhopcuda_amd.env import Boundary, c2_env, munk_env
 import cases
 import mlp_ref
 import oracle
-from parity import env_context, tl_db
+from parity import env_context, tl_err
 
 pytestmark = pytest.mark.gpu
 
@@ -21,12 +21,6 @@ pytestmark = pytest.mark.gpu
 def _announce(name):
     print("\n[gpu-case]", name, flush=True)
     sys.stdout.flush()
-
-
-def _tl_err(a, b):
-    ta, tb = tl_db(a), tl_db(b)
-    m = ta < 120
-    return np.max(np.abs(ta - tb)[m]) if m.any() else 0.0
 
 
 def _same_as_oracle(env, ctx):
@@ -37,7 +31,7 @@ def _same_as_oracle(env, ctx):
     assert np.array_equal(g.ntop, o.ntop) and np.array_equal(g.nbot, o.nbot)
     assert g.total_steps == o.total_steps and g.total_contrib == o.total_contrib
     # the parity bar for TL: FP32 atomics in another order
-    assert _tl_err(g.problem.scale_pressure(g.field), oracle.scale_pressure(env, o.field)) <= 0.1
+    assert tl_err(g.problem.scale_pressure(g.field), oracle.scale_pressure(env, o.field)) <= 0.1
 
 
 @pytest.mark.parametrize("nbeams", [2, 63, 64, 65, 1023, 1025, 4097])
@@ -85,14 +79,14 @@ def test_chosen_scatter_mapping_equals_each_one(name, gpu_ctx):
     ref = bh.field_run(p, ctx=gpu_ctx)
     o = oracle.field_run(env, nthreads=0)
     assert ref.total_contrib == o.total_contrib
-    assert _tl_err(p.scale_pressure(ref.field), oracle.scale_pressure(env, o.field)) <= 0.1
+    assert tl_err(p.scale_pressure(ref.field), oracle.scale_pressure(env, o.field)) <= 0.1
     dev = bh.Resident(p, gpu_ctx)
     for mode in (1, 2, 3):
         dev.set_scatter(mode)
         dev.launch()
         g = dev.download()
         assert g.total_contrib == ref.total_contrib, mode
-        assert _tl_err(p.scale_pressure(g.field), p.scale_pressure(ref.field)) <= 0.01, mode
+        assert tl_err(p.scale_pressure(g.field), p.scale_pressure(ref.field)) <= 0.01, mode
     dev.release()
 
 
@@ -129,7 +123,7 @@ def test_sweep_order_long_rays_and_wavefronts(precision, segment_mb, gpu_ctx):
             g = sw.download(i)
             assert (g.err, g.warn) == (s.err, s.warn), (lds, i)
             assert np.array_equal(g.nsteps, s.nsteps) and np.array_equal(g.xend, s.xend), (lds, i)
-            assert _tl_err(p.scale_pressure(g.field), p.scale_pressure(s.field)) <= 0.01, (lds, i)
+            assert tl_err(p.scale_pressure(g.field), p.scale_pressure(s.field)) <= 0.01, (lds, i)
     sw.release()
     if segment_mb is not None:
         ctx.close()
@@ -154,7 +148,7 @@ def test_kept_blocks_hold_no_earlier_run(gpu_ctx):
         elif "E" in e.run_type:
             assert g.neigen == f.neigen
         else:
-            assert _tl_err(g.problem.scale_pressure(g.field), f.problem.scale_pressure(f.field)) <= 0.01
+            assert tl_err(g.problem.scale_pressure(g.field), f.problem.scale_pressure(f.field)) <= 0.01
 
 
 @pytest.mark.parametrize("n,n_out,front", [(32, 1, 1), (160, 1, 0), (32, 32, 0), (160, 256, 1), (992, 96, 0)])
