@@ -194,6 +194,7 @@ template<typename real> __device__ inline void load_seg_rest(const DevOut &O, si
 }
 
 template<typename real> struct DevSink {
+    static constexpr bool IN_LDS = false;
     const DevOut *O;
     const Prob2D<real> *P;
     unsigned long long nc;
@@ -373,8 +374,12 @@ __device__ inline int wave_owner(int excl, int t)
 }
 
 // Ray-centred rows of up to this many receivers are walked by the row's own
-// lane, without the prefix sum and the search per item: on a 400-ray seamount
-// field whose rows hold 1-6 receivers the scatter went from 86 to 77 ms.
+// lane, without the prefix sum and the search per item, where the receivers lie
+// in an LDS tile (20001-beam seamount field, tile scatter: 79.5 ms, 92.5 without).
+// Atomics to global memory need the flattened order, which puts neighbouring
+// receivers of a row on neighbouring lanes: a row per lane touches a line of
+// memory per lane (2001 beams, 201 x 1001 receivers, one wavefront per segment:
+// 7.4 ms a row per lane, 2.8 flattened; 1366 x 1001: 40.4 and 15.1).
 constexpr int RAYCEN_DIRECT = 6;
 // Scatter one segment's receivers with the 64 lanes of a wavefront (d is
 // wavefront-uniform). Both geometries have rows of different lengths --
@@ -409,10 +414,12 @@ __device__ inline void scatter_seg(const SegDesc<real> &d, const Prob2D<real> &P
         int blo = 0, bhi = -1;
         if(g + lane < d.nz && !raycen_range(d, iz, P, Rr, P.Rz, nA, rA, nB, rB, blo, bhi)) bhi = blo - 1;
         const int cnt = bhi - blo + 1;
-        if(!__any(cnt > RAYCEN_DIRECT)) {
-            for(int k = 0; __any(k < cnt); ++k)
-                if(k < cnt) raycen_one<real, RT, Sink, FAST>(d, blo + k, iz, nA, rA, nB, rB, P, Rr, sink);
-            continue;
+        if constexpr(Sink::IN_LDS) {
+            if(!__any(cnt > RAYCEN_DIRECT || !sink.holds(d.isz))) {
+                for(int k = 0; __any(k < cnt); ++k)
+                    if(k < cnt) raycen_one<real, RT, Sink, FAST>(d, blo + k, iz, nA, rA, nB, rB, P, Rr, sink);
+                continue;
+            }
         }
         int excl;
         const int total = wave_excl_scan(cnt, lane, excl);
@@ -787,11 +794,13 @@ template<typename real> __global__ void __launch_bounds__(256) k_bin_fill(Prob2D
 }
 
 template<typename real> struct TileSink {
+    static constexpr bool IN_LDS = true;
     float *tile;          // LDS [tile_w][nz] complex, of source isz0
     int col0, tile_w, nz, nrr, isz0;
     unsigned long long nc;
     // (the cell, not its index: an index would have to be divided back into
     // range and depth, several hundred instructions of 64-bit division)
+    __device__ bool holds(int isz) const { return isz == isz0; }
     __device__ void add_cell(const Prob2D<real> &Pp, int isz, int iz, int ir, float re, float im)
     {
         const int c = ir - col0;
