@@ -1,5 +1,6 @@
 """GPU: which fields have LDS tiles for their scatter, at the edges of the rule:
-the depths that a 64 KiB tile of six range columns still holds."""
+the depths that a 64 KiB tile of six range columns still holds, and sources
+that get range bins of their own while 16384 bins last."""
 import sys
 
 import numpy as np
@@ -56,3 +57,12 @@ def test_narrowest_tile_is_used(gpu_ctx):
         assert dev.autotune() == 1
     finally:
         dev.release()
+
+
+# steps of 500 m and ranges 2 m apart: one range per bin
+@pytest.mark.parametrize("sources,nrr", [(1, 16384), (1, 16385), (2, 9001), (3, 6001), (5, 6001)])
+def test_sources_beyond_the_bins(sources, nrr, gpu_ctx):
+    _announce("tile_sources_%d_%d" % (sources, nrr))
+    env = munk_env(nbeams=33, nrz=51, nrr=nrr, r_max_km=0.002 * (nrr - 1), run_type="CB")
+    env.Sz = np.linspace(400.0, 3000.0, sources).astype(np.float32)
+    _mappings_agree(env, gpu_ctx)
