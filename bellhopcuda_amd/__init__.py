@@ -52,6 +52,7 @@ def lib():
         "bhc_ctx_destroy": (None, [C.c_void_p]),
         "bhc_ctx_set_launch": (C.c_int, [C.c_void_p, C.c_int, C.c_int]),
         "bhc_ctx_synchronize": (C.c_int, [C.c_void_p]),
+        "bhc_ctx_trim": (C.c_int, [C.c_void_p]),
         "bhc_copy_calibrate": (C.c_int, [C.c_void_p, C.c_longlong, P(C.c_double)]),
         "bhc_last_kernel_ms": (C.c_int, [C.c_void_p, P(C.c_double)]),
         "bhc_field_run2d": (C.c_int, [C.c_void_p, P(_abi.Problem2D), P(_abi.FieldOut)]),
@@ -194,6 +195,10 @@ class Context:
 
     def set_launch(self, blocks_per_cu=0):
         _check(lib().bhc_ctx_set_launch(self._h, 0, blocks_per_cu))
+
+    def trim(self):
+        """Give the device memory kept from earlier runs back to the device."""
+        _check(lib().bhc_ctx_trim(self._h))
 
     def progress(self):
         """(rays finished, rays of the run) of the current or last run."""

@@ -32,13 +32,12 @@
 #include <algorithm>
 #include <cmath>
 #include <atomic>
-#include <map>
 #include <mutex>
 #include <thread>
-#include <unordered_map>
 
 #include "../../include/bhc_hip.h"
 #include "core2d.h"
+#include "devpool.h"
 #include "pack2d.h"
 #include "nx2d.h"
 #include "pack3d.h"
@@ -1264,65 +1263,13 @@ __global__ void __launch_bounds__(256) k_arr_merge(const ArrCand *cand, const in
 // next ones: a run allocates a dozen arrays, among them the arrivals'
 // candidate slots (up to 16 GiB, for which hipMalloc waits until the driver
 // has cleared as much memory: 249 ms for a 2121-receiver run whose kernels
-// take 7 ms, 4 ms when cleared memory was at hand). At most POOL_BYTES are
-// kept; destroying the context gives them back to the device, and any
-// allocation of the library that finds no memory first gives back those of
-// every context (bhc_give_back_pools). A block is put here only after the
+// take 7 ms, 4 ms when cleared memory was at hand). At most BHC_POOL_MB
+// (default 20 GiB) are kept; bhc_ctx_trim and destroying the context give them
+// back to the device, and an allocation of the library that finds no memory
+// first gives back those of every context. A block is put here only after the
 // context's stream has been waited for, so an idle block is in no one's use.
-constexpr size_t POOL_BYTES = size_t(20) << 30;
-struct DevPool;
-std::mutex g_pools_mu;
-std::vector<DevPool *> g_pools;                     // of every context
-struct DevPool {
-    std::mutex mu;
-    std::multimap<size_t, void *> idle;             // by size
-    std::unordered_map<void *, size_t> size;        // of every block handed out or idle
-    size_t held = 0;                                // bytes idle
-    DevPool()
-    {
-        std::lock_guard<std::mutex> lk(g_pools_mu);
-        g_pools.push_back(this);
-    }
-    ~DevPool()
-    {
-        {
-            std::lock_guard<std::mutex> lk(g_pools_mu);
-            g_pools.erase(std::find(g_pools.begin(), g_pools.end(), this));
-        }
-        trim();
-    }
-    void trim()
-    {
-        std::lock_guard<std::mutex> lk(mu);
-        for(auto &b : idle) {
-            (void)hipFree(b.second);
-            size.erase(b.second);
-        }
-        idle.clear();
-        held = 0;
-    }
-    // a block of at least n bytes, and at most twice that (or 1 MiB) from the idle ones
-    hipError_t get(void **p, size_t n);
-    void put(void *p)
-    {
-        if(!p) return;
-        std::lock_guard<std::mutex> lk(mu);
-        const size_t n = size[p];
-        if(held + n > POOL_BYTES) {
-            size.erase(p);
-            (void)hipFree(p);
-            return;
-        }
-        idle.emplace(n, p);
-        held += n;
-    }
-};
-
-void bhc_give_back_pools()
-{
-    std::lock_guard<std::mutex> lk(g_pools_mu);
-    for(DevPool *p : g_pools) p->trim();
-}
+constexpr size_t POOL_MB = 20480;
+void bhc_give_back_pools();
 
 // hipMalloc that gives the pools back before it gives up
 hipError_t bhc_device_malloc(void **p, size_t n)
@@ -1334,25 +1281,30 @@ hipError_t bhc_device_malloc(void **p, size_t n)
     return hipMalloc(p, n);
 }
 
-hipError_t DevPool::get(void **p, size_t n)
-{
-    n = (n + 255) / 256 * 256;
+struct DevMem {
+    static int alloc(void **p, size_t n) { return (int)bhc_device_malloc(p, n); }
+    static void free(void *p) { (void)hipFree(p); }
+};
+struct DevPool;
+std::mutex g_pools_mu;
+std::vector<DevPool *> g_pools;                     // of every context
+struct DevPool : BlockPool<DevMem> {
+    DevPool() : BlockPool<DevMem>(POOL_MB << 20)
     {
-        std::lock_guard<std::mutex> lk(mu);
-        auto it = idle.lower_bound(n);
-        if(it != idle.end() && it->first <= std::max(2 * n, size_t(1) << 20)) {
-            *p = it->second;
-            held -= it->first;
-            idle.erase(it);
-            return hipSuccess;
-        }
+        std::lock_guard<std::mutex> lk(g_pools_mu);
+        g_pools.push_back(this);
     }
-    const hipError_t e = bhc_device_malloc(p, n);
-    if(e == hipSuccess) {
-        std::lock_guard<std::mutex> lk(mu);
-        size[*p] = n;
+    ~DevPool()
+    {
+        std::lock_guard<std::mutex> lk(g_pools_mu);
+        g_pools.erase(std::find(g_pools.begin(), g_pools.end(), this));
     }
-    return e;
+};
+
+void bhc_give_back_pools()
+{
+    std::lock_guard<std::mutex> lk(g_pools_mu);
+    for(DevPool *p : g_pools) p->trim();
 }
 
 struct bhc_ctx {
@@ -1523,15 +1475,16 @@ extern "C" int bhc_ctx_create(int device, bhc_ctx **out)
     c->scatter3_map = 2;
     if(const char *e = getenv("BHC_SCATTER3_MAP")) c->scatter3_map = std::min(std::max(atoi(e), 0), 2);
     if(const char *e = getenv("BHC_SEG_BUFFER_MB")) c->seg_mb = (size_t)std::max(16L, atol(e));
+    if(const char *e = getenv("BHC_POOL_MB")) c->pool.set_limit((size_t)std::max(0L, atol(e)) << 20);
     HIPCHECK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
     HIPCHECK(hipEventCreate(&c->ev0));
     HIPCHECK(hipEventCreate(&c->ev1));
     HIPCHECK(hipEventCreate(&c->evm));
     HIPCHECK(hipEventCreate(&c->pa));
     HIPCHECK(hipEventCreate(&c->pb));
-    HIPCHECK(hipMalloc((void **)&c->d_seg_count, sizeof(uint32_t)));
-    HIPCHECK(hipMalloc((void **)&c->d_overflow, sizeof(uint32_t)));
-    HIPCHECK(hipMalloc((void **)&c->d_prog, sizeof(unsigned long long)));
+    HIPCHECK(bhc_device_malloc((void **)&c->d_seg_count, sizeof(uint32_t)));
+    HIPCHECK(bhc_device_malloc((void **)&c->d_overflow, sizeof(uint32_t)));
+    HIPCHECK(bhc_device_malloc((void **)&c->d_prog, sizeof(unsigned long long)));
     HIPCHECK(hipHostMalloc((void **)&c->h_prog, 64, hipHostMallocMapped | hipHostMallocCoherent));
     *c->h_prog = 0ull;
     if(scratch_address(device, &c->scratch)) return -1;
@@ -1595,6 +1548,13 @@ extern "C" int bhc_ctx_synchronize(bhc_ctx *ctx)
     return 0;
 }
 
+extern "C" int bhc_ctx_trim(bhc_ctx *ctx)
+{
+    if(!ctx) return fail("bhc_ctx_trim: null context");
+    ctx->pool.trim();
+    return 0;
+}
+
 namespace {
 // Plain streaming copy (16 B per lane per iteration): the known-size kernel
 // against which profiler byte counters (FETCH_SIZE, WRITE_SIZE) are scaled.
@@ -1611,8 +1571,8 @@ extern "C" int bhc_copy_calibrate(bhc_ctx *ctx, long long bytes, double *ms)
     if(bytes < 16 || (bytes & 15)) return fail("bhc_copy_calibrate: bytes must be a positive multiple of 16");
     HIPCHECK(hipSetDevice(ctx->device));
     void *a = nullptr, *b = nullptr;
-    HIPCHECK(hipMalloc(&a, (size_t)bytes));
-    if(hipMalloc(&b, (size_t)bytes) != hipSuccess) {
+    HIPCHECK(bhc_device_malloc(&a, (size_t)bytes));
+    if(bhc_device_malloc(&b, (size_t)bytes) != hipSuccess) {
         (void)hipFree(a);
         return fail("bhc_copy_calibrate: allocation failed");
     }
@@ -1679,7 +1639,7 @@ template<typename T> int palloc(bhc_ctx *c, T **p, size_t n)
 {
     *p = nullptr;
     if(n == 0) return 0;
-    HIPCHECK(c->pool.get((void **)p, n * sizeof(T)));
+    HIPCHECK((hipError_t)c->pool.get((void **)p, n * sizeof(T)));
     return 0;
 }
 

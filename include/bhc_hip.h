@@ -341,6 +341,9 @@ int bhc_problem_autotune(bhc_ctx *ctx, bhc_dev_problem *dp, int *mode_out);
 /* Force a scatter mapping (0 = automatic choice, 1 tiles, 2 wavefront, 3 lane). */
 int bhc_problem_set_scatter(bhc_dev_problem *dp, int mode);
 int bhc_ctx_synchronize(bhc_ctx *ctx);
+/* Give the device blocks that the context keeps from earlier runs for later
+ * ones (at most the environment setting BHC_POOL_MB, in MiB) back to the device. */
+int bhc_ctx_trim(bhc_ctx *ctx);
 /* Measurement aid with no counterpart in the reference: one launch of a plain
  * 16-byte-per-lane copy kernel (k_copy16) over `bytes` (a multiple of 16) on
  * the context's stream, *ms its duration. Profiler byte counters read for it
