@@ -3099,6 +3099,7 @@ struct bhc_sweep {
     int32_t *d_save_pid[2];
     int max_waves;
     int lds_bytes, lds_bytes_max;
+    int lds_limit;              // largest budget that can be set
     int passes;
     int scatter_blocks;
     int scatter_lanes;          // 0: one wavefront per segment, 1: one lane per segment, 2: 64 segments' receivers flattened over a wavefront
@@ -3152,7 +3153,7 @@ int sweep_upload(bhc_sweep *sw, const bhc_problem2d *const *probs)
     std::vector<size_t> boff(n);
     std::vector<float> rzsz;
     std::vector<size_t> rzoff(n), szoff(n);
-    size_t max_staged = 0;
+    size_t max_staged = 0, max_whole = 0;
     sw->field_off.resize(n);
     sw->stats_off.resize(n);
     sw->field_floats = 0;
@@ -3172,6 +3173,12 @@ int sweep_upload(bhc_sweep *sw, const bhc_problem2d *const *probs)
         // 30.3). Cartesian beams' descriptors do not need them.
         if(!(P[i].isRayCen && P[i].staged_reals * sizeof(real) <= (size_t)SWEEP_LDS2)) P[i].staged_reals = P[i].o_rzs;
         max_staged = std::max(max_staged, (size_t)P[i].staged_reals);
+        // the tables with every column: receiver depths, whole boundary nodes and
+        // the sound speeds that splines do not read
+        const size_t whole = (size_t)P[i].o_rzs + p->NRz
+            + (P[i].node == NODE_LINE ? (size_t)(NODE_SHORT - NODE_LINE) * (p->ati_npts + p->bty_npts) : 0)
+            + (p->ssp_type == 'S' || p->ssp_type == 'P' ? 4 * (size_t)p->ssp_npts : 0);
+        max_whole = std::max(max_whole, whole);
         rzoff[i] = rzsz.size();
         rzsz.insert(rzsz.end(), p->Rz, p->Rz + p->NRz);
         szoff[i] = rzsz.size();
@@ -3198,6 +3205,7 @@ int sweep_upload(bhc_sweep *sw, const bhc_problem2d *const *probs)
     size_t lds_reals = std::min(max_staged, cap_reals);
     sw->lds_bytes_max = (int)(lds_reals * sizeof(real));
     sw->lds_bytes = std::min(sw->lds_bytes_max, SWEEP_LDS2);
+    sw->lds_limit = (int)(std::min(max_whole, cap_reals) * sizeof(real));
     if(dalloc((real **)&sw->d_blobs, blobs.size()) || dalloc(&sw->d_rzsz, rzsz.size())
        || dalloc(&sw->d_fields, sw->field_floats) || dalloc((Prob2D<real> **)&sw->d_probs, (size_t)n)
        || dalloc(&sw->d_order, (size_t)n) || dalloc(&sw->d_ray_next, (size_t)n) || dalloc(&sw->d_pcursor, 1) || dalloc(&sw->d_resume, 1)
@@ -3578,9 +3586,8 @@ extern "C" int bhc_sweep_set_launch(bhc_sweep *sw, int scatter_blocks, int lds_b
     if(!sw) return fail("bhc_sweep_set_launch: null sweep");
     const int rsz = sw->precision == 64 ? (int)sizeof(double) : (int)sizeof(float);
     if(scatter_blocks < 1 || scatter_blocks > (1 << 20)) return fail("bhc_sweep_set_launch: scatter_blocks out of range");
-    const int most = std::max(sw->lds_bytes_max, std::min(2 * SWEEP_LDS2, sw->ctx->lds_max));
-    if(lds_bytes < 0 || lds_bytes > most || lds_bytes % rsz)
-        return fail("bhc_sweep_set_launch: lds_bytes must be a multiple of %d in [0, %d]", rsz, most);
+    if(lds_bytes < 0 || lds_bytes > sw->lds_limit || lds_bytes % rsz)
+        return fail("bhc_sweep_set_launch: lds_bytes must be a multiple of %d in [0, %d]", rsz, sw->lds_limit);
     sw->scatter_blocks = scatter_blocks;
     sw->lds_bytes = std::min(lds_bytes, sw->lds_bytes_max);
     sw->tuned = true;
