@@ -509,6 +509,7 @@ struct bhc_mlp {
     int32_t *idx;              // batches of a chunk of steps
     long long nset;
     long long step;
+    int last_loss;             // which half of `loss` holds the last step's
     hipEvent_t e0, e1;
     double last_ms;
 };
@@ -743,6 +744,7 @@ extern "C" int bhc_mlp_gradients(bhc_mlp *m, const float *x, const float *y, int
     MCHECK(hipMemcpyAsync(m->x, x, (size_t)n * D_IN * 4, hipMemcpyHostToDevice, m->stream));
     MCHECK(hipMemcpyAsync(m->y, y, (size_t)n * m->n_out * 4, hipMemcpyHostToDevice, m->stream));
     zero_grads(m);
+    m->last_loss = 0;
     forward_backward(m, m->x, m->y, nullptr, n, m->loss);
     MCHECK(hipGetLastError());
     if(grads)
@@ -779,7 +781,7 @@ extern "C" int bhc_mlp_train(bhc_mlp *m, int steps, int batch, float lr, unsigne
     std::uniform_int_distribution<long long> ud(0, m->nset - 1);
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
     MCHECK(hipEventRecord(m->e0, m->stream));
-    zero_grads(m);
+    if(steps > 0) zero_grads(m);
     // batches are drawn a chunk of steps at a time, while the GPU works on the
     // chunk before; the copy follows that chunk's steps on the stream
     std::vector<int32_t> idx((size_t)steps * batch);
@@ -791,6 +793,7 @@ extern "C" int bhc_mlp_train(bhc_mlp *m, int steps, int batch, float lr, unsigne
         for(int s = 0; s < ns; ++s) {
             float *loss = m->loss + 16 * ((s0 + s) & 1), *next = m->loss + 16 * ((s0 + s + 1) & 1);
             forward_backward(m, m->X, m->Y, m->idx + (size_t)s * batch, batch, loss);
+            m->last_loss = (s0 + s) & 1;
             ++m->step;
             float c1 = 1.0f - std::pow(b1, (float)m->step), c2 = 1.0f - std::pow(b2, (float)m->step);
             hipLaunchKernelGGL(k_adam<true>, dim3(n_tiles(m->n_out) + (n_loose(m->n_out) + 255) / 256, m->members),
@@ -801,8 +804,7 @@ extern "C" int bhc_mlp_train(bhc_mlp *m, int steps, int batch, float lr, unsigne
     MCHECK(hipEventRecord(m->e1, m->stream));
     MCHECK(hipGetLastError());
     if(loss_out)
-        MCHECK(hipMemcpyAsync(loss_out, m->loss + 16 * ((steps - 1) & 1), (size_t)m->members * 4, hipMemcpyDeviceToHost,
-                              m->stream));
+        MCHECK(hipMemcpyAsync(loss_out, m->loss + 16 * m->last_loss, (size_t)m->members * 4, hipMemcpyDeviceToHost, m->stream));
     MCHECK(hipStreamSynchronize(m->stream));
     float ms = 0.f;
     MCHECK(hipEventElapsedTime(&ms, m->e0, m->e1));
