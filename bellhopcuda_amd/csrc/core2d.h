@@ -284,7 +284,7 @@ template<typename real> struct Trace {
 };
 
 template<typename real> struct Infl {
-    real alpha, SrcDeclAngle, omega, BeamWindow, Ratio1, rcp_q0;
+    real alpha, SrcDeclAngle, omega, Ratio1, rcp_q0;
     real phase, qOld;
     v2<real> rayn1, x;
     v2<real> rbr;               // Cartesian: receiver ranges Rr[ir], Rr[ir + 1] (the walk's bracket)
@@ -958,7 +958,6 @@ __host__ __device__ inline bool RayInit(int isz, int ialpha, RayPt<real> &p0, Tr
     }
     // Init_Influence
     I.omega = FL(2.0) * RC<real>::PI * P.freq0;
-    I.BeamWindow = P.isGaussian ? RL(4.0) : RL(1.0);
     I.Ratio1 = std::sqrt(std::fabs(G[P.o_acos + ialpha]));
     if(P.run3 == 'X') I.Ratio1 = RL(1.0);
     if(P.isGaussian) I.Ratio1 /= std::sqrt(FL(2.0) * RC<real>::PI);
@@ -1134,7 +1133,7 @@ template<typename real> struct SegDesc {
     // arrivals and eigen hits
     v2<real> xb, tb;
     real RcvrDecl, SrcDecl;
-    real wmax;                  // ray-centred: upper bound of BeamWindow * sigma over the segment
+    real wmax;                  // ray-centred: upper bound of the beam window (4 sigma, hat beams sigma) over the segment
     int32_t lastValid;          // ray-centred
     int32_t ntop, nbot, ialpha, is;
 };

@@ -916,7 +916,7 @@ __host__ __device__ inline void Reflect3(const Ray3<real> &oldp, Ray3<real> &new
 // Ray init / update / terminate (src/trace.hpp, 3D)
 // ---------------------------------------------------------------------------
 template<typename real> struct Infl3 {
-    real Ratio1, rcp_q0, rcp_qhat0, omega, BeamWindow;
+    real Ratio1, rcp_q0, rcp_qhat0, omega;
     real phase, qOld;
     v3<real> xs;
     v3<real> rn1, rn2;     // ray-centred beams: the previous point's ray normals (c-scaled)
@@ -992,7 +992,6 @@ __host__ __device__ inline bool RayInit3(int ia, int ib, int isx, int isy, int i
     S.iSmall = 0;
     // Init_Influence
     I.omega = FL(2.0) * RC<real>::PI * P.freq0;
-    I.BeamWindow = P.isGaussian ? RL(4.0) : RL(1.0);
     I.Ratio1 = std::sqrt(std::fabs(ca));
     I.Ratio1 *= std::sqrt(P.Dalpha * P.Dbeta) / p0.c;
     if(P.isGaussian) I.Ratio1 /= FL(2.0) * RC<real>::PI;
@@ -1763,7 +1762,7 @@ template<typename real> struct Seg3R {
     m2<real> q0, dq;
     cpx<real> tau0, dtau;
     real A0, phase0, qOld, rcp_q0, rcp_qhat0, xs_x, xs_y;
-    real rmax_m, rmax_n;         // Gaussian: BeamWindow x the larger |q| (scaled) at A and B, per normal
+    real rmax_m, rmax_n;         // Gaussian: 4 x the larger |q| (scaled) at A and B, per normal
     int32_t nitems;              // > 0: rows (depth, bearing) to visit
     int32_t isrc, job, is, ntop, nbot;
 };

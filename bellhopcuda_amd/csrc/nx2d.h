@@ -308,7 +308,6 @@ __host__ __device__ inline bool RayInitNx(int ia, int ib, int isx, int isy, int 
     S.iSmall = 0;
     // Init_Influence, 2D geometric beams
     I.omega = FL(2.0) * RC<real>::PI * P.freq0;
-    I.BeamWindow = P.isGaussian ? RL(4.0) : RL(1.0);
     I.Ratio1 = std::sqrt(std::fabs(ca));
     if(P.run3 == 'X') I.Ratio1 = RL(1.0);
     if(P.isGaussian) I.Ratio1 /= std::sqrt(FL(2.0) * RC<real>::PI);
