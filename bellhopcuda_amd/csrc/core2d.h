@@ -1236,8 +1236,9 @@ __host__ __device__ inline bool cart_begin(SegGeo<real> &g, const RayPt<real> &p
 
 // WINDOW = false leaves the segment's depth window to the scatter (every
 // depth in the descriptor; the scatter's per-column band and the zmin / zmax
-// test of each receiver select the same contributions): a batched trace,
-// latency-bound at one wavefront per SIMD, hands that search to the scatter.
+// test of each receiver select the same contributions): a batched trace, which
+// is bound by the latency of its steps at two wavefronts per SIMD, hands that
+// search to the scatter.
 template<typename real, bool WINDOW>
 __host__ __device__ inline void cart_fill(SegDesc<real> &d, const SegGeo<real> &g, const RayPt<real> &p0,
                                           const RayPt<real> &p1, const Infl<real> &I, int is, const Prob2D<real> &P,
@@ -1436,7 +1437,9 @@ __host__ __device__ inline void put_field(Sink &sink, const Prob2D<real> &P, int
 // FAST = false follows the reference's arithmetic to the last bit. FAST = true
 // evaluates the final TL term -- a unit phasor and Gaussian weight that are
 // then rounded to the FP32 field -- at FP32 accuracy: the phase is reduced in
-// FP64 first, the geometry, delay and amplitude stay in `real`.
+// FP64 first, the geometry, delay and amplitude stay in `real`. The amplitude's
+// and the weight's divisions and square root are then reciprocals within an ulp
+// or two (recip, recip_sqrt).
 template<typename real, int RT, typename Sink, bool FAST = false>
 __host__ __device__ inline void contrib(const SegDesc<real> &d, real s, real n1, int ir, int iz, const Prob2D<real> &P,
                                         Sink &sink)

@@ -174,11 +174,14 @@ __device__ inline void add_col(const float *v, float *to, int lane)
 // ROWS batch rows of one member through the network, and in training (TRAIN)
 // the loss, the output gradient and every layer's gradient dZ back to the
 // first layer. Eight wavefronts, one 32-column tile of each layer apiece: two
-// per SIMD. 2048 rows of 4 members are 256 workgroups, one per CU. The vector
-// ALU bounds it: 12.6 million GELUs a step, whose erf and exp take some 65
-// instructions, made once (the slope is kept, not the pre-activation). A
-// layer's weights (128 KB per workgroup, from the L2) are loaded while the
-// layer before goes through its GELU.
+// per SIMD. 2048 rows of 4 members are 256 workgroups, one per CU. Waiting bounds
+// it: a wavefront waits for memory or a layer's barrier in 62 % of its cycles and
+// issues vector instructions in 16 % (12.6 million GELUs a step of some 65
+// instructions, made once: the slope is kept, not the pre-activation), and two
+// wavefronts per SIMD cannot cover that. In its 86 us it writes 105 MB (half of
+// it slopes) and reads 99, and the L2 answers 5.1 million requests, the weights'
+// above all. A layer's weights (128 KB per workgroup, from the L2) are loaded
+// while the layer before goes through its GELU.
 // Replaces one launch per layer and direction with FP32 pre-activations and
 // gradients in memory: a training step of 2048 rows, 4 members, 128 outputs
 // took 1270 us in 36 launches (28 us of it at the matrix cores' rate).

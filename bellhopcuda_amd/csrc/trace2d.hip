@@ -2841,10 +2841,12 @@ __device__ inline int run_problem_any(const BatchDev<real> &Bd, const DevOut &O,
 #undef BHC_RUN
 }
 
-// Two wavefronts per SIMD (at most 256 registers, which run_problem fits
-// without spilling now that the launch's structures are scalar): a single one
-// waits for memory and for its own dependent FP64 operations in half of its
-// cycles. Each gets half of the LDS (sweep_waves).
+// Two wavefronts per SIMD (at most 256 registers): a single one waits for memory
+// and for its own dependent FP64 operations in half of its cycles. Each gets half
+// of the LDS (sweep_waves). With the launch's structures in scalar registers
+// run_problem nearly fits: its 7 to 11 thousand instructions hold 5 to 14 scratch
+// reloads (fused in FP64 11 to 37); the kernel around it spills 75 registers
+// across its calls, once per problem.
 template<typename real, int MODE>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) k_trace_batch(BatchDev<real> Bd, DevOut O)
 {

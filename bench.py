@@ -351,7 +351,7 @@ def run_sweep(a):
         tuned = {"scatter_blocks": b, "lds_bytes": l, "scatter_lanes": m, "source": "--sweep-config"}
         log("launch configuration given: %s" % json.dumps(tuned))
     else:
-        log("uploaded; autotuning on the first 64 problems")
+        log("uploaded; autotuning on the first 64 problems (the staging budget on 256)")
         tuned = sw.autotune()
         log("autotuned: %s" % json.dumps(tuned))
     # kernel-by-kernel passes, so that HIP events time the trace and the scatter
