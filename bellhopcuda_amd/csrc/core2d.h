@@ -630,7 +630,9 @@ __host__ __device__ inline void CarrySSP(v2<real> x1, v2<real> x, v2<real> t, Tr
 
 // One polygon step. Profiles of depth alone (every type but 'Q') have no
 // range derivatives: the terms they would multiply are zero and are left out
-// (adding or subtracting zero changes no value). The step's own evaluations
+// (adding or subtracting zero changes no value). Without second derivatives p
+// keeps its value too, unless the q that their zeros multiply has grown past the
+// largest number: the product is NaN then, as q - q is. The step's own evaluations
 // are two: the start's is carried (S.at).
 template<typename real, char ST = 0>
 __host__ __device__ inline void Step(const RayPt<real> &ray0, RayPt<real> &ray2, Trace<real> &S, const Prob2D<real> &P,
@@ -667,15 +669,13 @@ __host__ __device__ inline void Step(const RayPt<real> &ray0, RayPt<real> &ray2,
     RayPt<real> ray1;
     ray1.x = ray0.x + sc(halfh, u0);
     ray1.t = turned(ray0.t, halfh, o0.gradc, csq0);
-    ray1.p = nocurv ? ray0.p : ray0.p + sc(halfh, pq0p);
+    ray1.p = nocurv ? ray0.p + (ray0.q - ray0.q) : ray0.p + sc(halfh, pq0p);
+    ray1.q = ray0.q + sc(halfh, pq0q);
 
     EvaluateSSP<real, ST>(ray1.x, ray1.t, o1, P, B, S.iz, S.ir, e);
     const real c1 = o1.c.re;
     v2<real> pq1p = V((real)0, (real)0);
-    if(!nocurv) {
-        ray1.q = ray0.q + sc(halfh, pq0q);
-        pq1p = sc(-bend(o1.crr, o1.crz, o1.czz, ray1.t), ray1.q);
-    }
+    if(!nocurv) pq1p = sc(-bend(o1.crr, o1.crz, o1.czz, ray1.t), ray1.q);
     const v2<real> pq1q = sc(c1, ray1.p);
     const real csq1 = c1 * c1;
     const v2<real> u1 = sc(c1, ray1.t);
@@ -690,8 +690,8 @@ __host__ __device__ inline void Step(const RayPt<real> &ray0, RayPt<real> &ray2,
     const real hw0 = h * w0, hw1 = h * w1;
     ray2.t = turned(turned(ray0.t, hw0, o0.gradc, csq0), hw1, o1.gradc, csq1);
     ray2.tau = (ray0.tau + slowness_term(hw0, o0.c)) + slowness_term(hw1, o1.c);
-    ray2.p = ray0.p;
-    if(!nocurv) ray2.p = (ray0.p + sc(hw0, pq0p)) + sc(hw1, pq1p);
+    if(nocurv) ray2.p = ray1.p + (ray1.q - ray1.q);
+    else ray2.p = (ray0.p + sc(hw0, pq0p)) + sc(hw1, pq1p);
     ray2.q = ray0.q + sc(hw0, pq0q);
     ray2.q = ray2.q + sc(hw1, pq1q);
     ray2.Amp = ray0.Amp;

@@ -586,10 +586,12 @@ __host__ __device__ inline PQ3<real> DeltaPQ3(const Ray3<real> &ray, const SSPOu
     pq.phi = (FL(1.0) / c) * ray.t.z * (ray.t.y * o.gradc.x - ray.t.x * o.gradc.y) / tt;
     pq.q = mscl(c, ray.p);
     // No second derivatives (the hexahedral grid and piecewise-linear
-    // profiles): p does not change, whatever the ray normals are as long as
-    // they are numbers.
+    // profiles): p does not change, as long as what the zeros multiply are
+    // numbers (a q that has grown past the largest one turns p into NaN).
+    const real sum = tt + std::fabs(ray.phi) + std::fabs(ray.q.a00) + std::fabs(ray.q.a01) + std::fabs(ray.q.a10)
+        + std::fabs(ray.q.a11);
     if(o.cxx == (real)0 && o.cyy == (real)0 && o.czz == (real)0 && o.cxy == (real)0 && o.cxz == (real)0
-       && o.cyz == (real)0 && tt > (real)0 && std::isfinite(ray.phi)) {
+       && o.cyz == (real)0 && tt > (real)0 && sum <= RC<real>::MAXV) {
         pq.p = M2((real)0, (real)0, (real)0, (real)0);
         return pq;
     }
